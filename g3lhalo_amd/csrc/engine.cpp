@@ -7,6 +7,7 @@
 #include <algorithm>
 #include <chrono>
 #include <cmath>
+#include <cstddef>
 #include <cstdio>
 #include <cstring>
 #include <new>
@@ -390,6 +391,76 @@ int run_engine(g3l_ctx *c, EngineJobs &E, std::vector<JobState> &out, bool timed
   return G3L_OK;
 }
 
+// ---------------------------------------------------------------------------
+// 1-D integrals (k_onedim).
+
+int run_one_dim(g3l_ctx *c, const std::vector<OneDimGroup> &groups,
+                const std::vector<OneDimJob> &jobs, bool precomp, double reltol, double scale) {
+  if (groups.size() >= (1u << 24)) return G3L_ENOMEM;
+  int cus = 0;
+  G3L_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device));
+  size_t total = 0;
+  for (const OneDimGroup &g : groups) total += g.count;
+  if (total >= (1ull << 31)) return G3L_ENOMEM;
+  const size_t resident = (size_t)std::max(1, cus) * one_dim_blocks_per_cu();
+  // integrals per unit: as many as still give every resident block one
+  const uint32_t per =
+      (uint32_t)std::min<size_t>(kOneDimMaxUnit, std::max<size_t>(1, total / resident));
+  std::vector<OneDimUnit> units;
+  units.reserve(total / per + groups.size());
+  for (size_t g = 0; g < groups.size(); ++g)
+    for (uint32_t i = 0; i < groups[g].count; i += per)
+      units.push_back(OneDimUnit{(uint32_t)g, i, std::min(per, groups[g].count - i)});
+  // one upload: outcome words, groups, jobs, units; the retry list behind them
+  struct Outcome {
+    unsigned long long failed;
+    uint32_t nretry, pad;
+  };
+  auto al = [](size_t x) { return (x + 255) & ~size_t(255); };
+  const size_t o_groups = al(sizeof(Outcome));
+  const size_t o_jobs = al(o_groups + groups.size() * sizeof(OneDimGroup));
+  const size_t o_units = al(o_jobs + jobs.size() * sizeof(OneDimJob));
+  const size_t o_retry = al(o_units + units.size() * sizeof(OneDimUnit));
+  const uint32_t blocks = (uint32_t)std::min(units.size(), resident);
+  int rc;
+  if ((rc = c->od_in.ensure(o_retry + total * sizeof(OneDimUnit)))) return rc;
+  if ((rc = c->od_store.ensure(blocks * one_dim_store_bytes()))) return rc;
+  std::vector<unsigned char> host(o_retry, 0);
+  Outcome oc{~0ull, 0, 0};
+  std::memcpy(host.data(), &oc, sizeof(oc));
+  std::memcpy(host.data() + o_groups, groups.data(), groups.size() * sizeof(OneDimGroup));
+  std::memcpy(host.data() + o_jobs, jobs.data(), jobs.size() * sizeof(OneDimJob));
+  std::memcpy(host.data() + o_units, units.data(), units.size() * sizeof(OneDimUnit));
+  unsigned char *base = c->od_in.as<unsigned char>();
+  hipStream_t s = c->stream;
+  G3L_HIP(hipMemcpyAsync(base, host.data(), host.size(), hipMemcpyHostToDevice, s));
+  OneDimLaunch L{};
+  L.T = c->T;
+  L.groups = reinterpret_cast<const OneDimGroup *>(base + o_groups);
+  L.jobs = reinterpret_cast<const OneDimJob *>(base + o_jobs);
+  L.units = reinterpret_cast<const OneDimUnit *>(base + o_units);
+  L.nunits = (uint32_t)units.size();
+  L.reltol = reltol;
+  L.scale = scale;
+  L.store = c->od_store.as<unsigned char>();
+  L.retry = reinterpret_cast<OneDimUnit *>(base + o_retry);
+  L.failed = reinterpret_cast<unsigned long long *>(base);
+  L.nretry = reinterpret_cast<uint32_t *>(base + offsetof(Outcome, nretry));
+  G3L_HIP(launch_one_dim(precomp, L, blocks, s));
+  G3L_HIP(hipMemcpyAsync(&oc, base, sizeof(oc), hipMemcpyDeviceToHost, s));
+  G3L_HIP(hipStreamSynchronize(s));
+  if (oc.nretry) {
+    // integrals whose block ran out of nodes, each alone in a block: no more
+    // retries (an integral's own nodes always fit)
+    L.units = L.retry;
+    L.nunits = oc.nretry;
+    G3L_HIP(launch_one_dim(precomp, L, std::min(blocks, oc.nretry), s));
+    G3L_HIP(hipMemcpyAsync(&oc, base, sizeof(oc), hipMemcpyDeviceToHost, s));
+    G3L_HIP(hipStreamSynchronize(s));
+  }
+  return oc.failed == ~0ull ? (int)G3L_OK : status_of((uint32_t)(oc.failed & 0xff));
+}
+
 }  // namespace g3l
 
 namespace {
@@ -577,7 +648,7 @@ int plain_cubature(g3l_ctx *c, int kind, const double *lo, const double *hi, uin
 
 // n_bar(z_i) = ln10 * int m n(m,z) (Ncen + Nsat) dlog10 m for every grid z
 // and both HODs of each new set (src/NNMap_Model.cu:244-282), all on the
-// device in one batched run.
+// device in one run.
 int compute_nbar(g3l_ctx *c, int first, int count) {
   const int nb = c->nb;
   const size_t need_chunks = ((size_t)first + count + kSetsPerChunk - 1) / kSetsPerChunk;
@@ -587,54 +658,22 @@ int compute_nbar(g3l_ctx *c, int first, int count) {
     if (rc) return rc;
     c->nbar_chunks.push_back(b);
   }
-  // run in chunks of sets to bound the pool
-  const int chunk = 64;
-  for (int s0 = first; s0 < first + count; s0 += chunk) {
-    int s1 = std::min(first + count, s0 + chunk);
-    EngineJobs E;
-    for (int s = s0; s < s1; ++s) {
-      for (int which = 0; which < 2; ++which) {
-        for (int i = 0; i < nb; ++i) {
-          JobDesc d{};
-          d.kind = kNbar;
-          d.dim = 1;
-          d.pts = 15;
-          d.args = (int)E.args.size();
-          d.cap = 2048;
-          d.reltol = 1e-4;
-          d.maxeval = 0;
-          TermArgs a{};
-          a.t1 = c->zmin + i * (c->zmax - c->zmin) / nb;
-          a.h1 = a.h2 = to_dev(which == 0 ? c->sets[s].h1 : c->sets[s].h2);
-          fill_logs(c, a);
-          E.args.push_back(a);
-          E.desc.push_back(d);
-          double box[2 * kMaxDim] = {0};
-          box[0] = std::log10(c->mmin_i);
-          box[kMaxDim] = std::log10(c->mmax_i);
-          E.boxes.insert(E.boxes.end(), box, box + 2 * kMaxDim);
-        }
-      }
+  std::vector<OneDimJob> zs(nb);
+  for (int i = 0; i < nb; ++i) zs[i] = OneDimJob{c->zmin + i * (c->zmax - c->zmin) / nb, 0, 0};
+  std::vector<OneDimGroup> groups;
+  groups.reserve(2 * (size_t)count);
+  for (int s = first; s < first + count; ++s)
+    for (int which = 0; which < 2; ++which) {
+      OneDimGroup g{};
+      g.h = to_dev(which == 0 ? c->sets[s].h1 : c->sets[s].h2);
+      g.lo = std::log10(c->mmin_i);
+      g.hi = std::log10(c->mmax_i);
+      g.out = const_cast<double *>(nbar_ptr(c, s, which));
+      g.count = (uint32_t)nb;
+      g.mode = kOneDNbar;
+      groups.push_back(g);
     }
-    std::vector<JobState> st;
-    g3l_batch_stats keep = c->last;
-    int rc = run_engine(c, E, st, false, G3L_FP64);
-    c->last = keep;
-    if (rc) return rc;
-    std::vector<double> nbv(st.size());
-    for (size_t j = 0; j < st.size(); ++j) {
-      if (st[j].flags & (kJobPoolFull | kJobNonfinite)) return status_of(st[j].flags);
-      nbv[j] = kLn10 * st[j].val;
-    }
-    // copy run by run: sets s0..s1 may straddle two storage chunks
-    for (int s = s0; s < s1;) {
-      int e = std::min(s1, (s / kSetsPerChunk + 1) * kSetsPerChunk);
-      G3L_HIP(hipMemcpy(const_cast<double *>(nbar_ptr(c, s, 0)), nbv.data() + (size_t)(s - s0) * 2 * nb,
-                        (size_t)(e - s) * 2 * nb * sizeof(double), hipMemcpyHostToDevice));
-      s = e;
-    }
-  }
-  return G3L_OK;
+  return run_one_dim(c, groups, zs, false, 1e-4, kLn10);
 }
 
 }  // namespace
@@ -724,6 +763,7 @@ int g3l_ctx_destroy(g3l_ctx *c) {
   c->state.release(); c->args.release(); c->boxes.release(); c->counters.release();
   c->hcounters.release();
   c->trace.release();
+  c->od_store.release(); c->od_in.release();
   c->pgeo.release(); c->psplit.release(); c->plist.release(); c->pjob.release();
   c->parg.release(); c->hgeo.release(); c->hsplit.release();
   for (auto &e : c->ev)

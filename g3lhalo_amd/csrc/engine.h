@@ -9,6 +9,7 @@
 #include "../../include/g3l.h"
 #include "kernels.h"
 #include "layout.h"
+#include "onedim.h"
 #include "physics.h"
 
 #define G3L_HIP(expr)                                           \
@@ -137,6 +138,8 @@ struct g3l_ctx {
   // batched engine
   DevBuf pool, split, lists, jobs, state, args, boxes, counters;
   HostBuf hcounters;
+  // 1-D integrals: node stores of the resident blocks, inputs, outcome
+  DevBuf od_store, od_in;
   // plain engine
   DevBuf pgeo, psplit, plist, pjob, parg;
   HostBuf hgeo, hsplit;
@@ -213,6 +216,12 @@ int refine_jobs(g3l_ctx *c, const EngineBufs &B, uint32_t nj, bool timed, int pr
 // Evaluation counts and wall time of c->last from the final states.
 void finish_stats(g3l_ctx *c, const JobDesc *desc, const JobState *st, uint32_t nj,
                   double wall_ms);
+// Refines every 1-D integral of the groups (sharing the parameter table jobs)
+// on c's stream and waits for them; group g's integral i leaves scale * value
+// in g.out[i] (device memory).  The status of the first integral, by group and
+// index, that ran out of regions or met a non-finite value, if any does.
+int run_one_dim(g3l_ctx *c, const std::vector<OneDimGroup> &groups,
+                const std::vector<OneDimJob> &jobs, bool precomp, double reltol, double scale);
 // A context with a stream and timing events but no tables, for engine runs
 // whose integrands need none (the table precomputation).
 int ctx_create_bare(g3l_ctx **out);

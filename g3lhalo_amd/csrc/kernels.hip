@@ -53,7 +53,6 @@ __host__ __device__ constexpr int make_kv(int kind, int v) { return kind | (v <<
 // 1 and 2 take fewer regions so that more blocks share a compute unit and
 // one block's barriers overlap another's work, and variant 3 is a group
 // size whose points fill their waves closely:
-//   n_bar  (1-D): 68 regions x 15 points = 1020 threads (all variants);
 //   1-halo (5-D): 11 x 93 = 1023 points, 5 x 93 = 465 of 512, 2 x 93 = 186 of 192,
 //                 4 x 93 = 372 of 384;
 //   2-halo (6-D):  6 x 149 = 894 points of 896 (u_NFW pass 6 x 318 = 1908 in
@@ -66,8 +65,7 @@ struct KGroup {
   static constexpr int D = kind_dim(kind_of_kv(KV));
   static constexpr int V = variant_of_kv(KV);
   static constexpr int P = rule_points(D);
-  static constexpr int G = D == 1   ? 68
-                           : D == 5 ? (V == 3 ? 4 : V == 2 ? 2 : V ? 5 : 11)
+  static constexpr int G = D == 5   ? (V == 3 ? 4 : V == 2 ? 2 : V ? 5 : 11)
                            : D == 6 ? (V == 3 ? 3 : V == 2 ? 1 : V ? 2 : 6)
                                     : (V == 3 ? 3 : V == 2 ? 1 : V ? 2 : 4);
   // the 2-halo kinds at three regions take 512 threads rather than 448, so
@@ -76,7 +74,7 @@ struct KGroup {
   static_assert(NT <= 1024, "one block holds every point of its regions");
 };
 
-// Region staging shared by both evaluation kernels: centre, half-width,
+// Region staging of the evaluation kernels: centre, half-width,
 // volume, slot and integral parameters of the block's regions.
 template <int D, int G>
 struct Stage {
@@ -131,69 +129,31 @@ __device__ __forceinline__ int stage_regions(const EvalLaunch &L, Stage<D, G> &S
   return ng;
 }
 
-// Rule reduction of the block's regions from the point values in f.  For the
-// Genz-Malik rule lanes 2g and 2g + 1 of the first wave sum region g's 4th
-// and 5th point groups (gm_group_sum), and lane 2g finishes the region.
+// Rule reduction of the block's regions from the point values in f: lanes 2g
+// and 2g + 1 of the first wave sum region g's 4th and 5th point groups
+// (gm_group_sum), and lane 2g finishes the region.
 template <int D, int G, int NP>
 __device__ __forceinline__ void reduce_regions(const EvalLaunch &L, const Stage<D, G> &S,
                                                const double *f, int ng) {
   const int tid = threadIdx.x;
   const uint64_t St = L.stride;
-  if constexpr (D == 1) {
-    if (tid < ng && S.slot[tid] != 0xffffffffu) {
+  static_assert(2 * G <= 64, "a region's two lanes are in the first wave");
+  if (tid < 2 * ng) {
+    const int g = tid >> 1;
+    const bool fifth = tid & 1;
+    const double *v = f + g * NP;
+    const double s = gm_group_sum<D>(v, fifth);
+    const double s5 = __shfl_xor(s, 1);   // every lane below 2 ng is here
+    if (!fifth && S.slot[g] != 0xffffffffu) {
       double val, err;
-      gk_reduce(f + tid * NP, S.h[tid][0], val, err);
-      const uint32_t sl = S.slot[tid];
+      int split = 0;
+      gm_finish<D>(v, S.vol[g], s, s5, val, err, split);
+      const uint32_t sl = S.slot[g];
       L.geo[kFieldVal * St + sl] = val;
       L.geo[kFieldErr * St + sl] = err;
-      L.split[sl] = 0;
-    }
-  } else {
-    static_assert(2 * G <= 64, "a region's two lanes are in the first wave");
-    if (tid < 2 * ng) {
-      const int g = tid >> 1;
-      const bool fifth = tid & 1;
-      const double *v = f + g * NP;
-      const double s = gm_group_sum<D>(v, fifth);
-      const double s5 = __shfl_xor(s, 1);   // every lane below 2 ng is here
-      if (!fifth && S.slot[g] != 0xffffffffu) {
-        double val, err;
-        int split = 0;
-        gm_finish<D>(v, S.vol[g], s, s5, val, err, split);
-        const uint32_t sl = S.slot[g];
-        L.geo[kFieldVal * St + sl] = val;
-        L.geo[kFieldErr * St + sl] = err;
-        L.split[sl] = (uint8_t)split;
-      }
+      L.split[sl] = (uint8_t)split;
     }
   }
-}
-
-// Direct evaluation (n_bar): every point evaluates its integrand in full.
-// Held to 64 VGPRs (8 waves per SIMD, two 1024-thread blocks per CU) as
-// k_eval is: the 256-HOD n_bar sweep runs 148 ms instead of 158 ms at 88.
-template <int KIND, class P>
-__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8))) void k_eval_direct(EvalLaunch L) {
-  constexpr int D = kind_dim(kind_of_kv(KIND));
-  constexpr int NP = KGroup<KIND>::P;
-  constexpr int G = KGroup<KIND>::G;
-  constexpr int NT = KGroup<KIND>::NT;
-  __shared__ Stage<D, G> S;
-  __shared__ double s_f[G * NP];
-  if (block_group() * G >= L.count) return;
-  const int ng = stage_regions<D, G, NT>(L, S);
-  const int tid = threadIdx.x;
-  const DevTables T = L.T;
-  if (tid < ng * NP) {
-    const int g = tid / NP, q = tid - g * NP;
-    if (S.slot[g] != 0xffffffffu) {
-      double x[D];
-      rule_point<D>(q, S.c[g], S.h[g], x);
-      s_f[tid] = integrand<kind_of_kv(KIND), P>(T, S.args[g], x);
-    }
-  }
-  __syncthreads();
-  reduce_regions<D, G, NP>(L, S, s_f, ng);
 }
 
 // ---------------------------------------------------- factored evaluation
@@ -1604,11 +1564,7 @@ static hipError_t launch_eval_kind(const EvalLaunch &L, hipStream_t s) {
   using Gr = KGroup<KV>;
   uint32_t blocks = (L.count + Gr::G - 1) / Gr::G;
   if (blocks == 0) return hipSuccess;
-  if constexpr (kind_of_kv(KV) == kNbar) {
-    hipLaunchKernelGGL((k_eval_direct<KV, P>), dim3(blocks), dim3(Gr::NT), 0, s, L);
-  } else {
-    hipLaunchKernelGGL((k_eval<KV, P>), dim3(blocks), dim3(Gr::NT), 0, s, L);
-  }
+  hipLaunchKernelGGL((k_eval<KV, P>), dim3(blocks), dim3(Gr::NT), 0, s, L);
   return hipGetLastError();
 }
 
@@ -1626,7 +1582,6 @@ static hipError_t launch_eval_variant(int kind, const EvalLaunch &L, hipStream_t
 }
 
 hipError_t launch_eval(int kind, int prec, int variant, const EvalLaunch &L, hipStream_t s) {
-  if (kind == kNbar) return launch_eval_kind<kNbar, P64>(L, s);
   if (variant < 0 || variant >= kNumVariants) return hipErrorInvalidValue;
   if (prec == 0) {
     if (variant == 3) return launch_eval_variant<3, P64>(kind, L, s);
@@ -1645,10 +1600,7 @@ template <int KV, class P>
 static KernelRef eval_ref_kind() {
   using Gr = KGroup<KV>;
   KernelRef r;
-  if constexpr (kind_of_kv(KV) == kNbar)
-    r.fn = reinterpret_cast<const void *>(&k_eval_direct<KV, P>);
-  else
-    r.fn = reinterpret_cast<const void *>(&k_eval<KV, P>);
+  r.fn = reinterpret_cast<const void *>(&k_eval<KV, P>);
   r.threads = (unsigned)Gr::NT;
   r.group = (unsigned)Gr::G;
   return r;
@@ -1668,10 +1620,6 @@ static int eval_ref_variant(int kind, KernelRef *out) {
 }
 
 int eval_kernel_ref(int kind, int prec, int variant, KernelRef *out) {
-  if (kind == kNbar) {
-    *out = eval_ref_kind<kNbar, P64>();
-    return 0;
-  }
   if (variant < 0 || variant >= kNumVariants) return -1;
   if (prec == 0) {
     if (variant == 3) return eval_ref_variant<3, P64>(kind, out);
@@ -1690,7 +1638,7 @@ KernelRef zero_kernel_ref() { return KernelRef{reinterpret_cast<const void *>(&k
 
 int eval_group_size(int kind, int variant) {
   const int d = kind_dim(kind);
-  if (d == 1) return KGroup<kNbar>::G;
+  if (d == 1) return 0;   // 1-D integrals have no launch shapes (onedim.hip)
   const int k = d == 5 ? kNN1 : d == 6 ? kNN2 : kNN3;
   if (variant == 3) {
     return k == kNN1 ? KGroup<make_kv(kNN1, 3)>::G

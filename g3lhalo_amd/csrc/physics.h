@@ -198,16 +198,12 @@ struct TermArgs {
   int same;                 // NsatNsat same-type branch
   // log-space HOD constants of PMix: log(mmin/M_th), log(mmin/M'), log(mmin)
   double lth1, lmp1, lth2, lmp2, lmmin;
-  // 1-D integrands: kOneDNbar, or a table-precomputation integral whose
-  // cosmology and transfer-function parameters are at aux (PrecompParams)
-  int mode;
-  const double *aux;
 };
 
 // ---------------------------------------------------- table precomputation
 // The 1-D integrands of the reference's table precomputation
-// (src/Cosmology.cpp:84-118, src/Powerspectrum.cpp:71-284), evaluated by the
-// batched GK15 engine like n_bar, with the per-integral parameters in t1..t3.
+// (src/Cosmology.cpp:84-118, src/Powerspectrum.cpp:71-284), refined like n_bar
+// by k_onedim, with the per-integral parameters in OneDimJob's t1..t3.
 enum OneDMode : int {
   kOneDNbar = 0,       // n_bar(z) (t1 = z)
   kOneDComoving = 1,   // c / H0 / sqrt(E(z))               -> w(z)
@@ -263,30 +259,17 @@ G3L_HD double eh_spectrum(const PrecompParams &p, double k, double growth) {
   return p.amplitude * trans * trans * growth * growth * pow(k, p.ns);
 }
 
-// One precomputation integrand value at x (src/Cosmology.cpp:104-118,
-// src/Powerspectrum.cpp:71-95, 229-245, 265-284).
-G3L_HD double precomp_kernel(const TermArgs &a, double x) {
-  const PrecompParams &p = *reinterpret_cast<const PrecompParams *>(a.aux);
-  switch (a.mode) {
-    case kOneDComoving: {
-      const double zp = 1 + x;
-      return p.c / p.H0 / sqrt(p.Om * zp * zp * zp + p.OL);
-    }
-    case kOneDAmplitude: {
-      const double W = tophat(x, a.t1);
-      const double T = eh_transfer(p, x);
-      return W * W * T * T * pow(x, p.ns + 2);
-    }
-    case kOneDSigma2: {
-      const double W = tophat(x, a.t1);
-      return x * x * W * W * eh_spectrum(p, x, a.t2);
-    }
-    default: {
-      const double W = tophat(x, a.t1);
-      const double Wprime = d_tophat(x, a.t1);
-      return x * x * W * Wprime * a.t3 * eh_spectrum(p, x, a.t2);
-    }
-  }
+// The distance and sigma8 integrands (src/Cosmology.cpp:104-118,
+// src/Powerspectrum.cpp:71-95); those of sigma^2 and d sigma^2/dm are put
+// together in k_onedim from the window and the spectrum.
+G3L_HD double precomp_distance(const PrecompParams &p, double x) {
+  const double zp = 1 + x;
+  return p.c / p.H0 / sqrt(p.Om * zp * zp * zp + p.OL);
+}
+G3L_HD double precomp_amplitude(const PrecompParams &p, double x, double R) {
+  const double W = tophat(x, R);
+  const double T = eh_transfer(p, x);
+  return W * W * T * T * pow(x, p.ns + 2);
 }
 
 // ---------------------------------------------------------------- indices
@@ -1230,12 +1213,10 @@ G3L_HD double integrand_src(const DevTables &T, const TermArgs &a, const S &s) {
   }
 }
 
-// n_bar integrand, x = log10 m, theta slot 1 = z (src/generalFunctions.cu:233-244);
-// the table-precomputation integrands share its 1-D kind (mode != kOneDNbar).
+// n_bar integrand, x = log10 m, theta slot 1 = z (src/generalFunctions.cu:233-244).
 template <class P>
 G3L_HD double nbar_kernel(const DevTables &T, const TermArgs &a,
                                               const double *x) {
-  if (a.mode != kOneDNbar) return precomp_kernel(a, x[0]);
   double z = a.t1;
   int zr = zix_round(T, z);
   Mass M = make_mass<P>(T, x[0], zix_trunc(T, z));

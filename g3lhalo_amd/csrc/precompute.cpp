@@ -2,8 +2,8 @@
 // redshift distribution (g3l_precompute), the device counterpart of the
 // reference's doPrecomputations.x (src/doPrecomputations.cpp:7-135).
 //
-// All adaptive integrals run as jobs of the batched 1-D Gauss-Kronrod engine
-// (the n_bar kind, integrand modes of physics.h): first the sigma8
+// All adaptive integrals run on the device's 1-D Gauss-Kronrod kernel
+// (k_onedim, integrand modes of physics.h): first the sigma8
 // normalisation and the comoving distances of the grid and of the source
 // redshifts, then sigma^2(m, z) and d sigma^2/dm on the model grid and
 // sigma^2 on the 256-mass grid of m*(z) -- about 4 N^2 integrals at N bins,
@@ -84,52 +84,26 @@ void eh_params(const Cosmo &c, PrecompParams &p) {
   p.beta_b = 0.5 + f_baryon + (3.0 - 2.0 * f_baryon) * std::sqrt(std::pow(17.2 * omhh, 2.0) + 1.0);
 }
 
-// One 1-D job of the engine over [lo, hi] (the settings of every integral
-// of the precomputation: tol 1e-4, no evaluation cap).
-void add_job(EngineJobs &E, int mode, double lo, double hi, const double *aux, double t1,
-             double t2, double t3) {
-  JobDesc d{};
-  d.kind = kNbar;
-  d.dim = 1;
-  d.pts = 15;
-  d.args = (int)E.args.size();
-  d.cap = 2048;
-  d.reltol = 1e-4;
-  d.maxeval = 0;
-  TermArgs a{};
-  a.mode = mode;
-  a.aux = aux;
-  a.t1 = t1;
-  a.t2 = t2;
-  a.t3 = t3;
-  E.args.push_back(a);
-  E.desc.push_back(d);
-  double box[2 * kMaxDim] = {0};
-  box[0] = lo;
-  box[kMaxDim] = hi;
-  E.boxes.insert(E.boxes.end(), box, box + 2 * kMaxDim);
+// One group of integrals over [lo, hi] (the settings of every integral of the
+// precomputation: tol 1e-4, no evaluation cap).
+OneDimGroup group_of(int mode, double lo, double hi, const double *aux, size_t job0, size_t count,
+                     double *out) {
+  OneDimGroup g{};
+  g.mode = mode;
+  g.lo = lo;
+  g.hi = hi;
+  g.aux = aux;
+  g.job0 = (uint32_t)job0;
+  g.count = (uint32_t)count;
+  g.out = out;
+  return g;
 }
+constexpr double kPrecompTol = 1e-4;
 
-// Runs the jobs in chunks that bound the region pool; values in job order.
-int run_jobs(g3l_ctx *c, EngineJobs &all, std::vector<double> &val) {
-  const size_t n = all.desc.size(), chunk = 16384;
-  val.assign(n, 0.0);
-  for (size_t s0 = 0; s0 < n; s0 += chunk) {
-    const size_t s1 = std::min(n, s0 + chunk);
-    EngineJobs E;
-    E.desc.assign(all.desc.begin() + s0, all.desc.begin() + s1);
-    E.args.assign(all.args.begin() + s0, all.args.begin() + s1);
-    E.boxes.assign(all.boxes.begin() + s0 * 2 * kMaxDim, all.boxes.begin() + s1 * 2 * kMaxDim);
-    for (auto &d : E.desc) d.args -= (int)s0;
-    std::vector<JobState> st;
-    if (int rc = run_engine(c, E, st, false, G3L_FP64)) return rc;
-    for (size_t j = 0; j < st.size(); ++j) {
-      if (st[j].flags & (kJobPoolFull | kJobNonfinite)) return status_of(st[j].flags);
-      val[s0 + j] = st[j].val;
-    }
-  }
-  return G3L_OK;
-}
+// A device buffer freed with its scope.
+struct OwnedBuf : DevBuf {
+  ~OwnedBuf() { release(); }
+};
 
 int precompute(g3l_ctx *c, const g3l_precompute_in &in, g3l_precompute_out &out) {
   const int N = in.nbins;
@@ -153,7 +127,7 @@ int precompute(g3l_ctx *c, const g3l_precompute_in &in, g3l_precompute_out &out)
   P.c = cs.c;
   P.ns = cs.ns;
   eh_params(cs, P);
-  DevBuf aux;
+  OwnedBuf aux;
   if (int rc = aux.ensure(sizeof(PrecompParams))) return rc;
   const double *daux = aux.as<double>();
   G3L_HIP(hipMemcpy(aux.p, &P, sizeof(P), hipMemcpyHostToDevice));
@@ -162,12 +136,23 @@ int precompute(g3l_ctx *c, const g3l_precompute_in &in, g3l_precompute_out &out)
   // comoving distances of the grid and of the source redshifts
   // (src/Cosmology.cpp:91-102)
   const int Ns = in.nz_count;
-  EngineJobs E1;
-  add_job(E1, kOneDAmplitude, 0, 1e12, daux, 8. / cs.H0 * 100, 0, 0);
-  for (int i = 0; i < N; ++i) add_job(E1, kOneDComoving, 0, zs[i], daux, 0, 0, 0);
-  for (int i = 0; i < Ns; ++i) add_job(E1, kOneDComoving, 0, in.nz_z[i], daux, 0, 0, 0);
-  std::vector<double> v1;
-  if (int rc = run_jobs(c, E1, v1)) return rc;
+  const size_t n1 = N, n2 = (size_t)N * N;
+  constexpr int kNStar = 256;
+  const size_t nstar = n1 * kNStar;
+  // values of the integrals: amplitude, distances (grid, sources), sigma^2
+  // (grid, m* grid), d sigma^2/dm
+  OwnedBuf vals;
+  if (int rc = vals.ensure((1 + n1 + Ns + 2 * n2 + nstar) * sizeof(double))) return rc;
+  double *dv1 = vals.as<double>(), *dv2 = dv1 + 1 + n1 + Ns;
+  std::vector<OneDimGroup> G;
+  std::vector<OneDimJob> J = {OneDimJob{8. / cs.H0 * 100, 0, 0}};
+  G.push_back(group_of(kOneDAmplitude, 0, 1e12, daux, 0, 1, dv1));
+  for (int i = 0; i < N; ++i) G.push_back(group_of(kOneDComoving, 0, zs[i], daux, 0, 1, dv1 + 1 + i));
+  for (int i = 0; i < Ns; ++i)
+    G.push_back(group_of(kOneDComoving, 0, in.nz_z[i], daux, 0, 1, dv1 + 1 + N + i));
+  if (int rc = run_one_dim(c, G, J, true, kPrecompTol, 1.0)) return rc;
+  std::vector<double> v1(1 + n1 + Ns);
+  G3L_HIP(hipMemcpy(v1.data(), dv1, v1.size() * sizeof(double), hipMemcpyDeviceToHost));
   const double factor = kPiExact * cs.s8;
   P.amplitude = 2 * factor * factor / v1[0];
   G3L_HIP(hipMemcpy(aux.p, &P, sizeof(P), hipMemcpyHostToDevice));
@@ -177,13 +162,14 @@ int precompute(g3l_ctx *c, const g3l_precompute_in &in, g3l_precompute_out &out)
   // src/Powerspectrum.cpp:209-263) and sigma^2 on m*'s 256-mass grid
   // (src/Powerspectrum.cpp:110-126)
   const double D0 = cs.growth(0.0);
-  constexpr int kNStar = 256;
   const double mstar_min = 1e10, mstar_max = 1e18;
   const double mstar_bin = std::log(mstar_max / mstar_min) / kNStar;
   std::vector<double> mgrid(kNStar);
   for (int s = 0; s < kNStar; ++s) mgrid[s] = std::exp(std::log(mstar_min) + mstar_bin * s);
-  EngineJobs E2;
   std::vector<double> growth(N), delta_c(N), rho_mean(N);
+  // parameters: sigma^2 on the model grid, on the m* grid, d sigma^2/dm
+  J.assign(2 * n2 + nstar, OneDimJob{});
+  OneDimJob *Js = J.data(), *Jm = Js + n2, *Jd = Jm + nstar;
   for (int i = 0; i < N; ++i) {
     const double z = zs[i];
     growth[i] = cs.growth(z) / D0;
@@ -194,31 +180,34 @@ int precompute(g3l_ctx *c, const g3l_precompute_in &in, g3l_precompute_out &out)
     for (int j = 0; j < N; ++j) {
       const double m = ms[j];
       const double R = std::pow(0.75 / kPiExact * m / rho_crit / om, 1. / 3.);
-      add_job(E2, kOneDSigma2, 0, 1e12, daux, R, growth[i], 0);
+      *Js++ = OneDimJob{R, growth[i], 0};
       const double Rd = 0.6204 * std::pow(m / rho_m, 1. / 3.);
       const double dR = 0.2068 * std::pow(rho_m * m * m, -1. / 3.);
-      add_job(E2, kOneDDSigma2, 0, 1e12, daux, Rd, growth[i], dR);
+      *Jd++ = OneDimJob{Rd, growth[i], dR};
     }
     for (int s = 0; s < kNStar; ++s) {
       const double R = std::pow(0.75 / kPiExact * mgrid[s] / rho_crit / om, 1. / 3.);
-      add_job(E2, kOneDSigma2, 0, 1e12, daux, R, growth[i], 0);
+      *Jm++ = OneDimJob{R, growth[i], 0};
     }
   }
-  std::vector<double> v2;
-  if (int rc = run_jobs(c, E2, v2)) return rc;
-  const size_t per_z = 2 * (size_t)N + kNStar;
-  std::vector<double> sig2((size_t)N * N), dsig2((size_t)N * N), mstar(N);
+  G.clear();
+  G.push_back(group_of(kOneDSigma2, 0, 1e12, daux, 0, n2 + nstar, dv2));
+  G.push_back(group_of(kOneDDSigma2, 0, 1e12, daux, n2 + nstar, n2, dv2 + n2 + nstar));
+  if (int rc = run_one_dim(c, G, J, true, kPrecompTol, 1.0)) return rc;
+  std::vector<double> v2(2 * n2 + nstar);
+  G3L_HIP(hipMemcpy(v2.data(), dv2, v2.size() * sizeof(double), hipMemcpyDeviceToHost));
+  const double *vstar = v2.data() + n2, *vdsig = vstar + nstar;
+  std::vector<double> sig2(n2), dsig2(n2), mstar(N);
   for (int i = 0; i < N; ++i) {
-    const double *v = v2.data() + i * per_z;
     for (int j = 0; j < N; ++j) {
-      sig2[(size_t)i * N + j] = v[2 * j] / 2 / kPiExact / kPiExact;
-      dsig2[(size_t)i * N + j] = v[2 * j + 1] / kPiExact / kPiExact;
+      sig2[(size_t)i * N + j] = v2[(size_t)i * N + j] / 2 / kPiExact / kPiExact;
+      dsig2[(size_t)i * N + j] = vdsig[(size_t)i * N + j] / kPiExact / kPiExact;
     }
     // m*(z): the first grid mass with the smallest |delta_c - sigma|
     int best = 0;
     double bestd = 0;
     for (int s = 0; s < kNStar; ++s) {
-      const double diff = delta_c[i] - std::sqrt(v[2 * N + s] / 2 / kPiExact / kPiExact);
+      const double diff = delta_c[i] - std::sqrt(vstar[(size_t)i * kNStar + s] / 2 / kPiExact / kPiExact);
       const double d = std::sqrt(diff * diff);
       if (s == 0 || d < bestd) {
         bestd = d;
@@ -243,8 +232,7 @@ int precompute(g3l_ctx *c, const g3l_precompute_in &in, g3l_precompute_out &out)
   }
 
   // 2-D tables on the device
-  const size_t n1 = N, n2 = (size_t)N * N;
-  DevBuf dbuf;
+  OwnedBuf dbuf;
   if (int rc = dbuf.ensure((7 * n1 + 6 * n2) * sizeof(double))) return rc;
   double *d = dbuf.as<double>();
   double *dzs = d, *dms = d + n1, *dks = d + 2 * n1, *dgr = d + 3 * n1, *ddc = d + 4 * n1,
