@@ -249,7 +249,7 @@ int refine_jobs(g3l_ctx *c, const EngineBufs &B, uint32_t nj, bool timed, int pr
     if (!graph.exec || key != c->graph_key) {
       c->graph_key.clear();
       if ((rc = graph.build(in_run, KL.prec, KL.variant, EL, SL, dcnt, kNumKinds + 1, hcnt, c->ev,
-                            c->kev)))
+                            c->kev, nj)))
         return rc;
       c->graph_key = key;
     }

@@ -99,6 +99,7 @@ struct RoundGraph {
   EvalLaunch eval_args[kNumKinds] = {};
   void *eval_params[kNumKinds][1] = {};
   hipGraphNode_t select_node = nullptr;
+  KernelRef select_ref = {};   // for the number of integrals it was built for
   SelectLaunch sel_args{};
   void *sel_params[1] = {};
   uint32_t *zero_ptr = nullptr;
@@ -108,7 +109,10 @@ struct RoundGraph {
   // bracket kind k's evaluation
   int build(const bool used[kNumKinds], const int prec[kNumKinds], const int variant[kNumKinds],
             const EvalLaunch &eval_base, const SelectLaunch &sel_base, uint32_t *dcounters,
-            int ncounters, uint32_t *hcounters, const hipEvent_t *ev, const hipEvent_t *kev);
+            int ncounters, uint32_t *hcounters, const hipEvent_t *ev, const hipEvent_t *kev,
+            uint32_t nselect);
+  // whether the selection kernel it holds is the one for nselect integrals
+  bool selects(uint32_t nselect) const { return select_kernel_ref(nselect).fn == select_ref.fn; }
   int launch(const uint32_t count[kNumKinds], EvalItem *const lists[kNumKinds], uint32_t nselect,
              hipStream_t s);
   void destroy();

@@ -96,7 +96,7 @@ struct KernelRef {
   unsigned group;
 };
 int eval_kernel_ref(int kind, int prec, int variant, KernelRef *out);
-KernelRef select_kernel_ref();   // k_select(SelectLaunch), one block per job
+KernelRef select_kernel_ref(uint32_t njobs);   // k_select(SelectLaunch), one block per job
 KernelRef zero_kernel_ref();     // k_zero(uint32_t *p, int n)
 
 // variant: block shape, 0 .. eval_num_variants() - 1 (the same values for all)

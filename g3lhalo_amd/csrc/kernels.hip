@@ -17,10 +17,18 @@
 #include "physics.h"
 #include "rules.h"
 #include "select_math.h"
+#include "select_wave.h"
 
 #pragma clang fp contract(off)
 
 namespace g3l {
+
+// Most integrals for which k_select takes 1024 threads each; the blocks of more
+// hide one another's latency better at 256.  Selection time of a whole run at
+// 256 / 1024 threads: 9 integrals of 5e6 evaluations 1.43 / 1.11 ms, 411 2.06 /
+// 1.80, 1650 5.16 / 4.68; 1500 of 2e5 evaluations 1.03 / 1.15, 9000 of 1e6
+// 7.12 / 8.72.
+constexpr uint32_t kSelectWideJobs = 512;
 
 // ------------------------------------------------------------ evaluation
 template <int KIND, class P>
@@ -74,8 +82,8 @@ struct KGroup {
   static_assert(NT <= 1024, "one block holds every point of its regions");
 };
 
-// Region staging of the evaluation kernels: centre, half-width,
-// volume, slot and integral parameters of the block's regions.
+// Region staging of the evaluation kernels: centre, half-width, volume, slot
+// and integral parameters of the block's regions.
 template <int D, int G>
 struct Stage {
   double c[G][D];
@@ -961,528 +969,630 @@ __global__ void k_zero(uint32_t *p, int n) {
 }
 
 // ---------------------------------------------------------------- select
-// One 256-thread block (4 waves of 64 lanes) per integral.  The passes over
-// the integral's regions are latency-bound (one block per integral, a few
-// hundred iterations per thread for the largest), so each iteration issues
-// four independent loads, and the scans use wave shuffles rather than
-// thread-serial loops.
-constexpr int kSelThreads = 256;
+// One block per integral: totals, stop tests, the Gladwell batch and its cuts.
+// It is bound by latency -- passes over the integral's errors in memory, with
+// few bytes each -- so the passes are few (totals; a histogram; the keys near
+// the batch's boundary; the cuts) and wide: 1024 threads per integral up to
+// kSelectWideJobs integrals, 256 beyond.  Up to 256 regions one wave does it
+// all, from registers and without a barrier.  An earlier form with 256 threads
+// and eight radix levels, each a pass over the errors, took 2.47 ms for a run
+// of 9 integrals and 6.9 ms for 1650 (now 1.11 and 5.2).
+//
+// Both thread counts and the one-wave form add in the same order and select by
+// the same rule: an integral's result does not depend on which of them runs.
 
-__device__ __forceinline__ uint64_t shfl_up_u64(uint64_t v, unsigned d) {
-  const uint32_t lo = __shfl_up((uint32_t)v, d, 64), hi = __shfl_up((uint32_t)(v >> 32), d, 64);
-  return ((uint64_t)hi << 32) | lo;
+// The totals' order: 256 partial sums over i = t, t + 256, ..., then pairwise
+// (t, t + 128), (t, t + 64), ..., (0, 1); value compensated, error plain.
+constexpr int kPartial = 256;
+
+template <int NT>
+struct SelectLds {
+  JobState st;
+  double vs[kPartial], vc[kPartial], es[kPartial];
+  uint64_t kmax[NT / 64];
+  uint32_t bad;
+  // histogram of the keys' distance below the largest, eight bins per octave
+  unsigned long long sum[256];
+  uint32_t cnt[256];
+  uint64_t lo, width;            // the bin that holds the boundary
+  uint32_t m, above;
+  unsigned long long rest;
+  // candidates: keys of that bin
+  uint64_t key[1024];
+  uint32_t nkey;
+  double bs[NT / 64], bc[NT / 64];
+  uint32_t wcnt[NT / 64], wtie[NT / 64];
+  SearchLds search;
+  Boundary B;
+  double V, E;
+  uint64_t maxkey;
+  int found, stop;
+  uint32_t listbase;
+  uint32_t sel[4 * NT];          // slots cut in one chunk, ascending
+};
+
+// Ends a job's selection: state to memory, the job to the done list.
+__device__ __forceinline__ void select_finish(const SelectLaunch &L, uint32_t J, const JobState &st) {
+  L.state[J] = st;
+  if (L.done) L.done[atomicAdd(&L.counters[kNumKinds + 1], 1u)] = J;
 }
 
-// Inclusive prefix sums over the block in thread order of (a, b); s_wa, s_wb
-// hold the wave totals (4 each).  Ends with a barrier, so the buffers can be
-// reused at once; ta, tb receive the block totals.
-__device__ __forceinline__ void block_scan2(uint64_t &a, uint64_t &b, uint64_t *s_wa,
-                                            uint64_t *s_wb, uint64_t &ta, uint64_t &tb) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-#pragma unroll
-  for (unsigned d = 1; d < 64; d <<= 1) {
-    const uint64_t xa = shfl_up_u64(a, d), xb = shfl_up_u64(b, d);
-    if (lane >= (int)d) {
-      a += xa;
-      b += xb;
-    }
+// Stop tests in the order of src/hcubature.cpp:938-939 on totals (V, E).
+__device__ __forceinline__ bool select_stops(const JobDesc &d, double V, double E, bool nonfinite,
+                                             JobState &st) {
+  st.val = V;
+  st.err = E;
+  if (nonfinite) st.flags |= kJobNonfinite;
+  if (d.maxeval != 0 && st.neval >= d.maxeval) {
+    st.flags |= kJobDone | kJobCapped;
+    return true;
   }
-  if (lane == 63) {
-    s_wa[wave] = a;
-    s_wb[wave] = b;
+  if (!(E > 0 && E > fabs(V) * d.reltol)) {
+    st.flags |= kJobDone | kJobConverged;
+    return true;
   }
-  __syncthreads();
-  uint64_t oa = 0, ob = 0;
-  for (int w = 0; w < wave; ++w) {
-    oa += s_wa[w];
-    ob += s_wb[w];
-  }
-  ta = s_wa[0] + s_wa[1] + s_wa[2] + s_wa[3];
-  tb = s_wb[0] + s_wb[1] + s_wb[2] + s_wb[3];
-  a += oa;
-  b += ob;
-  __syncthreads();
+  return false;
 }
 
-// Block-wide reductions over an integral's error keys for the exact stopping
-// point: the FP64 sum of the errors whose key is below T (Neumaier, each
-// thread over its strided entries, then a fixed tree), and the largest key
-// below T or smallest key above T with its multiplicity.  Every thread of the
-// block calls them; results are valid in every thread.
-__device__ double block_sum_below(const double *err, uint32_t n, uint64_t T, double *s_a,
-                                  double *s_b) {
-  const int tid = threadIdx.x;
-  double s = 0, c = 0;
-  for (uint32_t i = tid; i < n; i += kSelThreads) {
-    const uint64_t k = err_key(err[i]);
-    if (k >= T) continue;
-    const double e = __builtin_bit_cast(double, k);
-    const double t = s + e;
-    c += fabs(s) >= fabs(e) ? (s - t) + e : (e - t) + s;
-    s = t;
-  }
-  s_a[tid] = s;
-  s_b[tid] = c;
-  __syncthreads();
-  for (int w = kSelThreads / 2; w > 0; w >>= 1) {
-    if (tid < w) {
-      const double a = s_a[tid], b = s_a[tid + w];
-      const double t = a + b;
-      s_a[tid] = t;
-      s_b[tid] += s_b[tid + w] + (fabs(a) >= fabs(b) ? (a - t) + b : (b - t) + a);
-    }
-    __syncthreads();
-  }
-  const double r = s_a[0] + s_b[0];
-  __syncthreads();
-  return r;
+// The most regions the evaluation budget lets a batch pop.
+__device__ __forceinline__ uint64_t select_kcap(const JobDesc &d, const JobState &st) {
+  if (d.maxeval == 0) return st.n;
+  const uint64_t twoP = 2ull * (uint64_t)d.pts, room = d.maxeval - st.neval;
+  const uint64_t kc = (room + twoP - 1) / twoP;
+  return kc < st.n ? kc : st.n;
 }
 
-// below: the largest key < T; otherwise the smallest key > T.  Returns the
-// key (0 / ~0 when none) and sets cnt to its multiplicity.
-__device__ uint64_t block_next_key(const double *err, uint32_t n, uint64_t T, bool below,
-                                   uint64_t *s_k, uint32_t *s_c, uint32_t &cnt) {
-  const int tid = threadIdx.x;
-  uint64_t best = below ? 0ull : ~0ull;
-  bool any = false;
-  for (uint32_t i = tid; i < n; i += kSelThreads) {
-    const uint64_t k = err_key(err[i]);
-    if (below ? (k < T && (!any || k > best)) : (k > T && (!any || k < best))) {
-      best = k;
-      any = true;
-    }
+// Room for a batch of K regions: its place in the kind's list, or false when
+// the integral's slots or the list are full.  One thread calls it.
+__device__ __forceinline__ bool select_room(const SelectLaunch &L, const JobDesc &d, uint32_t K,
+                                            JobState &st, uint32_t &listbase) {
+  if (st.n + K > d.cap) {
+    st.flags |= kJobDone | kJobPoolFull;
+    return false;
   }
-  s_k[tid] = best;
-  s_c[tid] = any ? 1u : 0u;
-  __syncthreads();
-  for (int w = kSelThreads / 2; w > 0; w >>= 1) {
-    if (tid < w) {
-      const uint64_t a = s_k[tid], b = s_k[tid + w];
-      const uint32_t ha = s_c[tid], hb = s_c[tid + w];
-      if (hb && (!ha || (below ? b > a : b < a))) s_k[tid] = b;
-      s_c[tid] = ha | hb;
-    }
-    __syncthreads();
+  listbase = atomicAdd(&L.counters[d.kind], 2u * K);
+  if (listbase + 2u * K > L.list_cap[d.kind]) {
+    st.flags |= kJobDone | kJobPoolFull;
+    return false;
   }
-  const uint64_t key = s_k[0];
-  const bool found = s_c[0] != 0;
-  __syncthreads();
-  uint32_t m = 0;
-  if (found)
-    for (uint32_t i = tid; i < n; i += kSelThreads) m += err_key(err[i]) == key ? 1u : 0u;
-  s_c[tid] = m;
-  __syncthreads();
-  for (int w = kSelThreads / 2; w > 0; w >>= 1) {
-    if (tid < w) s_c[tid] += s_c[tid + w];
-    __syncthreads();
-  }
-  cnt = s_c[0];
-  __syncthreads();
-  return found ? key : (below ? 0ull : ~0ull);
+  atomicAdd(&L.counters[kNumKinds], 1u);
+  return true;
 }
 
-// Moves the batch boundary (key T with multiplicity cntT, `above` keys
-// larger than T, r of the T-ties taken) until the count K = above + r is the
-// first at which the remaining error meets thr (or K reaches kcap or n),
-// computing the remaining error in FP64.  Every thread calls it.
-__device__ void select_exact_count(const double *err, uint32_t n, uint64_t kcap, double thr,
-                                   uint64_t &T, uint32_t &cntT, uint32_t &above, uint32_t &r,
-                                   double *s_a, double *s_b, uint64_t *s_k, uint32_t *s_c) {
-  const int tid = threadIdx.x;
-  __shared__ double s_tail;
-  __shared__ int s_act;
-  const double below = block_sum_below(err, n, T, s_a, s_b);
-  if (tid == 0) s_tail = below + (double)(cntT - r) * __builtin_bit_cast(double, T);
-  // the loop ends: every step moves K by one towards the unique stopping count
-  for (int guard = 0; guard < 64; ++guard) {
-    if (tid == 0) {
-      double tail = s_tail;
-      int act = 0;
-      for (;;) {
-        const double eT = __builtin_bit_cast(double, T);
-        const uint64_t K = (uint64_t)above + r;
-        // not yet converged after K pops: pop one more (budget and regions left)
-        if (tail > 0 && tail > thr && K < kcap && K < n) {
-          if (r < cntT) {
-            ++r;
-            tail -= eT;
-            continue;
-          }
-          act = 1;  // the next key below T
-          break;
-        }
-        // converged already after K - 1 pops: one pop fewer
-        const double prev = tail + eT;
-        if (K > 1 && !(prev > 0 && prev > thr)) {
-          tail = prev;
-          if (r > 1) {
-            --r;
-            continue;
-          }
-          r = 0;
-          act = 2;  // the next key above T, all of its ties taken
-          break;
-        }
-        break;
-      }
-      s_tail = tail;
-      s_act = act;
-    }
-    __syncthreads();
-    const int act = s_act;
-    if (act == 0) break;
-    uint32_t c = 0;
-    const uint64_t nk = block_next_key(err, n, T, act == 1, s_k, s_c, c);
-    if (tid == 0) {
-      if (act == 1) {
-        above += cntT;
-        T = nk;
-        cntT = c;
-        r = 1;
-        s_tail -= __builtin_bit_cast(double, nk);
-      } else {
-        T = nk;
-        cntT = c;
-        above -= c;
-        r = c;
-      }
-    }
-    __syncthreads();
-  }
-}
-
-__global__ __launch_bounds__(kSelThreads) void k_select(SelectLaunch L) {
-  const uint32_t J = L.active ? L.active[blockIdx.x] : blockIdx.x;
-  const int tid = threadIdx.x;
-  __shared__ JobState s_st;
-  __shared__ double s_red[kSelThreads];
-  __shared__ double s_red2[kSelThreads];
-  __shared__ uint64_t s_redk[kSelThreads];
-  __shared__ uint32_t s_cnt[kSelThreads];
-  __shared__ unsigned long long s_sum[kSelThreads];
-  __shared__ uint64_t s_wa[4], s_wb[4];
-  __shared__ int s_flag;
-  __shared__ uint64_t s_prefix, s_mask, s_cumsum, s_need;
-  __shared__ uint32_t s_cumcnt, s_lastcnt, s_r, s_K, s_listbase;
-
-  if (tid == 0) s_st = L.state[J];
-  __syncthreads();
-  if (s_st.flags & kJobDone) return;
-  const JobDesc d = L.jobs[J];
+// Cuts the region in slot p along its split dimension, the a-th region of a
+// batch of K: the lower half keeps the slot, the upper one goes to slot q.  The
+// list holds the K kept slots first and the K new ones after them, both in
+// slot order, so that the regions an evaluation block stages sit in
+// neighbouring slots of each field.
+__device__ __forceinline__ void select_cut(const SelectLaunch &L, EvalItem *list, uint32_t J, int D,
+                                           uint32_t p, uint32_t q, uint32_t a, uint32_t K) {
   const uint64_t S = L.stride;
-  const uint32_t n = s_st.n;
-  const double *val = L.geo + kFieldVal * S + d.base;
-  const double *err = L.geo + kFieldErr * S + d.base;
-
-  // 1. totals: value with Neumaier compensation, error plain, each thread
-  //    over i = tid, tid + 256, ... in that order, then a fixed tree: the
-  //    result does not depend on scheduling.  Loads four at a time; absent
-  //    entries enter as zeros, which leave every sum unchanged.
-  double vs = 0, vc = 0, es = 0;
-  uint64_t kmax = 0;
-  bool bad = false;
-  for (uint32_t i0 = tid; i0 < n; i0 += 4 * kSelThreads) {
-    double v[4], e[4];
+  const int sd = L.split[p];
+  double c[kMaxDim], h[kMaxDim], hd = 0;
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const uint32_t i = i0 + u * kSelThreads;
-      v[u] = i < n ? val[i] : 0.0;
-      e[u] = i < n ? err[i] : 0.0;
+  for (int e = 0; e < kMaxDim; ++e) {
+    if (e < D) {
+      c[e] = L.geo[(kFieldC + e) * S + p];
+      h[e] = L.geo[(kFieldH + e) * S + p];
     }
+  }
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      bad |= !isfinite(v[u]) || !isfinite(e[u]);
-      const double t = vs + v[u];
-      vc += fabs(vs) >= fabs(v[u]) ? (vs - t) + v[u] : (v[u] - t) + vs;
-      vs = t;
-      es += e[u];
-      const uint64_t k = err_key(e[u]);
-      kmax = k > kmax ? k : kmax;
+  for (int e = 0; e < kMaxDim; ++e)
+    if (e < D && e == sd) hd = h[e] * 0.5;
+  const double vol = L.geo[kFieldVol * S + p];
+  double vq = 1;  // box_volume of the new half, the same products in order
+#pragma unroll
+  for (int e = 0; e < kMaxDim; ++e) {
+    if (e >= D) continue;
+    const double he = (e == sd) ? hd : h[e];
+    vq *= 2 * he;
+    L.geo[(kFieldC + e) * S + q] = (e == sd) ? c[e] + hd : c[e];
+    L.geo[(kFieldH + e) * S + q] = he;
+    if (e == sd) {
+      L.geo[(kFieldC + e) * S + p] = c[e] - hd;
+      L.geo[(kFieldH + e) * S + p] = hd;
     }
   }
-  s_red[tid] = vs;
-  s_red2[tid] = vc;
-  s_redk[tid] = kmax;
-  s_cnt[tid] = bad ? 1u : 0u;
-  __syncthreads();
-  for (int w = kSelThreads / 2; w > 0; w >>= 1) {
-    if (tid < w) {
-      double a = s_red[tid], b = s_red[tid + w];
-      double t = a + b;
-      double c = fabs(a) >= fabs(b) ? (a - t) + b : (b - t) + a;
-      s_red[tid] = t;
-      s_red2[tid] += s_red2[tid + w] + c;
-      s_redk[tid] = s_redk[tid] > s_redk[tid + w] ? s_redk[tid] : s_redk[tid + w];
-      s_cnt[tid] |= s_cnt[tid + w];
-    }
-    __syncthreads();
-  }
-  const double V = s_red[0] + s_red2[0];
-  const uint64_t maxkey = s_redk[0];
-  const bool nonfinite = s_cnt[0] != 0;
-  __syncthreads();
-  s_red[tid] = es;
-  __syncthreads();
-  for (int w = kSelThreads / 2; w > 0; w >>= 1) {
-    if (tid < w) s_red[tid] += s_red[tid + w];
-    __syncthreads();
-  }
-  const double E = s_red[0];
-  __syncthreads();
+  L.geo[kFieldVol * S + p] = vol * 0.5;
+  L.geo[kFieldVol * S + q] = vq;
+  list[a] = EvalItem{p, J};
+  list[K + a] = EvalItem{q, J};
+}
 
-  // 2. stop tests in the order of src/hcubature.cpp:938-939.
-  if (tid == 0) {
-    JobState st = s_st;
-    st.val = V;
-    st.err = E;
-    if (nonfinite) st.flags |= kJobNonfinite;
-    int flag = 0;
-    if (d.maxeval != 0 && st.neval >= d.maxeval) {
-      st.flags |= kJobDone | kJobCapped;
-      flag = 1;
-    } else if (!(E > 0 && E > fabs(V) * d.reltol)) {
-      st.flags |= kJobDone | kJobConverged;
-      flag = 1;
-    }
-    s_st = st;
-    s_flag = flag;
+// The job's state after a batch of K regions.  One thread calls it.
+__device__ __forceinline__ void select_commit(const SelectLaunch &L, const JobDesc &d, uint32_t J,
+                                              uint32_t K, JobState st) {
+  if (L.trace && st.rounds < L.trace_cap) L.trace[(size_t)J * L.trace_cap + st.rounds] = 2u * K;
+  st.n += K;
+  st.neval += 2ull * (uint64_t)d.pts * K;
+  st.rounds += 1;
+  L.state[J] = st;
+}
+
+// n <= 64 R regions by one wave.
+template <int R>
+__device__ __forceinline__ void select_wave(const SelectLaunch &L, uint32_t J, const JobDesc &d,
+                                            JobState st, SearchLds &W, uint32_t *list_p) {
+  const int lane = threadIdx.x & 63;
+  const uint32_t n = st.n;
+  const uint64_t S = L.stride;
+  const double *val = L.geo + kFieldVal * S + d.base, *err = L.geo + kFieldErr * S + d.base;
+  uint64_t k[R];
+  double v[R], e[R], c[R], check = 0;
+  uint64_t maxkey = 0;
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const uint32_t i = 64 * r + lane;
+    v[r] = i < n ? val[i] : 0.0;
+    e[r] = i < n ? err[i] : 0.0;
+    c[r] = 0;
   }
-  __syncthreads();
-  if (s_flag) {
-    if (tid == 0) {
-      L.state[J] = s_st;
-      if (L.done) L.done[atomicAdd(&L.counters[kNumKinds + 1], 1u)] = J;
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    check = fma(0.0, v[r], fma(0.0, e[r], check));
+    const uint64_t ke = err_key(e[r]);
+    k[r] = 64u * r + lane < n ? ke : ~0ull;
+    maxkey = ke > maxkey ? ke : maxkey;
+  }
+#pragma unroll
+  for (int w = R / 2; w > 0; w >>= 1) {
+#pragma unroll
+    for (int q = 0; q < w; ++q) {
+      const double t = v[q] + v[q + w];
+      c[q] += c[q + w] + sum_error(v[q], v[q + w], t);
+      v[q] = t;
+      e[q] += e[q + w];
     }
+  }
+  const double V = comp_total(v[0], c[0]);
+  double E = e[0];
+  tree([&](auto w) { E += from_above<decltype(w)::value>(E); });
+  E = readlane64(E, 0);
+  if (select_stops(d, V, E, __ballot(check != check) != 0, st)) {
+    if (lane == 0) select_finish(L, J, st);
     return;
   }
+  // every key is among these, so the boundary is
+  Boundary B{};
+  (void)find_boundary<R>(k, n, wave_max(maxkey), Goal{fabs(V) * d.reltol, select_kcap(d, st), 0, 0.0},
+                         W, B);
+  const uint32_t K = B.gt + B.take;
+  uint32_t listbase = 0, ok = 0;
+  if (lane == 0) ok = select_room(L, d, K, st, listbase) ? 1u : 0u;
+  listbase = __builtin_amdgcn_readfirstlane(listbase);
+  if (!__builtin_amdgcn_readfirstlane(ok)) {
+    if (lane == 0) select_finish(L, J, st);
+    return;
+  }
+  uint32_t at = 0, ties = 0;
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const bool in = k[r] != ~0ull, tie = in && k[r] == B.T;
+    const uint64_t tm = __ballot(tie);
+    const bool s = in && (k[r] > B.T || (tie && ties + lanes_below(tm) < B.take));
+    ties += (uint32_t)__popcll(tm);
+    const uint64_t sm = __ballot(s);
+    if (s) list_p[at + lanes_below(sm)] = 64 * r + lane;
+    at += (uint32_t)__popcll(sm);
+  }
+  wave_sync();
+  EvalItem *list = L.lists[d.kind] + listbase;
+  for (uint32_t a = lane; a < K; a += 64)
+    select_cut(L, list, J, d.dim, d.base + list_p[a], d.base + n + a, a, K);
+  if (lane == 0) select_commit(L, d, J, K, st);
+}
 
-  // 3. batch size: pops continue until the remaining error meets the
-  //    tolerance or the evaluation budget is spent (src/hcubature.cpp:971-985).
-  //    The pops take the regions in decreasing error; the batch is found by
-  //    a radix select over the 64-bit error keys, 8 bits per level from the
-  //    top, in fixed-point error units (sel_shift maps maxkey low enough that
-  //    a sum over all n keys stays below 2^63; integer sums are exact and
-  //    order-free).
-  const uint64_t twoP = 2ull * (uint64_t)d.pts;
-  uint64_t kcap = n;
-  if (d.maxeval != 0) {
-    uint64_t room = d.maxeval - s_st.neval;
-    uint64_t kc = (room + twoP - 1) / twoP;
-    kcap = kc < kcap ? kc : kcap;
+// Whether popping every key >= T of the integral is enough, over the whole
+// block (the bisection's test).
+template <int NT>
+__device__ bool block_enough(const double *err, uint32_t n, uint64_t T, const Goal &g,
+                             SelectLds<NT> &S, uint32_t &ge) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  double s = 0, c = 0;
+  uint32_t cnt = 0;
+  for (uint32_t i = tid; i < n; i += NT) {
+    const uint64_t k = err_key(err[i]);
+    comp_add(s, c, k < T ? __builtin_bit_cast(double, k) : 0.0);
+    cnt += k >= T;
   }
-  const int shift = sel_shift(maxkey, n);
-  const double thr = ldexp(fabs(V) * d.reltol, shift);
-  if (tid == 0) {
-    s_prefix = 0;
-    s_mask = 0;
-    s_cumsum = 0;
-    s_cumcnt = 0;
+  comp_tree(s, c);
+  tree([&](auto w) { cnt += from_above32<decltype(w)::value>(cnt); });
+  __syncthreads();
+  if (lane == 0) {
+    S.bs[wave] = s;
+    S.bc[wave] = c;
+    S.wcnt[wave] = cnt;
   }
-  for (int level = 0; level < 8; ++level) {
-    const int sh = 56 - 8 * level;
-    s_cnt[tid] = 0;
-    s_sum[tid] = 0;
-    __syncthreads();
-    const uint64_t prefix = s_prefix, mask = s_mask;
-    for (uint32_t i0 = tid; i0 < n; i0 += 4 * kSelThreads) {
-      uint64_t k[4];
+  __syncthreads();
+  double ts = 0, tc = 0;
+  ge = 0;
+  for (int w = 0; w < NT / 64; ++w) {
+    comp_add(ts, tc, S.bs[w]);
+    tc += S.bc[w];
+    ge += S.wcnt[w];
+  }
+  return ge >= g.kcap || meets(ts + tc, g.thr);
+}
+
+template <int NT>
+__device__ __forceinline__ void select_block(const SelectLaunch &L, uint32_t J, const JobDesc &d,
+                                             SelectLds<NT> &S) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const uint64_t St = L.stride;
+  const uint32_t n = S.st.n;
+  const double *val = L.geo + kFieldVal * St + d.base, *err = L.geo + kFieldErr * St + d.base;
+  constexpr int U = 8;   // loads in flight per thread
+
+  // 1. totals.  With 1024 threads the first four waves take the values and the
+  //    next four the errors.
+  const bool tv = tid < kPartial, te = NT == kPartial ? true : (tid >= kPartial && tid < 2 * kPartial);
+  double check = 0;
+  uint64_t kmax = 0;
+  if (tv) {
+    double s = 0, c = 0;
+    for (uint32_t i0 = tid; i0 < n; i0 += U * kPartial) {
+      double v[U];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const uint32_t i = i0 + u * kSelThreads;
-        k[u] = i < n ? err_key(err[i]) : ~0ull;  // ~0 matches no prefix
+      for (int u = 0; u < U; ++u) v[u] = i0 + u * kPartial < n ? val[i0 + u * kPartial] : 0.0;
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        check = fma(0.0, v[u], check);
+        comp_add(s, c, v[u]);
       }
+    }
+    S.vs[tid] = s;
+    S.vc[tid] = c;
+  }
+  if (te) {
+    const int t = tid & (kPartial - 1);
+    double s = 0;
+    for (uint32_t i0 = t; i0 < n; i0 += U * kPartial) {
+      double e[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) e[u] = i0 + u * kPartial < n ? err[i0 + u * kPartial] : 0.0;
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        check = fma(0.0, e[u], check);
+        s += e[u];
+        const uint64_t k = err_key(e[u]);
+        kmax = k > kmax ? k : kmax;
+      }
+    }
+    S.es[t] = s;
+    kmax = wave_max(kmax);
+    if (lane == 0) S.kmax[(tid & (kPartial - 1)) >> 6] = kmax;
+  }
+  if (__ballot(check != check) != 0 && lane == 0) atomicOr(&S.bad, 1u);
+  if (tid < 256) {
+    S.sum[tid] = 0;
+    S.cnt[tid] = 0;
+  }
+  __syncthreads();
+  if (wave == 0) {
+    double s[4], c[4], e[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      s[q] = S.vs[64 * q + lane];
+      c[q] = S.vc[64 * q + lane];
+      e[q] = S.es[64 * q + lane];
+    }
+#pragma unroll
+    for (int w = 2; w > 0; w >>= 1) {
+#pragma unroll
+      for (int q = 0; q < w; ++q) {
+        const double t = s[q] + s[q + w];
+        c[q] += c[q + w] + sum_error(s[q], s[q + w], t);
+        s[q] = t;
+        e[q] += e[q + w];
+      }
+    }
+    const double V = comp_total(s[0], c[0]);
+    double E = e[0];
+    tree([&](auto w) { E += from_above<decltype(w)::value>(E); });
+    E = readlane64(E, 0);
+    if (lane == 0) {
+      uint64_t k = S.kmax[0];
+      for (int w = 1; w < kPartial / 64; ++w) k = S.kmax[w] > k ? S.kmax[w] : k;
+      S.maxkey = k;
+      S.V = V;
+      S.E = E;
+      // 2. stop tests
+      JobState st = S.st;
+      S.stop = select_stops(d, V, E, S.bad != 0, st) ? 1 : 0;
+      S.st = st;
+      if (S.stop) select_finish(L, J, st);
+      S.lo = 0;
+      S.width = 1ull << 63;
+      S.above = 0;
+      S.rest = 0;
+      S.nkey = 0;
+      S.found = 0;
+    }
+  }
+  __syncthreads();
+  if (S.stop) return;
+
+  // 3. the batch's boundary.  A histogram pass names the bin that holds it
+  //    (narrowed while the bin has more keys than fit LDS), a second pass
+  //    collects that bin's keys and sums the smaller ones exactly, and the
+  //    first wave finds the boundary among them.
+  const uint64_t maxkey = S.maxkey;
+  const Goal goal{fabs(S.V) * d.reltol, select_kcap(d, S.st), 0, 0.0};
+  const int shift = sel_shift(maxkey, n);
+  const double thr_fx = ldexp(goal.thr, shift);
+  int s = 49;
+  for (;;) {
+    const uint64_t lo = S.lo, width = S.width;
+    for (uint32_t i0 = tid; i0 < n; i0 += 4 * NT) {
+      double e[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) e[u] = i0 + u * NT < n ? err[i0 + u * NT] : 0.0;
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
-        if ((k[u] & mask) == prefix && k[u] != ~0ull) {
-          const int dgt = (int)((k[u] >> sh) & 0xff);
-          atomicAdd(&s_cnt[dgt], 1u);
-          atomicAdd(&s_sum[dgt], fixed_err(k[u], shift));
+        const uint64_t k = err_key(e[u]), dd = maxkey - k - lo;
+        if (i0 + u * NT < n && k <= maxkey - lo && dd < width) {
+          const uint64_t q = dd >> s;
+          const int b = q < 255 ? (int)q : 255;
+          atomicAdd(&S.cnt[b], 1u);
+          atomicAdd(&S.sum[b], fixed_err(k, shift));
         }
       }
     }
     __syncthreads();
-    // bins in decreasing digit order, thread t <-> digit 255 - t: running
-    // sums from the top digit down
-    const int bin = kSelThreads - 1 - tid;
-    uint64_t cs = s_sum[bin], cc = s_cnt[bin], tot_s, tot_c;
-    block_scan2(cs, cc, s_wa, s_wb, tot_s, tot_c);
-    if (level == 0) {
-      // the level-0 histogram holds every key: its sum is the total error
-      if (tid == 0) s_need = batch_need(tot_s, thr);
-      __syncthreads();
-    }
-    const uint64_t need = s_need, cs0 = s_cumsum, cc0 = s_cumcnt;
-    // the pops end in the first non-empty bin (from the top) at which the
-    // error sum reaches need or the count reaches kcap; the running sums only
-    // grow in thread order, so the threads that pass the test are a suffix
-    // and the found bin is its first
-    const bool hit = cs0 + cs >= need || cc0 + cc >= kcap;
-    const uint64_t hb = __ballot(hit);
-    if ((tid & 63) == 0) s_wa[tid >> 6] = (uint64_t)__popcll(hb);
-    __syncthreads();
-    const int nhit = (int)(s_wa[0] + s_wa[1] + s_wa[2] + s_wa[3]);
-    // thread of the found bin: the first one that hits (bin 0 if none does,
-    // which the total meeting need rules out)
-    const int tf = nhit > 0 ? kSelThreads - nhit : kSelThreads - 1;
-    if (tid == tf) {
-      const int found = kSelThreads - 1 - tf;
-      s_prefix = prefix | ((uint64_t)found << sh);
-      s_mask = mask | (0xffull << sh);
-      s_cumsum = cs0 + cs - s_sum[found];
-      s_cumcnt = (uint32_t)(cc0 + cc - s_cnt[found]);
-      s_lastcnt = s_cnt[found];
-    }
-    __syncthreads();
-  }
-  // s_prefix is now the exact key of the last popped region; take r of the
-  // regions carrying that key, lowest slot first.
-  if (tid == 0) {
-    uint64_t T = s_prefix;
-    unsigned long long fxT = fixed_err(T, shift);
-    const uint64_t need = s_need;
-    uint64_t rest = need > s_cumsum ? need - s_cumsum : 0;
-    uint64_t r = fxT > 0 ? (rest + fxT - 1) / fxT : (uint64_t)s_lastcnt;
-    if (r < 1) r = 1;
-    if (r > s_lastcnt) r = s_lastcnt;
-    if ((uint64_t)s_cumcnt + r > kcap) r = kcap - s_cumcnt;
-    s_r = (uint32_t)r;
-  }
-  __syncthreads();
-
-  // 3b. The exact stopping point.  The reference pops in decreasing error,
-  //     subtracting each popped error from the running total in FP64, and
-  //     stops at the first count whose remaining error meets the tolerance
-  //     (src/hcubature.cpp:971-985, src/converged.h:10-14).  The fixed-point
-  //     keys above are truncated, by up to one unit (2^-46 of the largest
-  //     error) per region, so on integrals whose errors span many decades
-  //     their sum over thousands of small-error regions can misplace that
-  //     count by a region or two.  The remaining error is recomputed here in
-  //     FP64 (compensated) and the count stepped, one tie at a time and one
-  //     key at a time, until it is the reference's.
-  select_exact_count(err, n, kcap, fabs(V) * d.reltol, s_prefix, s_lastcnt, s_cumcnt, s_r,
-                     s_red, s_red2, s_redk, s_cnt);
-
-  if (tid == 0) {
-    const uint32_t K = s_cumcnt + s_r;
-    s_K = K;
-    JobState st = s_st;
-    if (st.n + K > d.cap) {
-      st.flags |= kJobDone | kJobPoolFull;
-      s_flag = 1;
-    } else {
-      s_listbase = atomicAdd(&L.counters[d.kind], 2u * K);
-      if (s_listbase + 2u * K > L.list_cap[d.kind]) {
-        st.flags |= kJobDone | kJobPoolFull;
-        s_flag = 1;
-      } else {
-        atomicAdd(&L.counters[kNumKinds], 1u);
+    if (wave == 0) {
+      // lane l takes bins 4 l .. 4 l + 3
+      unsigned long long bsum[4], own = 0;
+      uint32_t bcnt[4], cown = 0;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        bsum[q] = S.sum[4 * lane + q];
+        bcnt[q] = S.cnt[4 * lane + q];
+        own += bsum[q];
+        cown += bcnt[q];
+      }
+      unsigned long long suf = own;
+      uint32_t pre = cown;
+#pragma unroll
+      for (int w = 1; w < 64; w <<= 1) {
+        const uint32_t l2 = __shfl_down((uint32_t)suf, w), h2 = __shfl_down((uint32_t)(suf >> 32), w);
+        const uint32_t p2 = __shfl_up(pre, w);
+        if (lane + w < 64) suf += ((unsigned long long)h2 << 32) | l2;
+        if (lane >= w) pre += p2;
+      }
+      // the first non-empty bin after which enough is popped, else the last one
+      unsigned long long rest = suf + S.rest;     // remaining before this lane's bins
+      uint32_t cum = S.above + pre - cown;        // popped before them
+      int first = -1, last = -1;
+      uint32_t cfirst = 0, clast = 0;
+      unsigned long long rfirst = 0, rlast = 0;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        rest -= bsum[q];
+        if (bcnt[q]) {
+          if (first < 0 && ((double)rest <= thr_fx || (uint64_t)cum + bcnt[q] >= goal.kcap)) {
+            first = q;
+            cfirst = cum;
+            rfirst = rest;
+          }
+          last = q;
+          clast = cum;
+          rlast = rest;
+        }
+        cum += bcnt[q];
+      }
+      const uint64_t hit = __ballot(first >= 0), some = __ballot(last >= 0);
+      const int who = hit ? __ffsll((unsigned long long)hit) - 1 : 63 - __clzll((long long)some);
+      if (lane == who) {
+        const int q = hit ? first : last;
+        const int b = 4 * lane + q;
+        S.above = hit ? cfirst : clast;
+        S.rest = hit ? rfirst : rlast;
+        uint32_t mq = 0;
+#pragma unroll
+        for (int x = 0; x < 4; ++x) mq = x == q ? bcnt[x] : mq;
+        S.m = mq;
+        S.lo = lo + ((uint64_t)b << s);
+        S.width = b == 255 ? width - ((uint64_t)255 << s) : 1ull << s;
       }
     }
-    s_st = st;
+    __syncthreads();
+    if (S.m <= 1024 || S.width <= 1) break;
+    s = 56 - __clzll((long long)(S.width - 1));   // ceil(log2 width) - 8
+    s = s < 0 ? 0 : s;
+    if (tid < 256) {
+      S.sum[tid] = 0;
+      S.cnt[tid] = 0;
+    }
+    __syncthreads();
+  }
+  {
+    const uint64_t khi = maxkey - S.lo, w1 = S.width - 1, klo = khi >= w1 ? khi - w1 : 0;
+    const bool few = S.m <= 1024;
+    double bs = 0, bc = 0;
+    for (uint32_t i0 = tid; i0 < n; i0 += 4 * NT) {
+      double e[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) e[u] = i0 + u * NT < n ? err[i0 + u * NT] : 0.0;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const uint64_t k = err_key(e[u]);
+        comp_add(bs, bc, k < klo ? __builtin_bit_cast(double, k) : 0.0);
+        if (few && i0 + u * NT < n && k >= klo && k <= khi) S.key[atomicAdd(&S.nkey, 1u)] = k;
+      }
+    }
+    comp_tree(bs, bc);
+    if (lane == 0) {
+      S.bs[wave] = bs;
+      S.bc[wave] = bc;
+    }
+    __syncthreads();
+    if (wave == 0) {
+      double ts = 0, tc = 0;
+      for (int w = 0; w < NT / 64; ++w) {
+        comp_add(ts, tc, S.bs[w]);
+        tc += S.bc[w];
+      }
+      Goal g = goal;
+      g.above = S.above;
+      g.below = ts + tc;
+      const uint32_t m = S.m;
+      Boundary B{};
+      bool ok;
+      auto search = [&](auto tag) {
+        constexpr int R = decltype(tag)::value;
+        uint64_t k[R], km = 0;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          const uint32_t i = 64 * r + lane;
+          k[r] = i < m ? S.key[i] : ~0ull;
+          km = i < m && k[r] > km ? k[r] : km;
+        }
+        return find_boundary<R>(k, m, wave_max(km), g, S.search, B);
+      };
+      if (!few) {   // one key, many regions
+        const double all = g.below + (double)m * __builtin_bit_cast(double, khi);
+        ok = (meets(g.below, g.thr) || (uint64_t)g.above + m >= g.kcap) &&
+             (g.above == 0 || !(meets(all, g.thr) || g.above >= g.kcap));
+        B = Boundary{khi, m, fewest(g, khi, m, g.above, g.below), g.above};
+      } else if (m <= 64) {
+        ok = search(Int<1>{});
+      } else if (m <= 256) {
+        ok = search(Int<4>{});
+      } else {
+        ok = search(Int<16>{});
+      }
+      if (lane == 0) {
+        S.found = ok ? 1 : 0;
+        S.B = B;
+      }
+    }
+    __syncthreads();
+  }
+  if (!S.found) {
+    // the truncated sums named the wrong bin: bisection over the key's bits
+    uint64_t t = 0;
+    uint32_t ge = 0;
+    for (int bit = 62; bit >= 0; --bit) {
+      const uint64_t u = t | (1ull << bit);
+      if (u <= maxkey && block_enough<NT>(err, n, u, goal, S, ge)) t = u;
+    }
+    (void)block_enough<NT>(err, n, t, goal, S, ge);
+    uint32_t more = 0;
+    (void)block_enough<NT>(err, n, t + 1, goal, S, more);
+    // the sum below t once more, for the multiplicity's share
+    double ts = 0, tc = 0;
+    for (uint32_t i = tid; i < n; i += NT) {
+      const uint64_t k = err_key(err[i]);
+      comp_add(ts, tc, k < t ? __builtin_bit_cast(double, k) : 0.0);
+    }
+    comp_tree(ts, tc);
+    __syncthreads();
+    if (lane == 0) {
+      S.bs[wave] = ts;
+      S.bc[wave] = tc;
+    }
+    __syncthreads();
+    if (tid == 0) {
+      double a = 0, b = 0;
+      for (int w = 0; w < NT / 64; ++w) {
+        comp_add(a, b, S.bs[w]);
+        b += S.bc[w];
+      }
+      S.B = Boundary{t, ge - more, fewest(goal, t, ge - more, more, a + b), more};
+    }
+    __syncthreads();
+  }
+  const Boundary B = S.B;
+  const uint32_t K = B.gt + B.take;
+  if (tid == 0) {
+    JobState st = S.st;
+    S.stop = select_room(L, d, K, st, S.listbase) ? 0 : 1;
+    if (S.stop) select_finish(L, J, st);
   }
   __syncthreads();
-  if (s_flag) {
-    if (tid == 0) {
-      L.state[J] = s_st;
-      if (L.done) L.done[atomicAdd(&L.counters[kNumKinds + 1], 1u)] = J;
-    }
-    return;
-  }
+  if (S.stop) return;
 
-  // 4. mark and cut in slot order; children go to the kind's list.  Each
-  //    thread marks four consecutive slots per chunk of 1024; the ranks among
-  //    the tied keys and among the selected regions come from block scans of
-  //    the per-thread counts (carried across chunks in registers), and the
-  //    chunk's selected slots are listed in LDS in rank order, so that
-  //    consecutive lanes cut consecutive regions (contiguous child slots)
-  //    and each cut reads its region's geometry before writing any.  The
-  //    list holds the K halves that keep their parents' slots first and the
-  //    K new slots after them, both in slot order, so that the regions an
-  //    evaluation block stages sit in neighbouring slots of each field.
-  __shared__ uint32_t s_selp[4 * kSelThreads];
-  const uint64_t T = s_prefix;
-  const uint32_t r = s_r;
-  const uint32_t K = s_K;
-  const int D = d.dim;
-  EvalItem *list = L.lists[d.kind] + s_listbase;
-  uint64_t tie_carry = 0, sel_carry = 0;
-  for (uint32_t chunk = 0; chunk < n; chunk += 4 * kSelThreads) {
+  // 4. the cuts, in slot order: each thread looks at four consecutive slots of
+  //    a chunk; ranks among the batch (and, where only part of the regions at
+  //    T go, among those) come from wave scans and the waves' totals, and the
+  //    chunk's slots are listed in LDS in rank order, so that consecutive
+  //    lanes cut consecutive regions.
+  EvalItem *list = L.lists[d.kind] + S.listbase;
+  const bool some_ties = B.take != B.eq;
+  uint32_t done = 0, ties = 0;
+  for (uint32_t chunk = 0; chunk < n; chunk += 4 * NT) {
     const uint32_t i0 = chunk + 4 * tid;
     uint64_t k[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) k[u] = i0 + u < n ? err_key(err[i0 + u]) : 0;
-    uint64_t nt = 0;
-#pragma unroll
-    for (int u = 0; u < 4; ++u) nt += (i0 + u < n && k[u] == T) ? 1 : 0;
-    // ties before this thread's, then the selections it makes
-    uint64_t tie_incl = nt, dummy = 0, tot_t, tot_d;
-    block_scan2(tie_incl, dummy, s_wa, s_wb, tot_t, tot_d);
-    uint64_t trank = tie_carry + tie_incl - nt;
-    uint32_t selm = 0;
-    uint64_t ns = 0;
+    uint32_t selm = 0, tiem = 0;
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       const bool in = i0 + u < n;
-      const bool tie = in && k[u] == T;
-      const bool sel = in && (k[u] > T || (tie && trank < r));
-      if (tie) ++trank;
-      selm |= sel ? 1u << u : 0u;
-      ns += sel ? 1 : 0;
+      selm |= in && (some_ties ? k[u] > B.T : k[u] >= B.T) ? 1u << u : 0u;
+      tiem |= in && k[u] == B.T ? 1u << u : 0u;
     }
-    uint64_t sel_incl = ns, dummy2 = 0, tot_s2, tot_d2;
-    block_scan2(sel_incl, dummy2, s_wa, s_wb, tot_s2, tot_d2);
-    uint32_t at = (uint32_t)(sel_incl - ns);
+    auto scan = [&](uint32_t own, uint32_t *w_tot, uint32_t &total) {
+      uint32_t inc = own;
+#pragma unroll
+      for (int w = 1; w < 64; w <<= 1) {
+        const uint32_t x = __shfl_up(inc, w);
+        if (lane >= w) inc += x;
+      }
+      if (lane == 63) w_tot[wave] = inc;
+      __syncthreads();
+      uint32_t before = 0;
+      total = 0;
+#pragma unroll
+      for (int w = 0; w < NT / 64; ++w) {
+        const uint32_t x = w_tot[w];
+        before += w < wave ? x : 0u;
+        total += x;
+      }
+      return before + inc - own;
+    };
+    if (some_ties) {
+      uint32_t tot, rank = ties + scan((uint32_t)__popc(tiem), S.wtie, tot);
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (tiem >> u & 1u) {
+          selm |= rank < B.take ? 1u << u : 0u;
+          ++rank;
+        }
+      ties += tot;
+    }
+    uint32_t tot, at = scan((uint32_t)__popc(selm), S.wcnt, tot);
 #pragma unroll
     for (int u = 0; u < 4; ++u)
-      if (selm >> u & 1u) s_selp[at++] = i0 + u;
+      if (selm >> u & 1u) S.sel[at++] = i0 + u;
     __syncthreads();
-    for (uint32_t j = tid; j < (uint32_t)tot_s2; j += kSelThreads) {
-      const uint32_t p = d.base + s_selp[j];
-      const uint64_t a = sel_carry + j;
-      const uint32_t q = d.base + n + (uint32_t)a;
-      const int sd = L.split[p];
-      double c[kMaxDim], h[kMaxDim], hd = 0;
-#pragma unroll
-      for (int e = 0; e < kMaxDim; ++e) {
-        if (e < D) {
-          c[e] = L.geo[(kFieldC + e) * S + p];
-          h[e] = L.geo[(kFieldH + e) * S + p];
-        }
-      }
-#pragma unroll
-      for (int e = 0; e < kMaxDim; ++e)
-        if (e < D && e == sd) hd = h[e] * 0.5;
-      const double vol = L.geo[kFieldVol * S + p];
-      double vq = 1;  // box_volume of the child, the same products in order
-#pragma unroll
-      for (int e = 0; e < kMaxDim; ++e) {
-        if (e >= D) continue;
-        const double he = (e == sd) ? hd : h[e];
-        vq *= 2 * he;
-        L.geo[(kFieldC + e) * S + q] = (e == sd) ? c[e] + hd : c[e];
-        L.geo[(kFieldH + e) * S + q] = he;
-        if (e == sd) {
-          L.geo[(kFieldC + e) * S + p] = c[e] - hd;
-          L.geo[(kFieldH + e) * S + p] = hd;
-        }
-      }
-      L.geo[kFieldVol * S + p] = vol * 0.5;
-      L.geo[kFieldVol * S + q] = vq;
-      list[a] = EvalItem{p, (uint32_t)J};
-      list[K + a] = EvalItem{q, (uint32_t)J};
-    }
-    tie_carry += tot_t;
-    sel_carry += tot_s2;
+    for (uint32_t j = tid; j < tot; j += NT)
+      select_cut(L, list, J, d.dim, d.base + S.sel[j], d.base + n + done + j, done + j, K);
+    done += tot;
     __syncthreads();
   }
-  if (tid == 0) {
-    JobState st = s_st;
-    if (L.trace && st.rounds < L.trace_cap) L.trace[(size_t)J * L.trace_cap + st.rounds] = 2u * s_K;
-    st.n = n + s_K;
-    st.neval += twoP * s_K;
-    st.rounds += 1;
-    L.state[J] = st;
+  if (tid == 0) select_commit(L, d, J, K, S.st);
+}
+
+template <int NT>
+__global__ __launch_bounds__(NT) void k_select(SelectLaunch L) {
+  __shared__ SelectLds<NT> S;
+  const uint32_t J = L.active ? L.active[blockIdx.x] : blockIdx.x;
+  // through LDS: the last act of the block's first thread is a new state
+  if (threadIdx.x == 0) {
+    S.st = L.state[J];
+    S.bad = 0;
   }
+  __syncthreads();
+  if (S.st.flags & kJobDone) return;
+  const JobDesc d = L.jobs[J];
+  if (S.st.n <= 256) {
+    if (threadIdx.x >= 64) return;
+    if (S.st.n <= 64) select_wave<1>(L, J, d, S.st, S.search, S.sel);
+    else select_wave<4>(L, J, d, S.st, S.search, S.sel);
+    return;
+  }
+  select_block<NT>(L, J, d, S);
 }
 
 
@@ -1631,8 +1741,10 @@ int eval_kernel_ref(int kind, int prec, int variant, KernelRef *out) {
   return variant ? eval_ref_variant<1, PMix>(kind, out) : eval_ref_variant<0, PMix>(kind, out);
 }
 
-KernelRef select_kernel_ref() {
-  return KernelRef{reinterpret_cast<const void *>(&k_select), (unsigned)kSelThreads, 1u};
+static bool select_wide(uint32_t njobs) { return njobs <= kSelectWideJobs; }
+KernelRef select_kernel_ref(uint32_t njobs) {
+  if (select_wide(njobs)) return KernelRef{reinterpret_cast<const void *>(&k_select<1024>), 1024u, 1u};
+  return KernelRef{reinterpret_cast<const void *>(&k_select<256>), 256u, 1u};
 }
 KernelRef zero_kernel_ref() { return KernelRef{reinterpret_cast<const void *>(&k_zero), 256u, 1u}; }
 
@@ -1663,7 +1775,8 @@ hipError_t launch_roots(const RootsLaunch &L, hipStream_t s) {
 
 hipError_t launch_select(const SelectLaunch &L, uint32_t njobs, hipStream_t s) {
   if (njobs == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_select, dim3(njobs), dim3(kSelThreads), 0, s, L);
+  if (select_wide(njobs)) hipLaunchKernelGGL((k_select<1024>), dim3(njobs), dim3(1024), 0, s, L);
+  else hipLaunchKernelGGL((k_select<256>), dim3(njobs), dim3(256), 0, s, L);
   return hipGetLastError();
 }
 

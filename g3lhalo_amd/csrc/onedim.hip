@@ -31,6 +31,7 @@
 #include "onedim.h"
 #include "rules.h"
 #include "select_math.h"
+#include "select_wave.h"
 
 #pragma clang fp contract(off)
 
@@ -57,11 +58,8 @@ struct Store {
 };
 
 struct WaveLds {
-  // selection: 64 bins of fixed-point error sums and counts
-  unsigned long long sum[64];
-  uint32_t cnt[64];
-  uint64_t key[64];        // keys of the boundary bin
-  uint16_t split[kMaxSplit];
+  SearchLds search;
+  uint16_t split[kMaxSplit];   // slots of the batch, ascending
 };
 
 struct Lds {
@@ -116,236 +114,6 @@ __device__ __forceinline__ double precomp_point(int mode, const OneDimJob &j, do
   return x * x * W * d_tophat(x, j.t1) * j.t3 * spectrum;
 }
 
-__device__ __forceinline__ double lane0(double v) {
-  const uint64_t b = __builtin_bit_cast(uint64_t, v);
-  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)b);
-  const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(b >> 32));
-  return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
-}
-// The value of lane l + w, for lanes l < w of a wave (the others get whatever
-// the permute leaves): register permutes, which take a tenth of the latency of
-// a shuffle through LDS.
-template <int w>
-__device__ __forceinline__ uint32_t from_above32(uint32_t v) {
-  if constexpr (w == 32) return __builtin_amdgcn_permlane32_swap(v, v, false, false)[1];
-  else if constexpr (w == 16) return __builtin_amdgcn_permlane16_swap(v, v, false, false)[1];
-  else return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x100 + w, 0xf, 0xf, true);   // row_shl
-}
-template <int w>
-__device__ __forceinline__ uint64_t from_above(uint64_t v) {
-  return ((uint64_t)from_above32<w>((uint32_t)(v >> 32)) << 32) | from_above32<w>((uint32_t)v);
-}
-template <int w>
-__device__ __forceinline__ double from_above(double v) {
-  return __builtin_bit_cast(double, from_above<w>(__builtin_bit_cast(uint64_t, v)));
-}
-template <int N>
-struct Int {
-  static constexpr int value = N;
-};
-// f(Int<w>) for w = 32, 16, 8, 4, 2, 1.
-template <class F>
-__device__ __forceinline__ void tree(F f) {
-  f(Int<32>{}), f(Int<16>{}), f(Int<8>{}), f(Int<4>{}), f(Int<2>{}), f(Int<1>{});
-}
-__device__ __forceinline__ uint64_t wave_max(uint64_t k) {
-  tree([&](auto w) {
-    const uint64_t o = from_above<decltype(w)::value>(k);
-    k = o > k ? o : k;
-  });
-  return __builtin_bit_cast(uint64_t, lane0(__builtin_bit_cast(double, k)));
-}
-// The LDS of a wave is its own: a compiler barrier orders its accesses.
-__device__ __forceinline__ void wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-}
-__device__ __forceinline__ uint32_t lanes_below(uint64_t m) {
-  return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
-}
-
-// One Neumaier step (s, c) += e.
-__device__ __forceinline__ void comp_add(double &s, double &c, double e) {
-  const double t = s + e;
-  c += fabs(s) >= fabs(e) ? (s - t) + e : (e - t) + s;
-  s = t;
-}
-// Lane 0's tree sum of the lanes' (s, c), in every lane.
-__device__ __forceinline__ double comp_total(double s, double c) {
-  tree([&](auto w) {
-    constexpr int W = decltype(w)::value;
-    const double b = from_above<W>(s), cb = from_above<W>(c);
-    const double t = s + b;
-    c += cb + (fabs(s) >= fabs(b) ? (s - t) + b : (b - t) + s);
-    s = t;
-  });
-  return lane0(s + c);
-}
-
-// The converged() test of the reference on a remaining error.
-__device__ __forceinline__ bool meets(double rest, double thr) { return !(rest > 0 && rest > thr); }
-
-// Sum of the keys below T, compensated, over a wave's R x 64 keys (~0: none).
-template <int R>
-__device__ __forceinline__ double sum_below(const uint64_t (&k)[R], uint32_t n, uint64_t T) {
-  double s = 0, c = 0;
-#pragma unroll
-  for (int r = 0; r < R; ++r)
-    if (64u * r < n) comp_add(s, c, k[r] < T ? __builtin_bit_cast(double, k[r]) : 0.0);
-  return comp_total(s, c);
-}
-
-// Boundary of the Gladwell batch over n keys (k[r] of lane l is slot 64 r + l,
-// ~0 where there is none): the key T of the last region popped and how many
-// regions with that key are popped, such that the count is the first at which
-// the remaining error meets thr.  The remaining error after popping every key
-// >= T falls with T, so T is the largest key at which it meets thr.
-//
-// At most 64 regions: every lane sums the keys below its own.  More: a
-// histogram of the keys' distance below the largest (two bins per octave,
-// exact fixed-point sums) names the bin that holds the boundary, narrowed
-// until at most 64 keys are left, whose lanes do the same; a boundary that the
-// truncated sums put into the wrong bin shows in the exact sums and is then
-// found by bisection over the key's bits.
-template <int R>
-__device__ __forceinline__ void find_boundary(const uint64_t (&k)[R], uint32_t n, uint64_t maxkey,
-                                              double thr, WaveLds &W, uint64_t &T, uint32_t &take) {
-  const int lane = threadIdx.x & 63;
-  uint64_t ck = ~0ull;      // this lane's candidate
-  uint32_t m = 0;           // candidates
-  double below = 0;         // sum of the keys below every candidate
-  bool found = false, top = true;
-  if constexpr (R == 1) {
-    // most often only the largest goes (the bisection towards a peak)
-    const uint64_t largest = __ballot(lane < (int)n && k[0] == maxkey);
-    if (__popcll(largest) == 1 && meets(sum_below(k, n, maxkey), thr)) {
-      T = maxkey;
-      take = 1;
-      return;
-    }
-    ck = k[0];
-    m = n;
-  } else {
-    const int shift = sel_shift(maxkey, n);
-    const double thr_fx = ldexp(thr, shift);
-    // candidates: distance d = maxkey - key in [lo, lo + width)
-    uint64_t lo = 0, width = 1ull << 63;
-    int s = 51;
-    unsigned long long rest_after = 0;  // fixed-point sum of the keys beyond the range
-    for (;;) {
-      W.sum[lane] = 0;
-      W.cnt[lane] = 0;
-      wave_sync();
-#pragma unroll
-      for (int r = 0; r < R; ++r) {
-        if (64u * r >= n) break;
-        const uint64_t d = maxkey - k[r] - lo;   // absent keys wrap to >= 2^63
-        if (k[r] <= maxkey && k[r] <= maxkey - lo && d < width) {
-          const uint64_t q = d >> s;
-          const int b = q < 63 ? (int)q : 63;
-          atomicAdd(&W.cnt[b], 1u);
-          atomicAdd(&W.sum[b], fixed_err(k[r], shift));
-        }
-      }
-      wave_sync();
-      // suffix sums: what remains in the range beyond bin `lane`
-      const unsigned long long own = W.sum[lane];
-      unsigned long long suf = own;
-#pragma unroll
-      for (int w = 1; w < 64; w <<= 1) {
-        const uint32_t l2 = __shfl_down((uint32_t)suf, w), h2 = __shfl_down((uint32_t)(suf >> 32), w);
-        if (lane + w < 64) suf += ((unsigned long long)h2 << 32) | l2;
-      }
-      const unsigned long long rest = suf - own + rest_after;
-      const uint64_t hit = __ballot((double)rest <= thr_fx && W.cnt[lane] != 0);
-      int b = hit ? __ffsll((unsigned long long)hit) - 1
-                  : 63 - __clzll((long long)__ballot(W.cnt[lane] != 0));
-      b = __builtin_amdgcn_readfirstlane(b);
-      m = (uint32_t)__builtin_amdgcn_readlane((int)W.cnt[lane], b);
-      {
-        const uint32_t rl = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)rest, b);
-        const uint32_t rh = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(rest >> 32), b);
-        rest_after = ((unsigned long long)rh << 32) | rl;
-      }
-      lo += (uint64_t)b << s;
-      width = b == 63 ? width - ((uint64_t)63 << s) : 1ull << s;
-      if (m <= 64 || width <= 1) break;
-      s = 58 - __clzll((long long)(width - 1));   // ceil(log2 width) - 6
-      s = s < 0 ? 0 : s;
-    }
-    top = lo == 0;
-    const uint64_t kmin = maxkey - lo >= width - 1 ? maxkey - lo - (width - 1) : 0;
-    below = sum_below(k, n, kmin);
-    if (m > 64) {   // one key, many regions
-      T = maxkey - lo;
-      uint32_t eq = m;
-      const double kt = __builtin_bit_cast(double, T);
-      found = meets(below, thr) && (top || !meets(below + (double)eq * kt, thr));
-      if (found) {
-        while (eq > 1 && meets(below + (double)(m - eq + 1) * kt, thr)) --eq;
-        take = eq;
-        return;
-      }
-    } else {
-      uint32_t at = 0;
-#pragma unroll
-      for (int r = 0; r < R; ++r) {
-        if (64u * r >= n) break;
-        const bool in = k[r] <= maxkey - lo && k[r] >= kmin;
-        const uint64_t bm = __ballot(in);
-        if (in) W.key[at + lanes_below(bm)] = k[r];
-        at += (uint32_t)__popcll(bm);
-      }
-      wave_sync();
-      ck = lane < (int)m ? W.key[lane] : ~0ull;
-    }
-  }
-  if (m <= 64) {
-    double s = 0, c = 0, all = 0, allc = 0;
-    uint32_t eq = 0;
-    for (uint32_t j = 0; j < m; ++j) {
-      const uint32_t jl = __builtin_amdgcn_readlane((int)(uint32_t)ck, j);
-      const uint32_t jh = __builtin_amdgcn_readlane((int)(uint32_t)(ck >> 32), j);
-      const uint64_t kj = ((uint64_t)jh << 32) | jl;
-      const double e = __builtin_bit_cast(double, kj);
-      comp_add(s, c, kj < ck ? e : 0.0);
-      eq += kj == ck;
-      if constexpr (R > 1) comp_add(all, allc, e);
-    }
-    const double after = below + (s + c);
-    const bool mine = lane < (int)m && meets(after, thr);
-    const bool early = !top && meets(below + (all + allc), thr);   // met before this bin
-    if (__ballot(mine) != 0 && !early) {
-      T = wave_max(mine ? ck : 0);
-      const int who = __ffsll((unsigned long long)__ballot(mine && ck == T)) - 1;
-      const uint32_t cntT = (uint32_t)__builtin_amdgcn_readlane((int)eq, who);
-      const uint64_t ab = __builtin_bit_cast(uint64_t, after);
-      const uint32_t al = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)ab, who);
-      const uint32_t ah = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(ab >> 32), who);
-      const double rest = __builtin_bit_cast(double, ((uint64_t)ah << 32) | al);
-      uint32_t r = cntT;
-      while (r > 1 && meets(rest + (double)(cntT - r + 1) * __builtin_bit_cast(double, T), thr)) --r;
-      take = r;
-      return;
-    }
-  }
-  // the largest T <= maxkey at which the keys below T meet thr (it is a key:
-  // the sum only changes just above one)
-  uint64_t t = 0;
-  for (int bit = 62; bit >= 0; --bit) {
-    const uint64_t u = t | (1ull << bit);
-    if (u <= maxkey && meets(sum_below(k, n, u), thr)) t = u;
-  }
-  uint32_t eq = 0;
-#pragma unroll
-  for (int r = 0; r < R; ++r) eq += (uint32_t)__popcll(__ballot(k[r] == t));
-  const double rest = sum_below(k, n, t);
-  uint32_t r = eq;
-  while (r > 1 && meets(rest + (double)(eq - r + 1) * __builtin_bit_cast(double, t), thr)) --r;
-  T = t;
-  take = r;
-}
-
 // One integral's state; every field is the same in all lanes of its wave.
 struct WaveState {
   uint32_t n, flags, K;
@@ -368,10 +136,15 @@ __device__ __noinline__ void wave_round(const double *val, const double *err, do
   constexpr int B = R < 8 ? R : 8;   // loads in flight per array
   uint64_t k[R];
   double vs[V4] = {}, vc[V4] = {}, es[V4] = {};
-  bool bad = false;
+  double check = 0;   // NaN once a value or error is not finite
   uint64_t maxkey = 0;
 #pragma unroll
   for (int r0 = 0; r0 < R; r0 += B) {
+    if (64u * r0 >= n) {
+#pragma unroll
+      for (int r = 0; r < B; ++r) k[r0 + r] = ~0ull;
+      continue;
+    }
     double v[B], e[B];
 #pragma unroll
     for (int r = 0; r < B; ++r) {
@@ -381,7 +154,7 @@ __device__ __noinline__ void wave_round(const double *val, const double *err, do
     }
 #pragma unroll
     for (int r = 0; r < B; ++r) {
-      bad |= !isfinite(v[r]) || !isfinite(e[r]);
+      check = fma(0.0, v[r], fma(0.0, e[r], check));
       comp_add(vs[r & (V4 - 1)], vc[r & (V4 - 1)], v[r]);
       es[r & (V4 - 1)] += e[r];
       const uint64_t ke = err_key(e[r]);   // 0 where there is no region
@@ -394,7 +167,7 @@ __device__ __noinline__ void wave_round(const double *val, const double *err, do
 #pragma unroll
     for (int q = 0; q < w; ++q) {
       const double a = vs[q], b = vs[q + w], t = a + b;
-      vc[q] += vc[q + w] + (fabs(a) >= fabs(b) ? (a - t) + b : (b - t) + a);
+      vc[q] += vc[q + w] + sum_error(a, b, t);
       vs[q] = t;
       es[q] += es[q + w];
     }
@@ -402,42 +175,37 @@ __device__ __noinline__ void wave_round(const double *val, const double *err, do
   const double V = comp_total(vs[0], vc[0]);
   double E = es[0];
   tree([&](auto w) { E += from_above<decltype(w)::value>(E); });
-  E = lane0(E);
+  E = readlane64(E, 0);
   st.V = V;
   st.K = 0;
-  if (__ballot(bad) != 0) st.flags |= kJobNonfinite;
+  if (__ballot(check != check) != 0) st.flags |= kJobNonfinite;
   const double thr = fabs(V) * reltol;
   if (!(E > 0 && E > thr)) {
     st.flags |= kJobDone | kJobConverged;
     return;
   }
-  maxkey = wave_max(maxkey);
-  uint64_t T = 0;
-  uint32_t take = 0;
-  find_boundary<R>(k, n, maxkey, thr, W, T, take);
-  // regions above T and the first `take` of those at T, in slot order
-  uint32_t ties = 0, K = 0;
-  uint32_t sel = 0;
-#pragma unroll
-  for (int r = 0; r < R; ++r) {
-    if (64u * r >= n) break;
-    const bool in = k[r] != ~0ull, tie = in && k[r] == T;
-    const uint64_t tm = __ballot(tie);
-    const bool s = in && (k[r] > T || (tie && ties + lanes_below(tm) < take));
-    ties += (uint32_t)__popcll(tm);
-    sel |= s ? 1u << r : 0u;
-    K += (uint32_t)__popcll(__ballot(s));
-  }
+  // every key is among these, so the boundary is
+  Boundary Bd{};
+  (void)find_boundary<R>(k, n, wave_max(maxkey), Goal{thr, ~0ull, 0, 0.0}, W.search, Bd);
+  const uint32_t K = Bd.gt + Bd.take;
   if (n + K > kOneDimCap) {
     st.flags |= kJobDone | kJobPoolFull;
     return;
   }
   st.K = K;
-  uint32_t at = 0;
+  // regions above T and the first `take` of those at T, in slot order
+  uint32_t at = 0, ties = 0;
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     if (64u * r >= n) break;
-    const bool s = sel >> r & 1u;
+    const bool in = k[r] != ~0ull;
+    bool s = in && k[r] >= Bd.T;
+    if (Bd.take != Bd.eq) {
+      const bool tie = in && k[r] == Bd.T;
+      const uint64_t tm = __ballot(tie);
+      s = s && (!tie || ties + lanes_below(tm) < Bd.take);
+      ties += (uint32_t)__popcll(tm);
+    }
     const uint64_t sm = __ballot(s);
     if (s) W.split[at + lanes_below(sm)] = (uint16_t)(64 * r + lane);
     at += (uint32_t)__popcll(sm);

@@ -48,7 +48,7 @@ int RoundGraph::build(const bool used[kNumKinds], const int prec[kNumKinds],
                       const int variant[kNumKinds],
                       const EvalLaunch &eval_base, const SelectLaunch &sel_base, uint32_t *dcounters,
                       int ncounters, uint32_t *hcounters, const hipEvent_t *ev,
-                      const hipEvent_t *kev) {
+                      const hipEvent_t *kev, uint32_t nselect) {
   destroy();
   G3L_GR(hipGraphCreate(&graph, 0));
   hipGraphNode_t last = nullptr;
@@ -88,7 +88,8 @@ int RoundGraph::build(const bool used[kNumKinds], const int prec[kNumKinds],
   sel_args = sel_base;
   sel_params[0] = &sel_args;
   {
-    hipKernelNodeParams p = kparams(select_kernel_ref(), 1, sel_params);
+    select_ref = select_kernel_ref(nselect);
+    hipKernelNodeParams p = kparams(select_ref, 1, sel_params);
     G3L_GR(hipGraphAddKernelNode(&select_node, graph, &last, dep(), &p));
     last = select_node;
   }
@@ -118,8 +119,8 @@ int RoundGraph::launch(const uint32_t count[kNumKinds], EvalItem *const lists[kN
     hipKernelNodeParams p = kparams(eval_ref[k], (unsigned)blocks, eval_params[k]);
     G3L_GR(hipGraphExecKernelNodeSetParams(exec, eval_node[k], &p));
   }
-  if (nselect == 0 || nselect > 0x7fffffffu) return G3L_EINVAL;
-  hipKernelNodeParams p = kparams(select_kernel_ref(), nselect, sel_params);
+  if (nselect == 0 || nselect > 0x7fffffffu || !selects(nselect)) return G3L_EINVAL;
+  hipKernelNodeParams p = kparams(select_ref, nselect, sel_params);
   G3L_GR(hipGraphExecKernelNodeSetParams(exec, select_node, &p));
   G3L_GR(hipGraphLaunch(exec, s));
   return G3L_OK;

@@ -57,7 +57,8 @@ struct g3l_server {
   uint32_t fill[kNumKinds] = {};  // evaluation-list entries for the next round
   uint64_t rounds = 0;
   // the round as a graph (launch mode G3L_LAUNCH_GRAPH), built at the first
-  // step and again whenever the context's launch variants change
+  // step and again whenever the context's launch variants or the selection
+  // kernel for the integrals in flight change
   RoundGraph graph;
   int graph_variant[kNumKinds] = {};
   int graph_prec[kNumKinds] = {};
@@ -320,12 +321,12 @@ int g3l_server_step(g3l_server *s, g3l_server_status *status) {
   const KindLaunch KL = kind_launch(c, s->precision);
   const int *var = KL.variant;
   if (c->launch_mode == G3L_LAUNCH_GRAPH) {
-    if (!s->graph.exec || !std::equal(var, var + kNumKinds, s->graph_variant) ||
+    if (!s->graph.exec || !s->graph.selects(na) || !std::equal(var, var + kNumKinds, s->graph_variant) ||
         !std::equal(KL.prec, KL.prec + kNumKinds, s->graph_prec)) {
       bool in_use[kNumKinds];
       for (int k = 0; k < kNumKinds; ++k) in_use[k] = k != kNbar;  // the six terms
       if ((rc = s->graph.build(in_use, KL.prec, var, EL, SL, dcnt, kNumKinds + 2, hc, c->ev,
-                               c->kev)))
+                               c->kev, na)))
         return rc;
       std::copy(var, var + kNumKinds, s->graph_variant);
       std::copy(KL.prec, KL.prec + kNumKinds, s->graph_prec);
