@@ -45,7 +45,7 @@ KindLaunch kind_launch(const g3l_ctx *c, int prec) {
 }
 
 const double *nbar_ptr(const g3l_ctx *c, int set, int which) {
-  return c->nbar_chunks[set / kSetsPerChunk].as<double>() +
+  return c->nbar_chunks[set / kSetsPerChunk].dev.as<double>() +
          ((size_t)(set % kSetsPerChunk) * 2 + which) * c->nb;
 }
 
@@ -424,7 +424,17 @@ int run_one_dim(g3l_ctx *c, const std::vector<OneDimGroup> &groups,
   const uint32_t blocks = (uint32_t)std::min(units.size(), resident);
   int rc;
   if ((rc = c->od_in.ensure(o_retry + total * sizeof(OneDimUnit)))) return rc;
-  if ((rc = c->od_store.ensure(blocks * one_dim_store_bytes()))) return rc;
+  // the top of the groups' trees as tables, where several blocks would work
+  // them out for themselves
+  const bool top = !precomp && 2 * groups.size() <= blocks;
+  // nodes per block: an integral alone in a block mostly needs fewer than 2048,
+  // all of a precomputation's about 300 (those that need more are refined again
+  // below); a small store keeps a context's first run cheap to allocate
+  const uint32_t nodes = precomp ? 1024 : per == 1 ? 2048 : kOneDimNodes;
+  const size_t solo = one_dim_store_bytes(kOneDimNodes, 1);   // of a block of the second launch
+  const size_t store_bytes = std::max(blocks * one_dim_store_bytes(nodes, per), solo);
+  if ((rc = c->od_store.ensure(store_bytes + (top ? groups.size() * one_dim_top_bytes() : 0))))
+    return rc;
   std::vector<unsigned char> host(o_retry, 0);
   Outcome oc{~0ull, 0, 0};
   std::memcpy(host.data(), &oc, sizeof(oc));
@@ -443,18 +453,28 @@ int run_one_dim(g3l_ctx *c, const std::vector<OneDimGroup> &groups,
   L.reltol = reltol;
   L.scale = scale;
   L.store = c->od_store.as<unsigned char>();
+  L.store_bytes = one_dim_store_bytes(nodes, per);
+  L.nodes = nodes;
+  L.waves = per;
+  L.top = top ? L.store + store_bytes : nullptr;
   L.retry = reinterpret_cast<OneDimUnit *>(base + o_retry);
   L.failed = reinterpret_cast<unsigned long long *>(base);
   L.nretry = reinterpret_cast<uint32_t *>(base + offsetof(Outcome, nretry));
+  if (top) G3L_HIP(launch_one_dim_top(L, (uint32_t)groups.size(), s));
   G3L_HIP(launch_one_dim(precomp, L, blocks, s));
   G3L_HIP(hipMemcpyAsync(&oc, base, sizeof(oc), hipMemcpyDeviceToHost, s));
   G3L_HIP(hipStreamSynchronize(s));
   if (oc.nretry) {
-    // integrals whose block ran out of nodes, each alone in a block: no more
-    // retries (an integral's own nodes always fit)
+    // integrals whose block ran out of nodes, each alone in a block with room
+    // for all it can need: no more retries
+    const uint32_t sb = (uint32_t)std::min<size_t>(
+        {(size_t)oc.nretry, resident, store_bytes / solo});
     L.units = L.retry;
     L.nunits = oc.nretry;
-    G3L_HIP(launch_one_dim(precomp, L, std::min(blocks, oc.nretry), s));
+    L.store_bytes = solo;
+    L.nodes = kOneDimNodes;
+    L.waves = 1;
+    G3L_HIP(launch_one_dim(precomp, L, sb, s));
     G3L_HIP(hipMemcpyAsync(&oc, base, sizeof(oc), hipMemcpyDeviceToHost, s));
     G3L_HIP(hipStreamSynchronize(s));
   }
@@ -653,10 +673,11 @@ int compute_nbar(g3l_ctx *c, int first, int count) {
   const int nb = c->nb;
   const size_t need_chunks = ((size_t)first + count + kSetsPerChunk - 1) / kSetsPerChunk;
   while (c->nbar_chunks.size() < need_chunks) {
-    DevBuf b;
-    int rc = b.ensure((size_t)kSetsPerChunk * 2 * nb * sizeof(double));
+    NbarChunk b;
+    b.host.resize((size_t)kSetsPerChunk * 2 * nb);
+    int rc = b.dev.ensure(b.host.size() * sizeof(double));
     if (rc) return rc;
-    c->nbar_chunks.push_back(b);
+    c->nbar_chunks.push_back(std::move(b));
   }
   std::vector<OneDimJob> zs(nb);
   for (int i = 0; i < nb; ++i) zs[i] = OneDimJob{c->zmin + i * (c->zmax - c->zmin) / nb, 0, 0};
@@ -673,7 +694,18 @@ int compute_nbar(g3l_ctx *c, int first, int count) {
       g.mode = kOneDNbar;
       groups.push_back(g);
     }
-  return run_one_dim(c, groups, zs, false, 1e-4, kLn10);
+  if (int rc = run_one_dim(c, groups, zs, false, 1e-4, kLn10)) return rc;
+  // one copy per storage chunk that the sets touch
+  for (int s = first; s < first + count;) {
+    const int e = std::min(first + count, (s / kSetsPerChunk + 1) * kSetsPerChunk);
+    const size_t at = (size_t)(s % kSetsPerChunk) * 2 * nb;
+    G3L_HIP(hipMemcpyAsync(c->nbar_chunks[s / kSetsPerChunk].host.data() + at, nbar_ptr(c, s, 0),
+                           (size_t)(e - s) * 2 * nb * sizeof(double), hipMemcpyDeviceToHost,
+                           c->stream));
+    s = e;
+  }
+  G3L_HIP(hipStreamSynchronize(c->stream));
+  return G3L_OK;
 }
 
 }  // namespace
@@ -757,7 +789,7 @@ int g3l_ctx_destroy(g3l_ctx *c) {
   if (!c) return G3L_EINVAL;
   if (c->stream) (void)hipStreamSynchronize(c->stream);
   c->tables.release();
-  for (auto &b : c->nbar_chunks) b.release();
+  for (auto &b : c->nbar_chunks) b.dev.release();
   c->nbar_chunks.clear();
   c->pool.release(); c->split.release(); c->lists.release(); c->jobs.release();
   c->state.release(); c->args.release(); c->boxes.release(); c->counters.release();
@@ -812,10 +844,10 @@ int g3l_hodset_densities(g3l_ctx *c, int32_t set, double *rho_bar, double *n_bar
                          double *n_bar2) {
   if (!c || set < 0 || set >= (int)c->sets.size()) return G3L_EINVAL;
   if (rho_bar) std::memcpy(rho_bar, c->rho.data(), c->nb * sizeof(double));
-  if (n_bar1) G3L_HIP(hipMemcpy(n_bar1, nbar_ptr(c, set, 0), c->nb * sizeof(double),
-                                hipMemcpyDeviceToHost));
-  if (n_bar2) G3L_HIP(hipMemcpy(n_bar2, nbar_ptr(c, set, 1), c->nb * sizeof(double),
-                                hipMemcpyDeviceToHost));
+  const double *h = c->nbar_chunks[set / kSetsPerChunk].host.data() +
+                    (size_t)(set % kSetsPerChunk) * 2 * c->nb;
+  if (n_bar1) std::memcpy(n_bar1, h, c->nb * sizeof(double));
+  if (n_bar2) std::memcpy(n_bar2, h + c->nb, c->nb * sizeof(double));
   return G3L_OK;
 }
 

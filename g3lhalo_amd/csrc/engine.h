@@ -84,6 +84,13 @@ struct HodSet {
   int identical;
 };
 
+// n_bar of kSetsPerChunk HOD sets on the device and, for
+// g3l_hodset_densities, on the host.
+struct NbarChunk {
+  DevBuf dev;
+  std::vector<double> host;
+};
+
 // One refinement round recorded as an instantiated HIP graph (round_graph.cpp):
 // an evaluation node per kind in use, each between two event records (kev),
 // the counter clear, the selection over the integrals in flight, an event
@@ -138,7 +145,7 @@ struct g3l_ctx {
   std::vector<HodSet> sets;
   // n_bar per HOD set, [set][2][nb], in chunks of kSetsPerChunk sets that
   // never move: integrals in flight hold pointers into them.
-  std::vector<DevBuf> nbar_chunks;
+  std::vector<g3l::NbarChunk> nbar_chunks;
   // batched engine
   DevBuf pool, split, lists, jobs, state, args, boxes, counters;
   HostBuf hcounters;

@@ -36,11 +36,13 @@ struct OneDimUnit {
 };
 constexpr int kOneDimMaxUnit = 8;
 
-// Regions an integral may hold, nodes (regions of all its integrals, split
-// ones included) a block may hold.  An integral alone in a block cannot run
-// out of nodes: 2048 regions are the leaves of a tree of 4095.
+// Regions an integral may hold; most nodes (regions of all its integrals, split
+// ones included) a block may have room for.  An integral alone in a block with
+// that much room cannot run out: 2048 regions are the leaves of a tree of 4095.
 constexpr uint32_t kOneDimCap = 2048;
 constexpr uint32_t kOneDimNodes = 8192;
+// Nodes of a group's table of the top of its tree: twelve levels.
+constexpr uint32_t kOneDimTop = 4095;
 
 struct OneDimLaunch {
   DevTables T;                // kOneDNbar
@@ -49,7 +51,10 @@ struct OneDimLaunch {
   const OneDimUnit *units;
   uint32_t nunits;
   double reltol, scale;
-  unsigned char *store;       // one_dim_store_bytes() per block
+  unsigned char *store;       // store_bytes per block
+  size_t store_bytes;         // one_dim_store_bytes(nodes, waves)
+  uint32_t nodes, waves;      // nodes a block has room for; most integrals per unit
+  unsigned char *top;         // one_dim_top_bytes() per group, or null (n_bar)
   OneDimUnit *retry;          // integrals of units that ran out of nodes
   uint32_t *nretry;
   // smallest (integral's rank << 8 | job flags) over the integrals that end
@@ -57,10 +62,13 @@ struct OneDimLaunch {
   unsigned long long *failed;
 };
 
-// Device memory one block needs for its nodes and regions, and the blocks a
-// compute unit holds at a time.
-size_t one_dim_store_bytes();
+// Device memory of one block, and of a group's table; the blocks a compute
+// unit holds at a time.
+size_t one_dim_store_bytes(uint32_t nodes, uint32_t waves);
+size_t one_dim_top_bytes();
 int one_dim_blocks_per_cu();
+// Fills L.top for the groups [0, ngroups).
+hipError_t launch_one_dim_top(const OneDimLaunch &L, uint32_t ngroups, hipStream_t s);
 // Launches `blocks` blocks (at most L.nunits), each over a range of L.units.  precomp: the groups hold
 // precomputation modes (kOneDNbar otherwise).
 hipError_t launch_one_dim(bool precomp, const OneDimLaunch &L, uint32_t blocks, hipStream_t s);

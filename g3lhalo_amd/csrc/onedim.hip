@@ -22,9 +22,12 @@
 // integrals a block takes from one group.  Point values are the same
 // expressions in the same order whichever integral asked first.
 //
-// Measured: one HOD set (256 integrals) 3.7 -> 1.35 ms, 256 sets 104 -> 35 ms,
-// the precomputation 118 -> 14 ms.  What is left is instruction issue and the
-// latency of the selection, whose waves are alone with their integrals.
+// Measured, a call to its results on the host: one HOD set (256 integrals)
+// 3.7 -> 0.77 ms, 256 sets 104 -> 25 ms, the precomputation 118 -> 9 ms.  A round
+// of a block is a chain of a few microseconds each: the selection of one wave,
+// the scattered loads of the nodes' values (384 MB of them at 256 sets, from
+// HBM), the rule's 450 dependent instructions, three barriers; two blocks per
+// compute unit do not fill it.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -46,15 +49,46 @@ constexpr uint32_t kMaxSplit = kOneDimCap / 2;   // regions cut in one round
 constexpr uint32_t kChunk = 32;                  // regions reduced together (precomputation)
 static_assert(kChunk * kPts <= kThreads, "a point per thread");
 
-// Device memory of a block.  Node values are field-major so that the lanes of
-// a wave, which reduce neighbouring nodes, read neighbouring words.
+// Device memory of a block: `nodes` nodes and the regions of `waves` integrals.
+// Node values are field-major so that the lanes of a wave, which reduce
+// neighbouring nodes, read neighbouring words.
 struct Store {
-  double2 ab[kPts][kOneDimNodes];
-  int32_t ix[kPts][kOneDimNodes];
-  double c[kOneDimNodes], h[kOneDimNodes];
-  // regions of each wave's integral: rule value, error, node
-  double val[kWaves][kOneDimCap], err[kWaves][kOneDimCap];
-  uint16_t node[kWaves][kOneDimCap];
+  double2 *ab;            // [kPts][nodes]
+  int32_t *ix;            // [kPts][nodes]
+  double *c, *h;          // [nodes]
+  double *val, *err;      // [waves][kOneDimCap]: rule value, error
+  uint16_t *node;         // [waves][kOneDimCap]
+  uint32_t nodes;
+  __device__ __forceinline__ Store(unsigned char *p, uint32_t nodes_, uint32_t waves)
+      : nodes(nodes_) {
+    ab = reinterpret_cast<double2 *>(p);
+    c = reinterpret_cast<double *>(ab + (size_t)kPts * nodes);
+    h = c + nodes;
+    val = h + nodes;
+    err = val + (size_t)waves * kOneDimCap;
+    ix = reinterpret_cast<int32_t *>(err + (size_t)waves * kOneDimCap);
+    node = reinterpret_cast<uint16_t *>(ix + (size_t)kPts * nodes);
+  }
+};
+
+// The nodes a block reads: the first nd of them, the whole top of the tree in
+// breadth-first order, from its group's table (k_onedim_top; nd 0: none), the
+// others from its own store.
+struct TopStore {
+  double2 ab[kPts][kOneDimTop];
+  int32_t ix[kPts][kOneDimTop];
+  double c[kOneDimTop], h[kOneDimTop];
+};
+struct Nodes {
+  const TopStore *top;
+  Store own;
+  uint32_t nd;
+  __device__ __forceinline__ double c(uint32_t id) const {
+    return *(id < nd ? &top->c[id] : &own.c[id - nd]);
+  }
+  __device__ __forceinline__ double h(uint32_t id) const {
+    return *(id < nd ? &top->h[id] : &own.h[id - nd]);
+  }
 };
 
 struct WaveLds {
@@ -64,7 +98,9 @@ struct WaveLds {
 
 struct Lds {
   WaveLds w[kWaves];
-  uint32_t child[kOneDimNodes];        // first of a node's two children, 0: none
+  // first of a node's two children, 0: none; of node id at id - the number of
+  // nodes whose children are in the table (child_of)
+  uint32_t child[kOneDimNodes];
   uint16_t fresh[kOneDimNodes / 2];    // nodes split for the first time this round
   double f[kChunk * kPts];             // point values (precomputation)
   uint32_t nnodes, nfresh, full;
@@ -76,12 +112,22 @@ struct Lds {
 extern __shared__ __align__(16) unsigned char lds_raw[];
 __device__ __forceinline__ Lds &lds() { return *reinterpret_cast<Lds *>(lds_raw); }
 
+// Nodes of the table whose children are in the table too.
+__device__ __forceinline__ uint32_t inner(uint32_t nd) { return nd / 2; }
+__device__ __forceinline__ uint32_t child_of(uint32_t nd, uint32_t v) {
+  return v < inner(nd) ? 2 * v + 1 : lds().child[v - inner(nd)];
+}
+
 // The part of the integrand that depends on the abscissa alone.
 //   n_bar: ab = (m, Ncen + Nsat), ix = the mass index;
 //   sigma^2, d sigma^2/dm: ab = (amplitude T(k)^2, k^ns);
 //   distance, amplitude: ab.x = the integrand (one integral per group).
+//
+// Out of line, like wave_round: the kernel's loops around the inlined code kept
+// its FP64 constants in registers and spilled the rest (nbar of one HOD set
+// 0.89 ms inlined, 0.77 so).
 template <bool PRE>
-__device__ __forceinline__ void one_dim_node(const DevTables &T, const OneDimGroup &g, double t1,
+__device__ __noinline__ void one_dim_node(const DevTables &T, const OneDimGroup &g, double t1,
                                              double x, double2 &ab, int32_t &ix) {
   if constexpr (!PRE) {
     TermArgs a{};
@@ -105,7 +151,7 @@ __device__ __forceinline__ void one_dim_node(const DevTables &T, const OneDimGro
 }
 
 // The integrand of one integral from its node values.
-__device__ __forceinline__ double precomp_point(int mode, const OneDimJob &j, double x,
+__device__ __noinline__ double precomp_point(int mode, const OneDimJob &j, double x,
                                                 const double2 &ab) {
   if (mode == kOneDComoving || mode == kOneDAmplitude) return ab.x;
   const double spectrum = ab.x * j.t2 * j.t2 * ab.y;   // eh_spectrum's order
@@ -120,18 +166,18 @@ struct WaveState {
   double V;
 };
 
-// Totals, stop test and batch of one integral's n <= 64 R regions.  Sets
-// st.flags when it ends, otherwise st.K and the batch in W.split.
+// Totals, stop test and batch of one integral's n <= 64 R regions: its flags
+// when it ends, otherwise the size K of the batch, whose slots are in W.split.
 //
 // The totals keep the order they have in k_select, whose 256 threads take the
 // slots in strides and then add pairwise: lane l holds the threads l, l + 64,
 // l + 128 and l + 192.
 template <int R>
-__device__ __noinline__ void wave_round(const double *val, const double *err, double reltol,
-                                    WaveState &st) {
+__device__ __noinline__ WaveState wave_round(const double *val, const double *err, double reltol,
+                                             uint32_t n) {
   const int lane = threadIdx.x & 63;
   WaveLds &W = lds().w[threadIdx.x >> 6];
-  const uint32_t n = st.n;
+  WaveState st{n, 0, 0, 0.0};
   constexpr int V4 = R < 4 ? R : 4;
   constexpr int B = R < 8 ? R : 8;   // loads in flight per array
   uint64_t k[R];
@@ -182,7 +228,7 @@ __device__ __noinline__ void wave_round(const double *val, const double *err, do
   const double thr = fabs(V) * reltol;
   if (!(E > 0 && E > thr)) {
     st.flags |= kJobDone | kJobConverged;
-    return;
+    return st;
   }
   // every key is among these, so the boundary is
   Boundary Bd{};
@@ -190,7 +236,7 @@ __device__ __noinline__ void wave_round(const double *val, const double *err, do
   const uint32_t K = Bd.gt + Bd.take;
   if (n + K > kOneDimCap) {
     st.flags |= kJobDone | kJobPoolFull;
-    return;
+    return st;
   }
   st.K = K;
   // regions above T and the first `take` of those at T, in slot order
@@ -210,110 +256,115 @@ __device__ __noinline__ void wave_round(const double *val, const double *err, do
     if (s) W.split[at + lanes_below(sm)] = (uint16_t)(64 * r + lane);
     at += (uint32_t)__popcll(sm);
   }
+  return st;
 }
 
 // One round of this wave's integral, by the number of its regions, and the
 // nodes its batch needs: the first wave to split a node makes its children.
 __device__ __forceinline__ void wave_select(const double *val, const double *err,
-                                            const uint16_t *node, double reltol, WaveState &st) {
-  if (st.n <= 64) wave_round<1>(val, err, reltol, st);
-  else if (st.n <= 256) wave_round<4>(val, err, reltol, st);
-  else if (st.n <= 1024) wave_round<16>(val, err, reltol, st);
-  else wave_round<32>(val, err, reltol, st);
+                                            const uint16_t *node, double reltol, uint32_t nd,
+                                            uint32_t limit, WaveState &st) {
+  if (st.n <= 64) st = wave_round<1>(val, err, reltol, st.n);
+  else if (st.n <= 256) st = wave_round<4>(val, err, reltol, st.n);
+  else if (st.n <= 1024) st = wave_round<16>(val, err, reltol, st.n);
+  else st = wave_round<32>(val, err, reltol, st.n);
   Lds &S = lds();
   const WaveLds &W = S.w[threadIdx.x >> 6];
   wave_sync();
   for (uint32_t a = threadIdx.x & 63; a < st.K; a += 64) {
     const uint32_t v = node[W.split[a]];
-    if (atomicCAS(&S.child[v], 0u, ~0u) == 0u) {
+    if (v < inner(nd)) continue;
+    uint32_t *child = S.child - inner(nd);
+    if (atomicCAS(&child[v], 0u, ~0u) == 0u) {
       const uint32_t id = atomicAdd(&S.nnodes, 2u);
-      if (id + 2 <= kOneDimNodes) {
-        S.child[id] = 0;
-        S.child[id + 1] = 0;
-        S.child[v] = id;
+      if (id + 2 <= limit) {
+        child[id] = 0;
+        child[id + 1] = 0;
+        child[v] = id;
         S.fresh[atomicAdd(&S.nfresh, 1u)] = (uint16_t)v;
       } else {
-        S.child[v] = 0;
+        child[v] = 0;
         S.full = 1;
       }
     }
   }
 }
 
-// Region i of the block's round: the integral it belongs to (w), its node and
-// its slot.  An integral's regions are the left (even) and right (odd) halves
-// of those in its W.split; the left half keeps its parent's slot, the right
-// one takes the next free slot.
-__device__ __forceinline__ void place(const Store &G, uint32_t i, bool root, uint32_t &w,
-                                      uint32_t &id, uint32_t &slot) {
+// Region i of the block's round: region r = i / count of integral w = i mod
+// count (false if it has fewer), its node and its slot.  An integral's regions
+// are the left (even) and right (odd) halves of those in its W.split; the left
+// half keeps its parent's slot, the right one takes the next free slot.
+// Neighbouring lanes take the same rank of different integrals, mostly the
+// same node, whose values they then read together.
+__device__ __forceinline__ bool place(const Nodes &N, uint32_t i, uint32_t count, bool root,
+                                      uint32_t &w, uint32_t &id, uint32_t &slot) {
   const Lds &S = lds();
-  w = 0;
-  if (root) {
-    w = i;
-    id = 0;
-    slot = 0;
-    return;
-  }
-  uint32_t at = 0;
-#pragma unroll
-  for (int q = 0; q < kWaves - 1; ++q) {
-    const uint32_t next = at + 2 * S.cut[q];
-    if (i >= next && w == (uint32_t)q) {
-      ++w;
-      at = next;
-    }
-  }
-  const uint32_t r = i - at, p = S.w[w].split[r >> 1];
-  id = S.child[G.node[w][p]] + (r & 1u);
+  const uint32_t r = i / count;
+  w = i - r * count;
+  id = 0;
+  slot = 0;
+  if (root) return true;
+  if (r >= 2 * S.cut[w]) return false;
+  const uint32_t p = S.w[w].split[r >> 1];
+  id = child_of(N.nd, N.own.node[w * kOneDimCap + p]) + (r & 1u);
   slot = (r & 1u) ? S.n[w] + (r >> 1) : p;
+  return true;
 }
 
-// Rule sums of the `total` regions of the block's round (place), or of the
-// root of each of `total` integrals.  Every thread of the block calls it.
+// gk_reduce out of line.
+__device__ __noinline__ double2 gk_sums(const double *f, double h) {
+  double2 r;
+  gk_reduce(f, h, r.x, r.y);
+  return r;
+}
+
+// Rule sums of the `total` regions (place) of the round of the block's `count`
+// integrals, or of their roots.  Every thread of the block calls it.
 template <bool PRE>
-__device__ __forceinline__ void block_reduce(const OneDimLaunch &L, int mode, Store &G,
-                                             uint32_t total, bool root) {
+__device__ __forceinline__ void block_reduce(const OneDimLaunch &L, int mode, const Nodes &N,
+                                             uint32_t count, uint32_t total, bool root) {
   Lds &S = lds();
+  const Store &G = N.own;
   const uint32_t tid = threadIdx.x;
   if constexpr (!PRE) {
     // a region per thread: a point is two loads, a table look-up and two products
     for (uint32_t i = tid; i < total; i += kThreads) {
       uint32_t w, id, slot;
-      place(G, i, root, w, id, slot);
+      if (!place(N, i, count, root, w, id, slot)) continue;
       const double *hmf = L.T.hmf + S.row[w];
+      const bool top = id < N.nd;
+      const size_t stride = top ? kOneDimTop : G.nodes;
+      const double2 *ab = top ? &N.top->ab[0][id] : G.ab + (id - N.nd);
+      const int32_t *ix = top ? &N.top->ix[0][id] : G.ix + (id - N.nd);
       double f[kPts], v, e;
 #pragma unroll
       for (int j = 0; j < kPts; ++j) {
-        const double2 ab = G.ab[j][id];
-        f[j] = ab.x * hmf[G.ix[j][id]] * ab.y;
+        const double2 q = ab[j * stride];
+        f[j] = q.x * hmf[ix[j * stride]] * q.y;
       }
-      gk_reduce(f, G.h[id], v, e);
-      G.val[w][slot] = v;
-      G.err[w][slot] = e;
-      G.node[w][slot] = (uint16_t)id;
+      gk_reduce(f, N.h(id), v, e);
+      G.val[w * kOneDimCap + slot] = v;
+      G.err[w * kOneDimCap + slot] = e;
+      G.node[w * kOneDimCap + slot] = (uint16_t)id;
     }
   } else {
     // a point per thread: a point takes the window's sin and cos of a large
     // argument, and in most rounds every integral has two regions
     for (uint32_t i0 = 0; i0 < total; i0 += kChunk) {
       const uint32_t q = tid / kPts, i = i0 + q, j = tid - kPts * q;
-      if (q < kChunk && i < total) {
-        uint32_t w, id, slot;
-        place(G, i, root, w, id, slot);
-        const double c = G.c[id], h = G.h[id];
+      uint32_t w, id, slot;
+      if (q < kChunk && i < total && place(N, i, count, root, w, id, slot)) {
+        const double c = N.c(id), h = N.h(id);
         double x;
         rule_point<1>((int)j, &c, &h, &x);
-        S.f[tid] = precomp_point(mode, S.job[w], x, G.ab[j][id]);
+        S.f[tid] = precomp_point(mode, S.job[w], x, G.ab[(size_t)j * G.nodes + id]);
       }
       __syncthreads();
-      if (tid < kChunk && i0 + tid < total) {
-        uint32_t w, id, slot;
-        place(G, i0 + tid, root, w, id, slot);
-        double v, e;
-        gk_reduce(S.f + kPts * tid, G.h[id], v, e);
-        G.val[w][slot] = v;
-        G.err[w][slot] = e;
-        G.node[w][slot] = (uint16_t)id;
+      if (tid < kChunk && i0 + tid < total && place(N, i0 + tid, count, root, w, id, slot)) {
+        const double2 r = gk_sums(S.f + kPts * tid, N.h(id));
+        G.val[w * kOneDimCap + slot] = r.x;
+        G.err[w * kOneDimCap + slot] = r.y;
+        G.node[w * kOneDimCap + slot] = (uint16_t)id;
       }
       __syncthreads();
     }
@@ -328,7 +379,11 @@ template <bool PRE>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) void k_onedim(
     OneDimLaunch L) {
   Lds &S = lds();
-  Store &G = reinterpret_cast<Store *>(L.store)[blockIdx.x];
+  const Store G(L.store + (size_t)blockIdx.x * L.store_bytes, L.nodes, L.waves);
+  Nodes N{nullptr, G, PRE ? 0u : L.top ? kOneDimTop : 0u};
+  const uint32_t in = inner(N.nd);
+  // ids end where the children's table or the store does
+  const uint32_t limit = min(in + kOneDimNodes, N.nd + L.nodes);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   // a block takes consecutive units, whose integrals mostly share one group,
   // and keeps the nodes as long as the group stays
@@ -340,7 +395,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
     const OneDimGroup &g = L.groups[U.group];
     const bool mine = wave < (int)U.count;
     __syncthreads();   // the previous unit's LDS is done with
-    const bool reuse = have == U.group && S.nnodes <= kOneDimNodes / 2;
+    const bool reuse = have == U.group && S.nnodes - N.nd <= L.nodes / 2;
+    if (N.nd) N.top = reinterpret_cast<const TopStore *>(L.top) + U.group;
     const double t1 = L.jobs[g.job0 + U.first].t1;
     if (tid < (int)U.count) {
       const OneDimJob job = L.jobs[g.job0 + U.first + tid];
@@ -349,37 +405,46 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
     }
     __syncthreads();
     if (!reuse) {
-      if (tid == 0) {
-        S.nnodes = 1;
-        S.child[0] = 0;
-        G.c[0] = 0.5 * (g.lo + g.hi);
-        G.h[0] = 0.5 * (g.hi - g.lo);
-      }
-      if (tid < kPts) {
-        const double c = 0.5 * (g.lo + g.hi), h = 0.5 * (g.hi - g.lo);
-        double x;
-        rule_point<1>(tid, &c, &h, &x);
-        one_dim_node<PRE>(L.T, g, t1, x, G.ab[tid][0], G.ix[tid][0]);
+      if (N.nd) {   // the table's last level has no children yet
+        if (tid == 0) S.nnodes = N.nd;
+        for (uint32_t v = tid; v < N.nd - in; v += kThreads) S.child[v] = 0;
+      } else {
+        if (tid == 0) {
+          S.nnodes = 1;
+          S.child[0] = 0;
+          G.c[0] = 0.5 * (g.lo + g.hi);
+          G.h[0] = 0.5 * (g.hi - g.lo);
+        }
+        if (tid < kPts) {
+          const double c = 0.5 * (g.lo + g.hi), h = 0.5 * (g.hi - g.lo);
+          double x;
+          rule_point<1>(tid, &c, &h, &x);
+          one_dim_node<PRE>(L.T, g, t1, x, G.ab[(size_t)tid * G.nodes], G.ix[(size_t)tid * G.nodes]);
+        }
       }
     }
     if (tid == 0) S.full = 0;
     __syncthreads();
     WaveState st{1, mine ? 0u : (uint32_t)kJobDone, 0, 0.0};
-    block_reduce<PRE>(L, g.mode, G, U.count, true);
+    block_reduce<PRE>(L, g.mode, N, U.count, U.count, true);
     bool again = false;
     for (;;) {
       if (tid == 0) S.nfresh = 0;
       __syncthreads();
       st.K = 0;
-      if (!(st.flags & kJobDone)) wave_select(G.val[wave], G.err[wave], G.node[wave], L.reltol, st);
+      if (!(st.flags & kJobDone)) {
+        const size_t at = (size_t)wave * kOneDimCap;
+        wave_select(G.val + at, G.err + at, G.node + at, L.reltol, N.nd, limit, st);
+      }
       if (lane == 0) {
         S.n[wave] = st.n;
         S.cut[wave] = st.K;
       }
       __syncthreads();
-      uint32_t total = 0;
+      uint32_t most = 0;
 #pragma unroll
-      for (int q = 0; q < kWaves; ++q) total += 2 * S.cut[q];
+      for (int q = 0; q < kWaves; ++q) most = S.cut[q] > most ? S.cut[q] : most;
+      const uint32_t total = 2 * most * U.count;
       if (S.full) {
         // out of nodes: from the start with an empty tree; or, if it was
         // empty, its integrals one by one
@@ -392,19 +457,19 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
         const uint32_t pr = i / (2 * kPts), r = i - pr * 2 * kPts;
         const uint32_t right = r >= kPts ? 1u : 0u;
         const int j = (int)(r - right * kPts);
-        const uint32_t v = S.fresh[pr], id = S.child[v] + right;
+        const uint32_t v = S.fresh[pr], id = S.child[v - in] + right - N.nd;
         // the halves of a split, as in the cut of src/hcubature.cpp:206-218
-        const double h = G.h[v] * 0.5, c = right ? G.c[v] + h : G.c[v] - h;
+        const double h = N.h(v) * 0.5, c = right ? N.c(v) + h : N.c(v) - h;
         double x;
         rule_point<1>(j, &c, &h, &x);
-        one_dim_node<PRE>(L.T, g, t1, x, G.ab[j][id], G.ix[j][id]);
+        one_dim_node<PRE>(L.T, g, t1, x, G.ab[(size_t)j * G.nodes + id], G.ix[(size_t)j * G.nodes + id]);
         if (j == 0) {
           G.c[id] = c;
           G.h[id] = h;
         }
       }
       if (np) __syncthreads();
-      block_reduce<PRE>(L, g.mode, G, total, false);
+      block_reduce<PRE>(L, g.mode, N, U.count, total, false);
       st.n += st.K;
     }
     have = again ? ~0u : U.group;
@@ -424,7 +489,37 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
   }
 }
 
-size_t one_dim_store_bytes() { return (sizeof(Store) + 255) / 256 * 256; }
+// The top of every group's tree, kOneDimTop nodes in breadth-first order, a
+// point per thread (n_bar).  With fewer than two groups for every resident
+// block, several blocks would evaluate the same nodes, and a block alone with
+// one integral spends most of its time on them.
+__global__ __launch_bounds__(256) void k_onedim_top(OneDimLaunch L, TopStore *top) {
+  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= kOneDimTop * kPts) return;
+  const int j = (int)(i / kOneDimTop);
+  const uint32_t id = i - (uint32_t)j * kOneDimTop;
+  const OneDimGroup &g = L.groups[blockIdx.y];
+  // the path from the root: the bits of id + 1 below its leading one
+  double c = 0.5 * (g.lo + g.hi), h = 0.5 * (g.hi - g.lo), x;
+  for (int b = 30 - __clz((int)(id + 1)); b >= 0; --b) {
+    h *= 0.5;
+    c = (id + 1) >> b & 1u ? c + h : c - h;
+  }
+  rule_point<1>(j, &c, &h, &x);
+  TopStore &t = top[blockIdx.y];
+  one_dim_node<false>(L.T, g, 0.0, x, t.ab[j][id], t.ix[j][id]);
+  if (j == 0) {
+    t.c[id] = c;
+    t.h[id] = h;
+  }
+}
+
+size_t one_dim_store_bytes(uint32_t nodes, uint32_t waves) {
+  const size_t b = (size_t)nodes * (kPts * (sizeof(double2) + sizeof(int32_t)) + 2 * sizeof(double)) +
+                   (size_t)waves * kOneDimCap * (2 * sizeof(double) + sizeof(uint16_t));
+  return (b + 255) / 256 * 256;
+}
+size_t one_dim_top_bytes() { return sizeof(TopStore); }
 int one_dim_blocks_per_cu() { return 2; }
 
 template <bool PRE>
@@ -438,9 +533,19 @@ static hipError_t launch(const OneDimLaunch &L, uint32_t blocks, hipStream_t s) 
   return hipGetLastError();
 }
 
+hipError_t launch_one_dim_top(const OneDimLaunch &L, uint32_t ngroups, hipStream_t s) {
+  if (ngroups == 0 || ngroups > 65535) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_onedim_top, dim3((kOneDimTop * kPts + 255) / 256, ngroups), dim3(256), 0, s, L,
+                     reinterpret_cast<TopStore *>(L.top));
+  return hipGetLastError();
+}
+
 hipError_t launch_one_dim(bool precomp, const OneDimLaunch &L, uint32_t blocks, hipStream_t s) {
   if (L.nunits == 0) return hipSuccess;
-  if (blocks == 0 || blocks > L.nunits) return hipErrorInvalidValue;
+  if (blocks == 0 || blocks > L.nunits || (precomp && L.top) || L.nodes == 0 ||
+      L.nodes > kOneDimNodes || L.waves == 0 || L.waves > (uint32_t)kOneDimMaxUnit ||
+      L.store_bytes < one_dim_store_bytes(L.nodes, L.waves))
+    return hipErrorInvalidValue;
   return precomp ? launch<true>(L, blocks, s) : launch<false>(L, blocks, s);
 }
 

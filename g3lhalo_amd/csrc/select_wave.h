@@ -122,8 +122,6 @@ __device__ __forceinline__ uint32_t fewest(const Goal &g, uint64_t T, uint32_t e
 
 // LDS of one search.
 struct SearchLds {
-  unsigned long long sum[64];
-  uint32_t cnt[64];
   uint64_t key[64];
 };
 
@@ -143,16 +141,16 @@ __device__ __forceinline__ double sum_below(const uint64_t (&k)[R], uint32_t n, 
 // for one, so T is the largest key at which popping every key >= T is enough.
 // False if it is not among these keys.
 //
-// At most 64 keys: every lane sums the keys below its own.  More: a histogram
-// of the keys' distance below the largest (two bins per octave, fixed-point
-// sums) names the bin that holds the boundary, narrowed until at most kFew
-// keys are left, whose lanes do the same.  A boundary that the truncated sums
-// put into the wrong bin shows in the exact sums and is then found by
+// A search over the keys' high words, with FP32 sums of what remains, leaves
+// an interval of at most kFew keys; every lane then sums the keys below its
+// own exactly.  All of it is in registers (a histogram in LDS, with its
+// atomics and scans, took five times as long).  A boundary that the FP32 sums
+// put outside the interval shows in the exact sums and is then found by
 // bisection over the key's bits.
 template <int R>
 __device__ __forceinline__ bool find_boundary(const uint64_t (&k)[R], uint32_t n, uint64_t maxkey,
                                               const Goal &g, SearchLds &W, Boundary &B) {
-  constexpr uint32_t kFew = 24;   // a lane's sum costs as much as a narrowing pass per 24 keys
+  constexpr uint32_t kFew = 12;   // a lane's sums over them cost as much as four search steps
   const int lane = threadIdx.x & 63;
   // most often in a bisection towards a peak, only the largest goes
   if constexpr (R == 1) {
@@ -167,81 +165,74 @@ __device__ __forceinline__ bool find_boundary(const uint64_t (&k)[R], uint32_t n
   uint32_t m = n;                        // candidates
   uint32_t above = g.above;              // keys above every candidate
   double below = g.below;                // sum of the keys below every candidate
-  if constexpr (R > 1) {
-    const int shift = sel_shift(maxkey, n);
-    const double thr_fx = ldexp(g.thr - g.below, shift);
-    // candidates: distance d = maxkey - key in [lo, lo + width)
-    uint64_t lo = 0, width = 1ull << 63;
-    int s = 51;
-    unsigned long long rest_after = 0;  // fixed-point sum of the keys beyond the range
-    for (;;) {
-      W.sum[lane] = 0;
-      W.cnt[lane] = 0;
-      wave_sync();
+  if (R > 1 || n > kFew) {
+    // keys in units of the largest's exponent
+    const int ex = -((int)(maxkey >> 52) - 1023);
+    const float thr = (float)ldexp(g.thr - g.below, ex);
+    float f[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) f[r] = (float)ldexp(__builtin_bit_cast(double, k[r]), ex);
+    const uint32_t mh = (uint32_t)(maxkey >> 32);
+    // whether popping every key with a high word >= t is enough; cnt: the keys
+    // below
+    auto enough = [&](uint32_t t, uint32_t &cnt) {
+      float s = 0;
+      cnt = 0;
 #pragma unroll
       for (int r = 0; r < R; ++r) {
         if (64u * r >= n) break;
-        const uint64_t d = maxkey - k[r] - lo;
-        if (k[r] <= maxkey && k[r] <= maxkey - lo && d < width) {
-          const uint64_t q = d >> s;
-          const int b = q < 63 ? (int)q : 63;
-          atomicAdd(&W.cnt[b], 1u);
-          atomicAdd(&W.sum[b], fixed_err(k[r], shift));
-        }
+        const bool b = (uint32_t)(k[r] >> 32) < t;
+        s += b ? f[r] : 0.0f;
+        cnt += (uint32_t)__popcll(__ballot(b));
       }
-      wave_sync();
-      const unsigned long long own = W.sum[lane];
-      const uint32_t cown = W.cnt[lane];
-      unsigned long long suf = own;   // in the range, this bin and beyond
-      uint32_t pre = cown;            // in the range, this bin and before
-#pragma unroll
-      for (int w = 1; w < 64; w <<= 1) {
-        const uint32_t l2 = __shfl_down((uint32_t)suf, w), h2 = __shfl_down((uint32_t)(suf >> 32), w);
-        const uint32_t p2 = __shfl_up(pre, w);
-        if (lane + w < 64) suf += ((unsigned long long)h2 << 32) | l2;
-        if (lane >= w) pre += p2;
+      tree([&](auto w) {
+        s += __builtin_bit_cast(float, from_above32<decltype(w)::value>(__builtin_bit_cast(uint32_t, s)));
+      });
+      s = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(uint32_t, s)));
+      return s <= thr || (uint64_t)g.above + n - cnt >= g.kcap;
+    };
+    // enough at lo, not at hi: two octaves below the largest key, then four,
+    // eight, ..., then halving
+    uint32_t lo = 0, hi = mh + 1, nlo = 0, nhi = n, c = 0;
+    for (uint32_t d = 2u << 20; d < mh && nhi - nlo > kFew; d <<= 1) {
+      if (enough(mh - d, c)) {
+        lo = mh - d;
+        nlo = c;
+        break;
       }
-      const unsigned long long rest = suf - own + rest_after;
-      const uint64_t some = __ballot(cown != 0);
-      const uint64_t hit =
-          __ballot(((double)rest <= thr_fx || (uint64_t)above + pre >= g.kcap) && cown != 0);
-      const int b = hit ? __ffsll((unsigned long long)hit) - 1 : 63 - __clzll((long long)some);
-      m = (uint32_t)__builtin_amdgcn_readlane((int)cown, b);
-      above += (uint32_t)__builtin_amdgcn_readlane((int)(pre - cown), b);
-      rest_after = readlane64((uint64_t)rest, b);
-      lo += (uint64_t)b << s;
-      width = b == 63 ? width - ((uint64_t)63 << s) : 1ull << s;
-      if (m <= kFew || width <= 1) break;
-      s = 58 - __clzll((long long)(width - 1));   // ceil(log2 width) - 6
-      s = s < 0 ? 0 : s;
+      hi = mh - d;
+      nhi = c;
     }
-    const uint64_t kmax = maxkey - lo, kmin = kmax >= width - 1 ? kmax - (width - 1) : 0;
+    while (nhi - nlo > kFew && hi - lo > 1) {
+      const uint32_t t = lo + ((hi - lo) >> 1);
+      if (enough(t, c)) {
+        lo = t;
+        nlo = c;
+      } else {
+        hi = t;
+        nhi = c;
+      }
+    }
+    m = nhi - nlo;
+    above += n - nhi;
+    const uint64_t klo = (uint64_t)lo << 32, khi = (uint64_t)hi << 32;
     double bs = 0, bc = 0;
     uint32_t at = 0;
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       if (64u * r >= n) break;
-      comp_add(bs, bc, k[r] < kmin ? __builtin_bit_cast(double, k[r]) : 0.0);
-      if (m <= kFew) {
-        const bool in = k[r] <= kmax && k[r] >= kmin;
+      comp_add(bs, bc, k[r] < klo ? __builtin_bit_cast(double, k[r]) : 0.0);
+      if (m <= 64) {
+        const bool in = k[r] < khi && k[r] >= klo;
         const uint64_t bm = __ballot(in);
         if (in) W.key[at + lanes_below(bm)] = k[r];
         at += (uint32_t)__popcll(bm);
       }
     }
     below += comp_total(bs, bc);
-    if (m > kFew) {   // one key, many regions
-      const double all = below + (double)m * __builtin_bit_cast(double, kmax);
-      if ((meets(below, g.thr) || (uint64_t)above + m >= g.kcap) &&
-          (above == 0 || !(meets(all, g.thr) || above >= g.kcap))) {
-        B = Boundary{kmax, m, fewest(g, kmax, m, above, below), above};
-        return true;
-      }
-      m = 0;
-    } else {
-      wave_sync();
-      ck = lane < (int)m ? W.key[lane] : ~0ull;
-    }
+    wave_sync();
+    if (m > 64) m = 0;   // more equal high words than lanes
+    ck = lane < (int)m ? W.key[lane] : ~0ull;
   }
   if (m) {
     double s = 0, c = 0;
@@ -268,7 +259,6 @@ __device__ __forceinline__ bool find_boundary(const uint64_t (&k)[R], uint32_t n
       B.take = fewest(g, T, B.eq, B.gt, readlane64(after, who));
       return true;
     }
-    if constexpr (R == 1) return false;
   }
   // the largest T <= maxkey at which popping every key >= T is enough (it is a
   // key: the remaining error and the count only change just above one)
