@@ -15,8 +15,9 @@
 //
 // Deviations of P64 from the reference that change only the last bits:
 // u_NFW by the cancellation-free branch identities noted at u_nfw, with
-// Si/Ci's polynomials summed over precomputed powers, sin/cos by our own
-// Cody-Waite/Taylor routine and the ln x of Ci(x) by fdlibm's method
+// polynomials of its own for Si/Ci and sin/cos below 4 (u_small), the
+// reference's approximants of Si/Ci by Horner's rule above, sin/cos there by
+// our own Cody-Waite routine and the ln x of Ci(x) by fdlibm's method
 // (log_pos); the HOD logarithms and powers from log(m/mmin); cbrt for
 // pow(., 1/3); exp10 for the 10^x of l1, l2; the redshift-only projection
 // factor multiplied into B in one step; shared sin/cos of one argument;
@@ -56,6 +57,20 @@ G3L_HD double fdiv(double a, double b) {
   return fma(fma(-b, q, a), r, q);
 #else
   return a / b;
+#endif
+}
+
+// a z + c, c a constant.  The compiler's choice for it, the two-address FMA,
+// takes the addend in vector registers, two moves per constant; the three-operand
+// FMA takes it from scalar registers, which makes a Horner step one vector
+// instruction.
+G3L_HD double fma_k(double a, double z, double c) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  double r;
+  asm("v_fma_f64 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(z), "s"(c));
+  return r;
+#else
+  return fma(a, z, c);
 #endif
 }
 
@@ -149,7 +164,7 @@ G3L_HD void sincos_cw(double x, double &s, double &c) {
 // sin and cos together as sincos_cw, with the minimax polynomials of
 // fdlibm's __kernel_sin and __kernel_cos (Sun Microsystems, 1993: degree 13
 // and 14 in r on |r| <= pi/4, approximation errors below 4e-18 relative)
-// instead of the Taylor series: two terms and one power of r^2 fewer.
+// instead of the Taylor series, by Horner's rule.
 G3L_HD void sincos_mm(double x, double &s, double &c) {
   if (!(fabs(x) < 1048576.0)) {
     sincos(x, &s, &c);
@@ -158,22 +173,18 @@ G3L_HD void sincos_mm(double x, double &s, double &c) {
   int q;
   const double r = sincos_reduce(x, q);
   const double z = r * r;
-  const double z2 = z * z, z3 = z2 * z, z4 = z2 * z2;
-  const double z5 = z4 * z, z6 = z3 * z3, z7 = z4 * z3;
-  double ps = -1.66666666666666324348e-01 * z;
-  ps = fma(8.33333333332248946124e-03, z2, ps);
-  ps = fma(-1.98412698298579493134e-04, z3, ps);
-  ps = fma(2.75573137070700676789e-06, z4, ps);
-  ps = fma(-2.50507602534068634195e-08, z5, ps);
-  ps = fma(1.58969099521155010221e-10, z6, ps);
-  double pc = -0.5 * z;
-  pc = fma(4.16666666666666019037e-02, z2, pc);
-  pc = fma(-1.38888888888741095749e-03, z3, pc);
-  pc = fma(2.48015872894767294178e-05, z4, pc);
-  pc = fma(-2.75573143513906633035e-07, z5, pc);
-  pc = fma(2.08757232129817482790e-09, z6, pc);
-  pc = fma(-1.13596475577881948265e-11, z7, pc);
-  sincos_select(q, fma(r, ps, r), 1.0 + pc, s, c);
+  double ps = 1.58969099521155010221e-10 * z + -2.50507602534068634195e-08;
+  ps = fma_k(ps, z, 2.75573137070700676789e-06);
+  ps = fma_k(ps, z, -1.98412698298579493134e-04);
+  ps = fma_k(ps, z, 8.33333333332248946124e-03);
+  ps = fma_k(ps, z, -1.66666666666666324348e-01);
+  double pc = -1.13596475577881948265e-11 * z + 2.08757232129817482790e-09;
+  pc = fma_k(pc, z, -2.75573143513906633035e-07);
+  pc = fma_k(pc, z, 2.48015872894767294178e-05);
+  pc = fma_k(pc, z, -1.38888888888741095749e-03);
+  pc = fma_k(pc, z, 4.16666666666666019037e-02);
+  pc = fma_k(pc, z, -0.5);
+  sincos_select(q, fma(r * z, ps, r), fma(pc, z, 1.0), s, c);
 }
 
 // Tables resident in HBM (z-major 2-D tables, nb*nb + nb for P_lin).
@@ -506,54 +517,178 @@ G3L_HD double u_nfw_a1(double a1, const Nfw &n) {
       (c1 - 1) * n.lc + fdiv(a1 * n.c - sx, a2) + c1 * (cr2 - cr1) + s1 * (si2 - si1);
   return 1 + fdiv(rest, n.F);
 }
-// u_nfw_a1 with sin and cos by sincos_mm and each branch's quotients over
-// one common denominator, so that one division replaces six (a2 < 4: Si and
-// Cr at a1 and a2, (a1 c - sin a1 c) / a2 and / F), five (a1 < 4 <= a2: Si and Cr at a1, g
-// and f - 1/x at a2, / F) or four (a1 >= 4: g at a1, g and f - 1/x at a2,
-// / F).  Equal to u_nfw_a1 in exact arithmetic; the denominators are
-// products of the approximants' denominators (each at least 1, and at most
-// about 6e5 for arguments near 4 or x itself for large ones) with a2 and F,
-// so nothing overflows and no new cancellation appears.  With a2 < 4, over D = a2 Cd1 Cd2 Sd1 Sd2 F:
-//   u = 1 + { [a2 (cos a1 - 1) ln(1+c) + a1 c - sin a1 c] Cd1 Cd2 Sd1 Sd2
-//             + a2 [cos a1 (Cn2 Cd1 - Cn1 Cd2) Sd1 Sd2
-//                   + sin a1 (Sn2 Sd1 - Sn1 Sd2) Cd1 Cd2] } / D.
+// The pieces of u_NFW for arguments below 4, as polynomials in z = x^2 on
+// [0, 16]: Chebyshev interpolants of the entire functions (degrees 10 and 11),
+// with errors below 3e-17 of the value at 0.
+// (x - sin x) / x^3
+G3L_HD double poly_xsin(double z) {
+  double p = 3.339444591791031e-23 * z + -1.937676456347459e-20;
+  p = fma_k(p, z, 8.216472067542675e-18);
+  p = fma_k(p, z, -2.811402128165303e-15);
+  p = fma_k(p, z, 7.647159031372368e-13);
+  p = fma_k(p, z, -1.6059043579072406e-10);
+  p = fma_k(p, z, 2.5052108376622883e-08);
+  p = fma_k(p, z, -2.7557319223809765e-06);
+  p = fma_k(p, z, 0.00019841269841268036);
+  p = fma_k(p, z, -0.008333333333333326);
+  p = fma_k(p, z, 0.16666666666666666);
+  return p;
+}
+// (cos x - 1) / x^2
+G3L_HD double poly_cosm(double z) {
+  double p = -7.582350097421893e-22 * z + 4.0616419875880403e-19;
+  p = fma_k(p, z, -1.5608887230789617e-16);
+  p = fma_k(p, z, 4.779340762698611e-14);
+  p = fma_k(p, z, -1.1470733957090858e-11);
+  p = fma_k(p, z, 2.087675634971086e-09);
+  p = fma_k(p, z, -2.7557319202155186e-07);
+  p = fma_k(p, z, 2.4801587301151354e-05);
+  p = fma_k(p, z, -0.0013888888888884423);
+  p = fma_k(p, z, 0.04166666666666649);
+  p = fma_k(p, z, -0.5);
+  return p;
+}
+// sin x / x
+G3L_HD double poly_sin(double z) {
+  double p = -3.294601866401345e-23 * z + 1.9338192090494286e-20;
+  p = fma_k(p, z, -8.215043677309279e-18);
+  p = fma_k(p, z, 2.8113723473966215e-15);
+  p = fma_k(p, z, -7.647155193625167e-13);
+  p = fma_k(p, z, 1.6059043263207725e-10);
+  p = fma_k(p, z, -2.5052108360050594e-08);
+  p = fma_k(p, z, 2.755731922327296e-06);
+  p = fma_k(p, z, -0.00019841269841258026);
+  p = fma_k(p, z, 0.008333333333333233);
+  p = fma_k(p, z, -0.16666666666666663);
+  p = fma_k(p, z, 1.0);
+  return p;
+}
+// Si(x) / x
+G3L_HD double poly_si(double z) {
+  double p = 7.948510839918774e-22 * z + -4.27584084925101e-19;
+  p = fma_k(p, z, 1.6527211282491636e-16);
+  p = fma_k(p, z, -5.097966588511523e-14);
+  p = fma_k(p, z, 1.2353098491764215e-11);
+  p = fma_k(p, z, -2.277464332056993e-09);
+  p = fma_k(p, z, 3.0619243559416514e-07);
+  p = fma_k(p, z, -2.8344671201358953e-05);
+  p = fma_k(p, z, 0.0016666666666662003);
+  p = fma_k(p, z, -0.05555555555555537);
+  p = fma_k(p, z, 1.0);
+  return p;
+}
+// (Ci(x) - gamma - ln x) / x^2
+G3L_HD double poly_cr(double z) {
+  double p = -3.493121348033495e-23 * z + 2.0347178104854336e-20;
+  p = fma_k(p, z, -8.672999135077456e-18);
+  p = fma_k(p, z, 2.987115889509022e-15);
+  p = fma_k(p, z, -8.193384814579168e-13);
+  p = fma_k(p, z, 1.7397297221300852e-10);
+  p = fma_k(p, z, -2.7557319214796103e-08);
+  p = fma_k(p, z, 3.1001984126800588e-06);
+  p = fma_k(p, z, -0.00023148148148146268);
+  p = fma_k(p, z, 0.01041666666666666);
+  p = fma_k(p, z, -0.25);
+  return p;
+}
+
+// g(x) = gn / gd and f(x) - 1/x = fn / fd as in sici_aux_nd, by Horner's rule.
+G3L_HD void sici_aux_k(double x, double &gn, double &gd, double &fn, double &fd) {
+  const double t = fdiv(1.0, x * x);
+  double fq = 1.11535493509914254097e13 * t + 1.43468549171581016479e13;
+  fq = fma_k(fq, t, 5.06084464593475076774e12);
+  fq = fma_k(fq, t, 7.08501308149515401563e11);
+  fq = fma_k(fq, t, 4.58595115847765779830e10);
+  fq = fma_k(fq, t, 1.47478952192985464958e9);
+  fq = fma_k(fq, t, 2.41535670165126845144e7);
+  fq = fma_k(fq, t, 1.97865247031583951450e5);
+  fq = fma_k(fq, t, 7.46437068161927678031e2);
+  fq = fma_k(fq, t, 1.0);
+  double dn = -4.94701168645415954590e11 * t + -6.20538246899190625000e12;
+  dn = fma_k(dn, t, -4.26733661912124414062e12);
+  dn = fma_k(dn, t, -8.51162840223981323242e11);
+  dn = fma_k(dn, t, -6.79674775754933776855e10);
+  dn = fma_k(dn, t, -2.48588769773332548141e9);
+  dn = fma_k(dn, t, -4.40554837171082794666e7);
+  dn = fma_k(dn, t, -3.78536003969501121901e5);
+  dn = fma_k(dn, t, -1.46887413643708168820e3);
+  dn = fma_k(dn, t, -1.99999999999097743952e0);
+  double gp = -1.36517137670871689e12 * t + 6.43291613143049485e12;
+  gp = fma_k(gp, t, 1.81004487464664575e13);
+  gp = fma_k(gp, t, 7.57664583257834349e12);
+  gp = fma_k(gp, t, 1.09049528450362786e12);
+  gp = fma_k(gp, t, 6.83052205423625007e10);
+  gp = fma_k(gp, t, 2.06297595146763354e9);
+  gp = fma_k(gp, t, 3.12557570795778731e7);
+  gp = fma_k(gp, t, 2.35239181626478200e5);
+  gp = fma_k(gp, t, 8.1359520115168615e2);
+  gp = fma_k(gp, t, 1.0);
+  double gq = 3.99653257887490811e13 * t + 4.01839087307656620e13;
+  gq = fma_k(gq, t, 1.17164723371736605e13);
+  gq = fma_k(gq, t, 1.39866710696414565e12);
+  gq = fma_k(gq, t, 7.87465017341829930e10);
+  gq = fma_k(gq, t, 2.23355543278099360e9);
+  gq = fma_k(gq, t, 3.26026661647090822e7);
+  gq = fma_k(gq, t, 2.40036752835578777e5);
+  gq = fma_k(gq, t, 8.19595201151451564e2);
+  gq = fma_k(gq, t, 1.0);
+  gn = gp * t;
+  gd = gq;
+  fn = dn * t;
+  fd = fq * x;
+}
+
+// u_NFW for a2 < 4, z1 = a1^2: with no reduction of the arguments and one
+// division,
+//   u = 1 + { a2 [(cos a1 - 1) ln(1+c) + cos a1 (Cr a2 - Cr a1)
+//             + sin a1 (Si a2 - Si a1)] + (a1 c - sin a1 c) } / (a2 F).
+G3L_HD double u_small(double a1, double a2, const Nfw &n) {
+  const double x = a1 * n.c;
+  const double z1 = a1 * a1, z2 = a2 * a2, zx = x * x;
+  const double cm = z1 * poly_cosm(z1);
+  const double s1 = a1 * poly_sin(z1);
+  const double dC = fma(z2, poly_cr(z2), -z1 * poly_cr(z1));
+  const double dS = fma(a2, poly_si(z2), -a1 * poly_si(z1));
+  const double rest = fma(cm, n.lc, fma(s1, dS, fma(cm, dC, dC)));
+  const double num = fma(a2, rest, x * zx * poly_xsin(zx));
+  return 1 + fdiv(num, a2 * n.F);
+}
+
+// u_nfw_a1 in the form of the FP64 policy: polynomials for what depends on
+// arguments below 4, Horner's rule throughout, and one division: where the
+// Si/Ci approximants of arguments above 4 enter, each branch's quotients are
+// over one common denominator (products of the approximants' denominators,
+// each at least 1 and at most about 6e5 for arguments near 4 or x itself for
+// large ones, with F: nothing overflows and no new cancellation appears).
+// Equal to u_nfw_a1 in exact arithmetic up to the approximants' own errors
+// below 4, which the polynomials do not have: against the transform at 40
+// digits (c from 0.04 to 25) the largest error with a2 < 4 is 2.7e-15 for c >= 1
+// and 3.8e-13 below (6.6e-15 and 9.6e-13 with the approximants), the other
+// branches' is unchanged.  About 105 vector instructions with a2 < 4 instead of
+// 175: NNMap 1h launches of the 550-triplet workload 90.2 -> 80.7 ms per run,
+// 2h 116 -> 104 ms, NMapMap 1h and 2h 11 % less.
 template <class P>
 G3L_HD double u_nfw_a1_1q(double a1, const Nfw &n) {
   const double a2 = a1 * (1 + n.c);
-  double sx, cx;
+  if (a2 < 4) return u_small(a1, a2, n);
+  double sx, cx, gn2, gd2, fn2, fd2;
   sincos_mm(a1 * n.c, sx, cx);
-  double s1 = 0, c1 = 0, sn1 = 0, sd1 = 1, cn1 = 0, cd1 = 1;
-  double gn2 = 0, gd2 = 1, fn2 = 0, fd2 = 1;
-  if (a1 < 4) {
-    sincos_mm(a1, s1, c1);
-    sici_small_nd(a1, sn1, sd1, cn1, cd1);
-  }
-  if (a2 >= 4) sici_aux_nd(a2, gn2, gd2, fn2, fd2);
+  sici_aux_k(a2, gn2, gd2, fn2, fd2);
+  const double p2 = fd2 * gd2;
+  const double r2 = sx * fn2 * gd2 - cx * gn2 * fd2;
   if (a1 >= 4) {
     // u F = g(a1) + sin(a1 c) (f(a2) - 1/a2) - g(a2) cos(a1 c)
     double gn1, gd1, fn1, fd1;
-    sici_aux_nd(a1, gn1, gd1, fn1, fd1);
-    const double p2 = fd2 * gd2;
-    const double r2 = sx * fn2 * gd2 - cx * gn2 * fd2;
+    sici_aux_k(a1, gn1, gd1, fn1, fd1);
     return fdiv(fma(gn1, p2, gd1 * r2), gd1 * p2 * n.F);
   }
-  if (a2 >= 4) {
-    // u F = pi/2 sin a1 - cos a1 (gamma + ln a1) - sin a1 Si(a1) - cos a1 Cr(a1)
-    //       + sin(a1 c) (f(a2) - 1/a2) - g(a2) cos(a1 c)
-    const double A = 0.5 * 3.14159265358979323846 * s1 - c1 * (0.5772156649 + P::ln_ci(a1));
-    const double p1 = sd1 * cd1, p2 = fd2 * gd2;
-    const double r1 = s1 * sn1 * cd1 + c1 * cn1 * sd1;
-    const double r2 = sx * fn2 * gd2 - cx * gn2 * fd2;
-    return fdiv(fma(A, p1, -r1) * p2 + r2 * p1, p1 * p2 * n.F);
-  }
-  double sn2, sd2, cn2, cd2;
-  sici_small_nd(a2, sn2, sd2, cn2, cd2);
-  const double C = cd1 * cd2, S = sd1 * sd2, CS = C * S;
-  const double dC = fma(cn2, cd1, -cn1 * cd2);
-  const double dS = fma(sn2, sd1, -sn1 * sd2);
-  const double t0 = fma((c1 - 1) * n.lc, a2, a1 * n.c - sx);
-  const double num = fma(t0, CS, a2 * fma(c1 * dC, S, s1 * dS * C));
-  return 1 + fdiv(num, a2 * CS * n.F);
+  // u F = pi/2 sin a1 - cos a1 (gamma + ln a1) - sin a1 Si(a1) - cos a1 Cr(a1)
+  //       + sin(a1 c) (f(a2) - 1/a2) - g(a2) cos(a1 c)
+  const double z1 = a1 * a1;
+  const double c1 = fma(z1, poly_cosm(z1), 1.0), s1 = a1 * poly_sin(z1);
+  const double ci = 0.5772156649 + P::ln_ci(a1) + z1 * poly_cr(z1);
+  const double A = s1 * (0.5 * 3.14159265358979323846 - a1 * poly_si(z1)) - c1 * ci;
+  return fdiv(fma(A, p2, r2), p2 * n.F);
 }
 // a1 = k r200 / c of u_NFW.
 G3L_HD double nfw_a1(const Nfw &n, double k) { return fdiv(k * n.r200, n.c); }
@@ -633,26 +768,6 @@ struct P64R : P64 {
   G3L_HD static double u(const Nfw &n, double k) { return u_nfw<P64R>(n, k); }
   G3L_HD static double u_a1(double a1, const Nfw &n) { return u_nfw_a1<P64R>(a1, n); }
 };
-
-// u_NFW for a2 < 4 (small k r_s), the FP64 branch of P64::u on its own:
-//   u = 1 + [(cos a1 - 1) ln(1+c) + (a1 c - sin a1 c)/a2
-//            + cos a1 (Cr(a2) - Cr(a1)) + sin a1 (Si a2 - Si a1)] / F,
-// over one common denominator as in u_nfw_a1_1q.  The Si/Ci differences of
-// nearby arguments and the 1 - O(a1^2) structure need FP64 here; equal to
-// P64::u bit for bit in this branch.
-G3L_HD double u_small64(const Nfw &n, double a1, double a2) {
-  double sx, cx, s1, c1, sn1, sd1, cn1, cd1, sn2, sd2, cn2, cd2;
-  sincos_mm(a1 * n.c, sx, cx);
-  sincos_mm(a1, s1, c1);
-  sici_small_nd(a1, sn1, sd1, cn1, cd1);
-  sici_small_nd(a2, sn2, sd2, cn2, cd2);
-  const double C = cd1 * cd2, S = sd1 * sd2, CS = C * S;
-  const double dC = fma(cn2, cd1, -cn1 * cd2);
-  const double dS = fma(sn2, sd1, -sn1 * sd2);
-  const double t0 = fma((c1 - 1) * n.lc, a2, a1 * n.c - sx);
-  const double num = fma(t0, CS, a2 * fma(c1 * dC, S, s1 * dS * C));
-  return 1 + fdiv(num, a2 * CS * n.F);
-}
 
 // ======================================================================
 // Mixed policy: FP32 transcendental bulk.
@@ -775,7 +890,7 @@ struct PMix {
     double a2d = a1d * (1 + n.c);
     // small k r_s: u = 1 - O(a1^2) from differences of nearby Si/Ci values,
     // kept in FP64
-    if (a2d < 4.0) return u_small64(n, a1d, a2d);
+    if (a2d < 4.0) return u_small(a1d, a2d, n);
     double xd = a1d * n.c;
     float sx, cxx;
     mix::sincos_red(xd, sx, cxx);
