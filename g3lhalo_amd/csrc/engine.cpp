@@ -26,7 +26,11 @@ const double kC = 2.99792e5;
 const double kGMsun = 1.327e11;
 const double kMpcKm = 3.086e19;
 
-DevHod to_dev(const g3l_hod &h) { return DevHod{h.f, h.alpha, h.mth, h.sigma, h.mprime, h.beta}; }
+// A sigma below 1e-300 is as good as 1e-300: log(m / M_th) is zero or at least
+// 1e-16, so the error function saturates either way, and x / sigma stays finite.
+DevHod to_dev(const g3l_hod &h) {
+  return DevHod{h.f, h.alpha, h.mth, std::max(h.sigma, 1e-300), h.mprime, h.beta};
+}
 
 }  // namespace
 
@@ -80,6 +84,8 @@ TermArgs make_args(const g3l_ctx *c, const g3l_request &r) {
     a.nb2 = nbar_ptr(c, r.hodset, a2 ? 0 : 1);
     a.same = (a1 == a2) || s.identical;
   }
+  a.rs1 = 1. / a.h1.sigma;
+  a.rs2 = 1. / a.h2.sigma;
   fill_logs(c, a);
   return a;
 }
@@ -687,6 +693,7 @@ int compute_nbar(g3l_ctx *c, int first, int count) {
     for (int which = 0; which < 2; ++which) {
       OneDimGroup g{};
       g.h = to_dev(which == 0 ? c->sets[s].h1 : c->sets[s].h2);
+      g.rs = 1. / g.h.sigma;
       g.lo = std::log10(c->mmin_i);
       g.hi = std::log10(c->mmax_i);
       g.out = const_cast<double *>(nbar_ptr(c, s, which));
@@ -745,7 +752,7 @@ int g3l_ctx_create(const g3l_tables *t, g3l_ctx **out) {
     c->rho[i] = c->Om * (1 + z) * (1 + z) * (1 + z) / E * c->rho_crit;
   }
   const size_t n1 = nb, n2 = (size_t)nb * nb;
-  const size_t total = 6 * n1 + 4 * n2 + n1;
+  const size_t total = 8 * n1 + 4 * n2 + n1;
   if (c->tables.ensure(total * sizeof(double))) {
     g3l_ctx_destroy(c);
     return G3L_ENOMEM;
@@ -758,6 +765,12 @@ int g3l_ctx_create(const g3l_tables *t, g3l_ctx **out) {
     p += n;
     return (size_t)(at - h.data());
   };
+  std::vector<double> rw(nb), rrho(nb);
+  for (int i = 0; i < nb; ++i) {
+    rw[i] = 1. / t->w[i];
+    rrho[i] = 1. / c->rho[i];
+  }
+  const size_t orw = put(rw.data(), n1), orr = put(rrho.data(), n1);
   size_t og = put(t->g, n1), op1 = put(t->p_lens1, n1),
          op2 = put(t->p_lens2 ? t->p_lens2 : t->p_lens1, n1), ow = put(t->w, n1),
          odw = put(t->dwdz, n1), orho = put(c->rho.data(), n1), ohmf = put(t->hmf, n2),
@@ -779,6 +792,13 @@ int g3l_ctx_create(const g3l_tables *t, g3l_ctx **out) {
   T.mmin = c->mmin; T.mmax = c->mmax;
   T.lmr = std::log(c->mmax / c->mmin);
   T.lkr = std::log(c->kmax / c->kmin);
+  T.rdz = 1. / (c->zmax - c->zmin);
+  T.rkmin = 1. / c->kmin;
+  T.rlkr = 1. / T.lkr;
+  T.rmmin = 1. / c->mmin;
+  T.rlmr = 1. / T.lmr;
+  T.rw = d + orw;
+  T.rrho = d + orr;
   T.g = d + og; T.p1 = d + op1; T.p2 = d + op2; T.w = d + ow; T.dwdz = d + odw;
   T.rho = d + orho; T.hmf = d + ohmf; T.plin = d + opl; T.bh = d + obh; T.conc = d + oc;
   *out = c;
@@ -945,6 +965,7 @@ int g3l_integrand(g3l_ctx *c, const g3l_request *r, int32_t precision, size_t np
     a.t1 = r->theta[0];
     const HodSet &s = c->sets[r->hodset];
     a.h1 = a.h2 = to_dev(r->type1 == 2 ? s.h2 : s.h1);
+    a.rs1 = a.rs2 = 1. / a.h1.sigma;
     fill_logs(c, a);
   } else {
     if ((rc = check_request(c, *r))) return rc;

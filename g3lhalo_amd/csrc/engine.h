@@ -140,7 +140,7 @@ struct g3l_ctx {
   double H0, Om, OL, rho_crit;
   double zmin_i, zmax_i, mmin_i, mmax_i;
   std::vector<double> rho;
-  DevBuf tables;     // g p1 p2 w dwdz rho | hmf plin(+nb) bh conc
+  DevBuf tables;     // 1/w 1/rho g p1 p2 w dwdz rho | hmf plin(+nb) bh conc
   g3l::DevTables T{};
   std::vector<HodSet> sets;
   // n_bar per HOD set, [set][2][nb], in chunks of kSetsPerChunk sets that

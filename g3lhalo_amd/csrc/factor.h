@@ -87,13 +87,44 @@ constexpr Proj<D, MASK> make_proj() {
   return p;
 }
 
-// Device copy of each table (constant memory, indexed per thread).
+// Number of classes, and the table itself on the host side.
 template <int D, unsigned MASK>
 struct ProjTab {
   static constexpr Proj<D, MASK> host = make_proj<D, MASK>();
   static constexpr int n = host.n;
 };
-template <int D, unsigned MASK>
-__constant__ constexpr Proj<D, MASK> kProj = make_proj<D, MASK>();
+// Packed per-class (or per-point) look-ups: one word from constant memory and
+// a few bit extracts instead of a byte load, with its address, per index.
+template <int N, class W = uint16_t>
+struct Packed {
+  W w[N] = {};
+};
+
+// Coordinate codes of the classes of (A, last dimension), then (B, last), then
+// (C, last): A's, B's or C's code in bits 0-2, the last dimension's in bits 4-6.
+template <int D, int A, int B, int C>
+constexpr Packed<3 * make_proj<D, bit(A) | bit(D - 1)>().n, uint8_t> make_codes() {
+  constexpr int n = make_proj<D, bit(A) | bit(D - 1)>().n;
+  Packed<3 * n, uint8_t> t{};
+  const Proj<D, bit(A) | bit(D - 1)> a = make_proj<D, bit(A) | bit(D - 1)>();
+  const Proj<D, bit(B) | bit(D - 1)> b = make_proj<D, bit(B) | bit(D - 1)>();
+  const Proj<D, bit(C) | bit(D - 1)> c = make_proj<D, bit(C) | bit(D - 1)>();
+  for (int i = 0; i < n; ++i) {
+    t.w[i] = (uint8_t)(gm_code(D, a.rep[i], A) | gm_code(D, a.rep[i], D - 1) << 4);
+    t.w[n + i] = (uint8_t)(gm_code(D, b.rep[i], B) | gm_code(D, b.rep[i], D - 1) << 4);
+    t.w[2 * n + i] = (uint8_t)(gm_code(D, c.rep[i], C) | gm_code(D, c.rep[i], D - 1) << 4);
+  }
+  return t;
+}
+// The code of class c of one dimension: the centre, then the axis points'
+// codes 1-4, then the last group's (all upper, 6, first).
+template <int D, int A>
+constexpr bool single_codes() {
+  constexpr Proj<D, bit(A)> p = make_proj<D, bit(A)>();
+  for (int c = 0; c < p.n; ++c)
+    if (gm_code(D, p.rep[c], A) != (c < 5 ? c : 11 - c)) return false;
+  return p.n == 7;
+}
+constexpr __host__ __device__ int single_code(int c) { return c < 5 ? c : 11 - c; }
 
 }  // namespace g3l

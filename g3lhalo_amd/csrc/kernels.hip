@@ -258,6 +258,101 @@ struct Cache {
   double bl[G * NB];
 };
 
+// Class indices of every point in one 16-byte load; a byte load with its address
+// arithmetic per index, and a region's points rebuilt by rule_point for every
+// class, were a fifth of a point's instructions.  Packed look-ups, coordinates
+// by code and quotients by known reciprocals (DevTables) together took the
+// evaluation of the 550-triplet workload from 281 to 254 ms, values
+// bit-identical.  Word 0 l1, l2, z (3 bits each), l3 (6),
+// the masses' (5 each); word 1 (l1, z), (l2, z) (5 each), (l1, l2, phi, z) (7)
+// and u factors 0 and 1 (7 each); word 2 u factors 2 to 5 (7 each).
+struct PointWords {
+  uint32_t w0, w1, w2, pad;
+};
+template <int KIND>
+constexpr Packed<rule_points(Spec<kind_of_kv(KIND)>::D), PointWords> make_points() {
+  using S = Spec<kind_of_kv(KIND)>;
+  constexpr int D = S::D;
+  constexpr unsigned z = bit(D - 1);
+  constexpr auto l1 = make_proj<D, kL1>();
+  constexpr auto l2 = make_proj<D, kL2>();
+  constexpr auto pz = make_proj<D, z>();
+  constexpr auto l3 = make_proj<D, kL3>();
+  constexpr auto m0 = make_proj<D, bit(S::mdim[0]) | z>();
+  constexpr auto m1 = make_proj<D, bit(S::mdim[S::NM > 1 ? 1 : 0]) | z>();
+  constexpr auto m2 = make_proj<D, bit(S::mdim[S::NM > 2 ? 2 : 0]) | z>();
+  constexpr auto l1z = make_proj<D, kL1 | z>();
+  constexpr auto l2z = make_proj<D, kL2 | z>();
+  constexpr auto l3z = make_proj<D, kL3 | z>();
+  constexpr auto u0 = make_proj<D, S::u[0].mask>();
+  constexpr auto u1 = make_proj<D, S::u[1].mask>();
+  constexpr auto u2 = make_proj<D, S::u[2].mask>();
+  constexpr auto u3 = make_proj<D, S::u[S::NU > 3 ? 3 : 0].mask>();
+  constexpr auto u4 = make_proj<D, S::u[S::NU > 4 ? 4 : 0].mask>();
+  constexpr auto u5 = make_proj<D, S::u[S::NU > 5 ? 5 : 0].mask>();
+  static_assert(l3.n <= 64 && l3z.n <= 128 && u0.n <= 128 && u1.n <= 128 && u2.n <= 128 &&
+                u3.n <= 128 && u4.n <= 128 && u5.n <= 128 && m0.n <= 32, "field widths");
+  Packed<rule_points(D), PointWords> t{};
+  for (int q = 0; q < rule_points(D); ++q) {
+    t.w[q].w0 = l1.cls[q] | l2.cls[q] << 3 | pz.cls[q] << 6 | l3.cls[q] << 9 | m0.cls[q] << 15 |
+                m1.cls[q] << 20 | (uint32_t)m2.cls[q] << 25;
+    t.w[q].w1 = l1z.cls[q] | l2z.cls[q] << 5 | l3z.cls[q] << 10 | u0.cls[q] << 17 |
+                (uint32_t)u1.cls[q] << 24;
+    t.w[q].w2 = u2.cls[q] | u3.cls[q] << 7 | u4.cls[q] << 14 | (uint32_t)u5.cls[q] << 21;
+  }
+  return t;
+}
+template <int KIND>
+__constant__ constexpr auto kPoints = make_points<kind_of_kv(KIND)>();
+
+// Per class of a u factor: its l (6 bits), z (3) and mass (5) classes.
+template <int KIND, int I>
+constexpr auto make_u_words() {
+  using S = Spec<KIND>;
+  constexpr int D = S::D;
+  constexpr USpec s = S::u[I];
+  constexpr auto p = make_proj<D, s.mask>();
+  constexpr auto l = make_proj<D, s.kidx == 1 ? kL1 : s.kidx == 2 ? kL2 : kL3>();
+  constexpr auto pz = make_proj<D, bit(D - 1)>();
+  constexpr auto pm = make_proj<D, bit(S::mdim[s.slot]) | bit(D - 1)>();
+  Packed<p.n> t{};
+  for (int c = 0; c < p.n; ++c)
+    t.w[c] = (uint16_t)(l.cls[p.rep[c]] | pz.cls[p.rep[c]] << 6 | pm.cls[p.rep[c]] << 9);
+  return t;
+}
+template <int KIND, int I>
+__constant__ constexpr auto kUWords = make_u_words<KIND, I>();
+
+// Per (l1, l2, phi) or (l1, l2, phi, z) class: the classes of l1, l2, phi, z
+// (3 bits each), and for the latter of l3 (6 bits).
+template <int D, unsigned MASK>
+constexpr auto make_geo_words() {
+  constexpr auto p = make_proj<D, MASK>();
+  constexpr auto l1 = make_proj<D, kL1>();
+  constexpr auto l2 = make_proj<D, kL2>();
+  constexpr auto ph = make_proj<D, bit(2)>();
+  constexpr auto pz = make_proj<D, bit(D - 1)>();
+  constexpr auto l3 = make_proj<D, kL3>();
+  Packed<p.n, uint32_t> t{};
+  for (int c = 0; c < p.n; ++c) {
+    const int q = p.rep[c];
+    t.w[c] = l1.cls[q] | l2.cls[q] << 3 | ph.cls[q] << 6 | pz.cls[q] << 9 | l3.cls[q] << 12;
+  }
+  return t;
+}
+template <int D, unsigned MASK>
+__constant__ constexpr auto kGeoWords = make_geo_words<D, MASK>();
+// Codes of the (mass, z) classes by mass slot, and of the (l1, z), (l2, z) ones.
+template <int KIND>
+__constant__ constexpr auto kMassCodes =
+    make_codes<Spec<KIND>::D, Spec<KIND>::mdim[0], Spec<KIND>::mdim[Spec<KIND>::NM > 1 ? 1 : 0],
+               Spec<KIND>::mdim[Spec<KIND>::NM > 2 ? 2 : 0]>();
+template <int D>
+__constant__ constexpr auto kLCodes = make_codes<D, 0, 1, 1>();
+__device__ __forceinline__ uint32_t bits(uint32_t w, int at, int n) {
+  return (w >> at) & ((1u << n) - 1u);
+}
+
 // Per-point view of the cache (the value source of the integrands).
 template <int KIND, class P>
 struct CachedSrc {
@@ -265,28 +360,23 @@ struct CachedSrc {
   static constexpr int D = S::D, G = KGroup<KIND>::G;
   const Cache<KIND> &C;
   const TermArgs &a;
-  int g, q;
+  int g;
+  PointWords pw;
   Geo G_;
-  __device__ __forceinline__ CachedSrc(const Cache<KIND> &C_, const TermArgs &a_, int g_, int q_)
-      : C(C_), a(a_), g(g_), q(q_) {
-    const int c1 = kProj<D, kL1>.cls[q], c2 = kProj<D, kL2>.cls[q];
-    const int cp = kProj<D, bit(2)>.cls[q], cz = kProj<D, bit(D - 1)>.cls[q];
-    G_.l1 = C.l1[g][c1];
-    G_.l2 = C.l2[g][c2];
-    G_.cphi = C.cphi[g][cp];
-    G_.z = C.z[g][cz];
-    G_.zr = C.zr[g][cz];
-    G_.zt = C.zt[g][cz];
-    G_.w = C.w[g][cz];
-    G_.l3 = C.l3[g][kProj<D, kL3>.cls[q]];
-    G_.k1 = G_.l1 / G_.w;
-    G_.k2 = G_.l2 / G_.w;
-    G_.k3 = G_.l3 / G_.w;
+  __device__ __forceinline__ CachedSrc(const Cache<KIND> &C_, const TermArgs &a_, int g_, int q)
+      : C(C_), a(a_), g(g_), pw(kPoints<kind_of_kv(KIND)>.w[q]) {
+    G_ = Geo{};
+    G_.l1 = C.l1[g][c1()];
+    G_.l2 = C.l2[g][c2()];
+    G_.zr = C.zr[g][cz()];
   }
+  __device__ __forceinline__ uint32_t c1() const { return bits(pw.w0, 0, 3); }
+  __device__ __forceinline__ uint32_t c2() const { return bits(pw.w0, 3, 3); }
+  __device__ __forceinline__ uint32_t cz() const { return bits(pw.w0, 6, 3); }
   __device__ __forceinline__ const MassC &mc(int i) const {
-    if (i == 0) return C.m[0][g][kProj<D, bit(S::mdim[0]) | bit(D - 1)>.cls[q]];
-    if (S::NM > 1 && i == 1) return C.m[S::NM > 1 ? 1 : 0][g][kProj<D, bit(S::mdim[1]) | bit(D - 1)>.cls[q]];
-    return C.m[S::NM > 2 ? 2 : 0][g][kProj<D, bit(S::mdim[2]) | bit(D - 1)>.cls[q]];
+    if (i == 0) return C.m[0][g][bits(pw.w0, 15, 5)];
+    if (S::NM > 1 && i == 1) return C.m[S::NM > 1 ? 1 : 0][g][bits(pw.w0, 20, 5)];
+    return C.m[S::NM > 2 ? 2 : 0][g][bits(pw.w0, 25, 5)];
   }
   __device__ __forceinline__ const Geo &geo() const { return G_; }
   __device__ __forceinline__ Mass mass(int i) const {
@@ -308,44 +398,34 @@ struct CachedSrc {
     return Occ{e.nc2, e.ns2};
   }
   __device__ __forceinline__ double nss(int i) const { return mc(i).nss; }
-  __device__ __forceinline__ Nfw nfw(int i, int fsel) const {
-    static_assert(cache_nfw<KIND>(), "per-point u_NFW normalisations come from the cache");
-    const int cls = i == 0   ? kProj<D, bit(S::mdim[0]) | bit(D - 1)>.cls[q]
-                    : i == 1 ? kProj<D, bit(S::mdim[S::NM > 1 ? 1 : 0]) | bit(D - 1)>.cls[q]
-                             : kProj<D, bit(S::mdim[S::NM > 2 ? 2 : 0]) | bit(D - 1)>.cls[q];
-    const NfwC &e = C.nf[i][g][cls];
-    return Nfw{mc(i).r200, e.c[fsel], e.lc[fsel], e.F[fsel]};
-  }
   template <int I>
   __device__ __forceinline__ double u() const {
     using F = UF<KIND, I>;
-    return C.u[UOff<KIND, I>::v + g * F::n + kProj<D, F::s.mask>.cls[q]];
+    const uint32_t c = I == 0   ? bits(pw.w1, 17, 7)
+                       : I == 1 ? bits(pw.w1, 24, 7)
+                                : bits(pw.w2, I < 2 ? 0 : 7 * (I - 2), 7);
+    return C.u[UOff<KIND, I>::v + g * F::n + c];
   }
-  __device__ __forceinline__ double ap1() const { return C.ap1[g][kProj<D, kL1>.cls[q]]; }
-  __device__ __forceinline__ double ap2() const { return C.ap2[g][kProj<D, kL2>.cls[q]]; }
+  __device__ __forceinline__ double ap1() const { return C.ap1[g][c1()]; }
+  __device__ __forceinline__ double ap2() const { return C.ap2[g][c2()]; }
   __device__ __forceinline__ double bl() const {
-    return C.bl[g * Cache<KIND>::NB + kProj<D, bilin_mask<D>()>.cls[q]];
+    return C.bl[g * Cache<KIND>::NB + bits(pw.w1, 10, 7)];
   }
-  __device__ __forceinline__ double ap3() const { return C.ap3[g][kProj<D, kL3>.cls[q]]; }
+  __device__ __forceinline__ double ap3() const { return C.ap3[g][bits(pw.w0, 9, 6)]; }
   __device__ __forceinline__ double pk3() const {
-    return C.pk3[S::has_pk ? g : 0][kProj<D, kL3 | bit(D - 1)>.cls[q]];
+    return C.pk3[S::has_pk ? g : 0][bits(pw.w1, 10, 7)];
   }
-  __device__ __forceinline__ double pk1() const {
-    return C.pk[0][g][kProj<D, kL1 | bit(D - 1)>.cls[q]];
-  }
+  __device__ __forceinline__ double pk1() const { return C.pk[0][g][bits(pw.w1, 0, 5)]; }
   __device__ __forceinline__ double pk2() const {
-    return C.pk[S::has_pk ? 1 : 0][g][kProj<D, kL2 | bit(D - 1)>.cls[q]];
+    return C.pk[S::has_pk ? 1 : 0][g][bits(pw.w1, 5, 5)];
   }
-  __device__ __forceinline__ double zpre() const {
-    return C.zpre[g][kProj<D, bit(D - 1)>.cls[q]];
-  }
+  __device__ __forceinline__ double zpre() const { return C.zpre[g][cz()]; }
   __device__ __forceinline__ double proj(double B) const {
-    const int cz = kProj<D, bit(D - 1)>.cls[q];
     if constexpr (kind_of_kv(KIND) == kNN3) {
-      const double *t = C.ztab[g][cz];
-      return proj_3h(B, t[0], t[1], t[2], t[3], t[4], C.w[g][cz], t[5], C.z[g][cz]);
+      const double *t = C.ztab[g][cz()];
+      return proj_3h(B, t[0], t[1], t[2], t[3], t[4], C.w[g][cz()], t[5], C.z[g][cz()]);
     } else {
-      return C.zfac[g][cz] * B;
+      return C.zfac[g][cz()] * B;
     }
   }
 };
@@ -372,7 +452,8 @@ __device__ __forceinline__ void pass1(const DevTables &T, const Stage<Spec<kind_
   using S = Spec<kind_of_kv(KIND)>;
   using Lay = P1Layout<KIND>;
   constexpr int D = S::D, G = KGroup<KIND>::G;
-  double x[D];
+  static_assert(single_codes<D, 0>() && single_codes<D, 1>() && single_codes<D, 2>() &&
+                    single_codes<D, D - 1>(), "coordinate codes by class");
   if (i < Lay::PHI) {
     const int r = i - Lay::L;
     if (r >= 2 * G * 7) return;
@@ -380,8 +461,7 @@ __device__ __forceinline__ void pass1(const DevTables &T, const Stage<Spec<kind_
     if (g >= ng || St.slot[g] == 0xffffffffu) return;
     const TermArgs &a = St.args[g];
     // l1 and l2 items share one wave: one code path with selected operands
-    rule_point<D>(which == 0 ? kProj<D, kL1>.rep[c] : kProj<D, kL2>.rep[c], St.c[g], St.h[g], x);
-    const double l = P::l(which == 0 ? x[0] : x[1]);
+    const double l = P::l(rule_coord(single_code(c), St.c[g][which], St.h[g][which]));
     const double ap = P::ap((which == 0 ? a.t1 : a.t2) * l);
     if (which == 0) {
       C.l1[g][c] = l;
@@ -395,22 +475,20 @@ __device__ __forceinline__ void pass1(const DevTables &T, const Stage<Spec<kind_
     if (r >= G * 7) return;
     const int g = r / 7, c = r - g * 7;
     if (g >= ng || St.slot[g] == 0xffffffffu) return;
-    rule_point<D>(kProj<D, bit(2)>.rep[c], St.c[g], St.h[g], x);
-    C.cphi[g][c] = cos(x[2]);
+    C.cphi[g][c] = cos(rule_coord(single_code(c), St.c[g][2], St.h[g][2]));
   } else if (i < Lay::MZ) {
     const int r = i - Lay::Z;
     if (r >= G * 7) return;
     const int g = r / 7, c = r - g * 7;
     if (g >= ng || St.slot[g] == 0xffffffffu) return;
-    rule_point<D>(kProj<D, bit(D - 1)>.rep[c], St.c[g], St.h[g], x);
-    const double z = x[D - 1];
+    const double z = rule_coord(single_code(c), St.c[g][D - 1], St.h[g][D - 1]);
     const int zr = zix_round(T, z);
     const double w = T.w[zr];
     C.z[g][c] = z;
     C.zr[g][c] = zr;
     C.zt[g][c] = zix_trunc(T, z);
     C.w[g][c] = w;
-    C.rw[g][c] = 1. / w;
+    C.rw[g][c] = T.rw[zr];
     zfactors<kind_of_kv(KIND)>(T, St.args[g], zr, z, w, C.zpre[g][c], C.zfac[g][c]);
     if constexpr (kind_of_kv(KIND) == kNN3) {
       double *t = C.ztab[g][c];
@@ -419,7 +497,7 @@ __device__ __forceinline__ void pass1(const DevTables &T, const Stage<Spec<kind_
       t[2] = T.g[zr];
       t[3] = T.p1[zr];
       t[4] = T.p2[zr];
-      t[5] = 1. / w;
+      t[5] = T.rw[zr];
     }
   } else if (i < Lay::PK) {
     const int r = i - Lay::MZ;
@@ -428,13 +506,9 @@ __device__ __forceinline__ void pass1(const DevTables &T, const Stage<Spec<kind_
     if (g >= ng || St.slot[g] == 0xffffffffu) return;
     const TermArgs &a = St.args[g];
     const int md = slot == 0 ? S::mdim[0] : slot == 1 ? S::mdim[1] : S::mdim[2];
-    int rep;
-    if (slot == 0) rep = kProj<D, bit(S::mdim[0]) | bit(D - 1)>.rep[c];
-    else if (slot == 1) rep = kProj<D, bit(S::mdim[S::NM > 1 ? 1 : 0]) | bit(D - 1)>.rep[c];
-    else rep = kProj<D, bit(S::mdim[S::NM > 2 ? 2 : 0]) | bit(D - 1)>.rep[c];
-    rule_point<D>(rep, St.c[g], St.h[g], x);
-    const int zt = zix_trunc(T, x[D - 1]);
-    const Mass M = make_mass<P>(T, x[md], zt);
+    const uint32_t code = kMassCodes<kind_of_kv(KIND)>.w[slot * 17 + c];
+    const int zt = zix_trunc(T, rule_coord(code >> 4, St.c[g][D - 1], St.h[g][D - 1]));
+    const Mass M = make_mass<P>(T, rule_coord(code & 7, St.c[g][md], St.h[g][md]), zt);
     MassC &e = C.m[slot][g][c];
     e.m = M.m;
     e.L = M.L;
@@ -447,8 +521,8 @@ __device__ __forceinline__ void pass1(const DevTables &T, const Stage<Spec<kind_
       // the NNMap 3-halo term needs the first HOD at m1 and the second at m2
       // only: one occupation per item, the HOD selected by the mass slot
       const bool second = slot == 1;
-      const Occ o = P::occ(second ? a.h2 : a.h1, second ? a.lth2 : a.lth1,
-                           second ? a.lmp2 : a.lmp1, M);
+      const Occ o = P::occ(second ? a.h2 : a.h1, second ? a.rs2 : a.rs1,
+                           second ? a.lth2 : a.lth1, second ? a.lmp2 : a.lmp1, M);
       e.nc1 = e.nc2 = o.nc;
       e.ns1 = e.ns2 = o.ns;
     } else {
@@ -482,11 +556,10 @@ __device__ __forceinline__ void pass1(const DevTables &T, const Stage<Spec<kind_
     const int which = r / (G * 17), rr = r - which * G * 17, g = rr / 17, c = rr - g * 17;
     if (g >= ng || St.slot[g] == 0xffffffffu) return;
     // P(k) at k = l / w, the same expressions as the per-point Geo
-    rule_point<D>(which == 0 ? kProj<D, kL1 | bit(D - 1)>.rep[c] : kProj<D, kL2 | bit(D - 1)>.rep[c],
-                  St.c[g], St.h[g], x);
-    const double l = P::l(x[which]);
-    const int zr = zix_round(T, x[D - 1]);
-    C.pk[which][g][c] = pk(T, zr, l / T.w[zr]);
+    const uint32_t code = kLCodes<D>.w[which * 17 + c];
+    const double l = P::l(rule_coord(code & 7, St.c[g][which], St.h[g][which]));
+    const int zr = zix_round(T, rule_coord(code >> 4, St.c[g][D - 1], St.h[g][D - 1]));
+    C.pk[which][g][c] = pk(T, zr, div_rn(l, T.w[zr], T.rw[zr]));
   }
 }
 
@@ -566,9 +639,9 @@ __device__ __forceinline__ void pass1b(const DevTables &T, const Stage<Spec<kind
   if (r >= G * N3) return;
   const int g = r / N3, c = r - g * N3;
   if (g >= ng || St.slot[g] == 0xffffffffu) return;
-  const int q = kProj<D, kL3>.rep[c];
-  const double l1 = C.l1[g][kProj<D, kL1>.cls[q]], l2 = C.l2[g][kProj<D, kL2>.cls[q]];
-  const double l3 = sqrt(l1 * l1 + l2 * l2 + 2 * l1 * l2 * C.cphi[g][kProj<D, bit(2)>.cls[q]]);
+  const uint32_t gw = kGeoWords<D, kL3>.w[c];
+  const double l1 = C.l1[g][bits(gw, 0, 3)], l2 = C.l2[g][bits(gw, 3, 3)];
+  const double l3 = sqrt(l1 * l1 + l2 * l2 + 2 * l1 * l2 * C.cphi[g][bits(gw, 6, 3)]);
   C.l3[g][c] = l3;
   C.ap3[g][c] = P::ap(St.args[g].t3 * l3);
 }
@@ -589,23 +662,22 @@ __device__ __forceinline__ bool u_inputs(const DevTables &T,
     if (i >= hi) return u_inputs<KIND, P, I + 1>(T, St, C, i, ng, dst, n, k, nfe);
     const int r = i - lo, g = r / F::n, c = r - g * F::n;
     if (g >= ng || St.slot[g] == 0xffffffffu) return false;
-    const int q = kProj<D, F::s.mask>.rep[c];
-    const int cz = kProj<D, bit(D - 1)>.cls[q];
+    const uint32_t uw = kUWords<kind_of_kv(KIND), I>.w[c];
+    const uint32_t cl = bits(uw, 0, 6), cz = bits(uw, 6, 3), cm = bits(uw, 9, 5);
     const double w = C.w[g][cz];
     double l;
     if constexpr (F::s.kidx == 1) {
-      l = C.l1[g][kProj<D, kL1>.cls[q]];
+      l = C.l1[g][cl];
     } else if constexpr (F::s.kidx == 2) {
-      l = C.l2[g][kProj<D, kL2>.cls[q]];
+      l = C.l2[g][cl];
     } else if constexpr (staged_p1<KIND>()) {
-      l = C.l3[g][kProj<D, kL3>.cls[q]];   // from pass 1, the same expression
+      l = C.l3[g][cl];   // from pass 1, the same expression
     } else {
-      const double l1 = C.l1[g][kProj<D, kL1>.cls[q]], l2 = C.l2[g][kProj<D, kL2>.cls[q]];
-      const double cp = C.cphi[g][kProj<D, bit(2)>.cls[q]];
-      l = sqrt(l1 * l1 + l2 * l2 + 2 * l1 * l2 * cp);
+      const uint32_t gw = kGeoWords<D, kL3>.w[cl];
+      const double l1 = C.l1[g][bits(gw, 0, 3)], l2 = C.l2[g][bits(gw, 3, 3)];
+      l = sqrt(l1 * l1 + l2 * l2 + 2 * l1 * l2 * C.cphi[g][bits(gw, 6, 3)]);
     }
     k = div_rn(l, w, C.rw[g][cz]);   // = l / w (IEEE), in three instructions
-    const int cm = kProj<D, bit(S::mdim[F::s.slot]) | bit(D - 1)>.cls[q];
     const MassC &e = C.m[F::s.slot][g][cm];
     if constexpr (cache_nfw<KIND>()) {
       const NfwC &en = C.nf[F::s.slot][g][cm];
@@ -671,11 +743,12 @@ __device__ __forceinline__ void pass2_rest(const DevTables &T, const Stage<Spec<
       if (r < 0 || r >= G * NB) return;
       const int g = r / NB, c = r - g * NB;
       if (g >= ng || St.slot[g] == 0xffffffffu) return;
-      const int q = kProj<D, bilin_mask<D>()>.rep[c];
-      const int cz = kProj<D, bit(D - 1)>.cls[q];
-      const double w = C.w[g][cz];
-      const double k1 = C.l1[g][kProj<D, kL1>.cls[q]] / w, k2 = C.l2[g][kProj<D, kL2>.cls[q]] / w;
-      C.bl[r] = bilin(T, k1, k2, C.cphi[g][kProj<D, bit(2)>.cls[q]], C.z[g][cz]);
+      const uint32_t gw = kGeoWords<D, bilin_mask<D>()>.w[c];
+      const uint32_t cz = bits(gw, 9, 3);
+      const double w = C.w[g][cz], rw = C.rw[g][cz];
+      const double k1 = div_rn(C.l1[g][bits(gw, 0, 3)], w, rw);
+      const double k2 = div_rn(C.l2[g][bits(gw, 3, 3)], w, rw);
+      C.bl[r] = bilin(T, k1, k2, C.cphi[g][bits(gw, 6, 3)], C.z[g][cz]);
     }
     return;
   }
@@ -686,9 +759,9 @@ __device__ __forceinline__ void pass2_rest(const DevTables &T, const Stage<Spec<
     if (r >= G * N3) return;
     const int g = r / N3, c = r - g * N3;
     if (g >= ng || St.slot[g] == 0xffffffffu) return;
-    const int q = kProj<D, kL3>.rep[c];
-    const double l1 = C.l1[g][kProj<D, kL1>.cls[q]], l2 = C.l2[g][kProj<D, kL2>.cls[q]];
-    const double l3 = sqrt(l1 * l1 + l2 * l2 + 2 * l1 * l2 * C.cphi[g][kProj<D, bit(2)>.cls[q]]);
+    const uint32_t gw = kGeoWords<D, kL3>.w[c];
+    const double l1 = C.l1[g][bits(gw, 0, 3)], l2 = C.l2[g][bits(gw, 3, 3)];
+    const double l3 = sqrt(l1 * l1 + l2 * l2 + 2 * l1 * l2 * C.cphi[g][bits(gw, 6, 3)]);
     C.l3[g][c] = l3;
     C.ap3[g][c] = P::ap(St.args[g].t3 * l3);
     return;
@@ -700,16 +773,16 @@ __device__ __forceinline__ void pass2_rest(const DevTables &T, const Stage<Spec<
     if (r >= G * N3Z) return;
     const int g = r / N3Z, c = r - g * N3Z;
     if (g >= ng || St.slot[g] == 0xffffffffu) return;
-    const int q = kProj<D, kL3 | bit(D - 1)>.rep[c];
-    const int cz = kProj<D, bit(D - 1)>.cls[q];
+    const uint32_t gw = kGeoWords<D, kL3 | bit(D - 1)>.w[c];
+    const uint32_t cz = bits(gw, 9, 3);
     double l3;
     if constexpr (staged_p1<KIND>()) {
-      l3 = C.l3[g][kProj<D, kL3>.cls[q]];
+      l3 = C.l3[g][bits(gw, 12, 6)];
     } else {
-      const double l1 = C.l1[g][kProj<D, kL1>.cls[q]], l2 = C.l2[g][kProj<D, kL2>.cls[q]];
-      l3 = sqrt(l1 * l1 + l2 * l2 + 2 * l1 * l2 * C.cphi[g][kProj<D, bit(2)>.cls[q]]);
+      const double l1 = C.l1[g][bits(gw, 0, 3)], l2 = C.l2[g][bits(gw, 3, 3)];
+      l3 = sqrt(l1 * l1 + l2 * l2 + 2 * l1 * l2 * C.cphi[g][bits(gw, 6, 3)]);
     }
-    C.pk3[g][c] = pk(T, C.zr[g][cz], l3 / C.w[g][cz]);
+    C.pk3[g][c] = pk(T, C.zr[g][cz], div_rn(l3, C.w[g][cz], C.rw[g][cz]));
   }
 }
 

@@ -16,6 +16,7 @@ namespace g3l {
 // scale * value in out[i].
 struct OneDimGroup {
   DevHod h;              // kOneDNbar
+  double rs;             // 1 / h.sigma
   double lo, hi;
   double *out;
   const double *aux;     // PrecompParams of the other modes

@@ -132,6 +132,7 @@ __device__ __noinline__ void one_dim_node(const DevTables &T, const OneDimGroup 
   if constexpr (!PRE) {
     TermArgs a{};
     a.h1 = g.h;
+    a.rs1 = g.rs;
     const Mass M = make_mass<P64R>(T, x, 0);
     const Occ o = occ1<P64R>(a, M);
     ab = double2{M.m, o.nc + o.ns};

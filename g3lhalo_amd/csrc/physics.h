@@ -187,13 +187,27 @@ G3L_HD void sincos_mm(double x, double &s, double &c) {
   sincos_select(q, fma(r * z, ps, r), fma(pc, z, 1.0), s, c);
 }
 
+// a / d correctly rounded from rd = RN(1/d): q = RN(a rd), then one FMA
+// residual correction (Markstein's theorem: with rd the correctly rounded
+// reciprocal the corrected quotient is RN(a / d) for normal operands, no
+// overflow or underflow).  Three instructions instead of the IEEE division
+// sequence, for divisors that repeat over many points.
+G3L_HD double div_rn(double a, double d, double rd) {
+  const double q = a * rd;
+  return fma(fma(-d, q, a), rd, q);
+}
+
 // Tables resident in HBM (z-major 2-D tables, nb*nb + nb for P_lin).
 struct DevTables {
   int nb;
   double zmin, zmax, kmin, kmax, mmin, mmax;
   double lmr;    // log(mmax / mmin), computed on the host
   double lkr;    // log(kmax / kmin), computed on the host
-  const double *g, *p1, *p2, *w, *dwdz, *hmf, *plin, *bh, *conc, *rho;
+  // correctly rounded reciprocals of zmax - zmin, kmin, lkr, mmin and lmr, and
+  // tables of those of w and rho: every quotient by one of them is the IEEE
+  // quotient in three instructions (div_rn) instead of about twelve
+  double rdz, rkmin, rlkr, rmmin, rlmr;
+  const double *g, *p1, *p2, *w, *dwdz, *hmf, *plin, *bh, *conc, *rho, *rw, *rrho;
 };
 
 struct DevHod {
@@ -207,6 +221,8 @@ struct TermArgs {
   const double *nb1, *nb2;  // n_bar selected by type (NMapMap: nb1)
   double A, eps;
   int same;                 // NsatNsat same-type branch
+  // 1 / sigma of the two HODs, correctly rounded
+  double rs1, rs2;
   // log-space HOD constants of PMix: log(mmin/M_th), log(mmin/M'), log(mmin)
   double lth1, lmp1, lth2, lmp2, lmmin;
 };
@@ -291,18 +307,18 @@ G3L_HD double precomp_amplitude(const PrecompParams &p, double x, double R) {
 // outside the tables.
 G3L_HD int clampi(int i, int hi) { return i < 0 ? 0 : (i > hi ? hi : i); }
 G3L_HD int zix_round(const DevTables &T, double z) {
-  return clampi((int)round((z - T.zmin) * T.nb / (T.zmax - T.zmin)), T.nb - 1);
+  return clampi((int)round(div_rn((z - T.zmin) * T.nb, T.zmax - T.zmin, T.rdz)), T.nb - 1);
 }
 G3L_HD int zix_trunc(const DevTables &T, double z) {
-  return clampi((int)((z - T.zmin) * T.nb / (T.zmax - T.zmin)), T.nb - 1);
+  return clampi((int)div_rn((z - T.zmin) * T.nb, T.zmax - T.zmin, T.rdz), T.nb - 1);
 }
-// Held in [-1, nb^2 + nb] before the conversion: an infinite k (a zero
-// comoving distance) would otherwise convert out of int's range, and
-// zi * nb + ki could overflow.  Every finite k in that range keeps its
-// index; beyond it the row-spill read lands past the padded table either
-// way and pk's clamp gives the same entry.  NaN maps to 0.
+// Held in [-1, nb^2 + nb] before the conversion: a huge k would otherwise
+// convert out of int's range, and zi * nb + ki could overflow.  Every finite k
+// in that range keeps its index; beyond it the row-spill read lands past the
+// padded table either way and pk's clamp gives the same entry.  NaN, and an
+// infinite k (a zero comoving distance, whose u_NFW is NaN), map to 0.
 G3L_HD int kix_round(const DevTables &T, double k) {
-  const double x = round(log(k / T.kmin) * T.nb / T.lkr);
+  const double x = round(div_rn(log(div_rn(k, T.kmin, T.rkmin)) * T.nb, T.lkr, T.rlkr));
   const double top = (double)T.nb * T.nb + T.nb;
   return x >= 0 ? (int)fmin(x, top) : (x < 0 ? (int)fmax(x, -1.0) : 0);
 }
@@ -312,7 +328,7 @@ G3L_HD int kix_round(const DevTables &T, double k) {
 G3L_HD double pk(const DevTables &T, int zi, double k) {
   int ki = kix_round(T, k);
   if (ki >= 0) return T.plin[clampi(zi * T.nb + ki, T.nb * T.nb + T.nb - 1)];
-  return T.plin[zi * T.nb] / T.kmin * k;
+  return div_rn(T.plin[zi * T.nb], T.kmin, T.rkmin) * k;
 }
 
 // One halo mass at one redshift: m = 10^x with the reference's rounding, its
@@ -326,10 +342,11 @@ template <class P>
 G3L_HD Mass make_mass(const DevTables &T, double x, int zt) {
   Mass M;
   M.m = pow(10.0, x);
-  M.L = log(M.m / T.mmin);
-  M.ir = clampi((int)round(M.L * T.nb / T.lmr), T.nb - 1);
-  M.it = clampi((int)(M.L * T.nb / T.lmr), T.nb - 1);
-  M.r200 = P::cbrt3(0.239 * M.m / T.rho[zt] / 200);
+  M.L = log(div_rn(M.m, T.mmin, T.rmmin));
+  const double ix = div_rn(M.L * T.nb, T.lmr, T.rlmr);
+  M.ir = clampi((int)round(ix), T.nb - 1);
+  M.it = clampi((int)ix, T.nb - 1);
+  M.r200 = P::cbrt3(div_rn(div_rn(0.239 * M.m, T.rho[zt], T.rrho[zt]), 200.0, 1.0 / 200.0));
   return M;
 }
 
@@ -697,6 +714,11 @@ G3L_HD double u_nfw(const Nfw &n, double k) {
   return u_nfw_a1<P>(nfw_a1(n, k), n);
 }
 
+// x / sigma / 1.414213562, rs = RN(1 / sigma).
+G3L_HD double over_sigma(double x, double sigma, double rs) {
+  return div_rn(div_rn(x, sigma, rs), 1.414213562, 1.0 / 1.414213562);
+}
+
 // FP64 policy
 struct P64 {
   static constexpr bool kMixed = false;
@@ -707,8 +729,8 @@ struct P64 {
   // Ncen and Nsat share log(m/M_th)/sigma/sqrt2 and its erf (src/HOD.cu:35-76);
   // the logarithms come from L = log(m/mmin): log(m/M_th) = L + log(mmin/M_th),
   // (m/M')^beta = exp(beta (L + log(mmin/M'))).
-  G3L_HD static Occ occ(const DevHod &h, double lth, double lmp, const Mass &M) {
-    double e = 1 + erf((M.L + lth) / h.sigma / 1.414213562);
+  G3L_HD static Occ occ(const DevHod &h, double rs, double lth, double lmp, const Mass &M) {
+    double e = 1 + erf(over_sigma(M.L + lth, h.sigma, rs));
     Occ o;
     o.nc = 0.5 * h.alpha * e;
     o.ns = 0.5 * e * exp(h.beta * (M.L + lmp));
@@ -750,10 +772,10 @@ struct P64R : P64 {
   // (src/NNMap_Model.cu:986-991, src/generalFunctions.cu:36)
   G3L_HD static double l(double x) { return pow(10.0, x); }
   G3L_HD static double cbrt3(double x) { return pow(x, 1. / 3.); }
-  G3L_HD static Occ occ(const DevHod &h, double lth, double lmp, const Mass &M) {
+  G3L_HD static Occ occ(const DevHod &h, double rs, double lth, double lmp, const Mass &M) {
     (void)lth;
     (void)lmp;
-    double e = 1 + erf(log(M.m / h.mth) / h.sigma / 1.414213562);
+    double e = 1 + erf(over_sigma(log(M.m / h.mth), h.sigma, rs));
     Occ o;
     o.nc = 0.5 * h.alpha * e;
     o.ns = 0.5 * e * pow(M.m / h.mprime, h.beta);
@@ -869,8 +891,8 @@ struct PMix {
   // exponentials and erf, as P64): they are evaluated once per (mass,
   // redshift) class of a region, so FP32 would save little, and their FP32
   // rounding moved whole integrals of this precision form by up to 2e-3.
-  G3L_HD static Occ occ(const DevHod &h, double lth, double lmp, const Mass &M) {
-    return P64::occ(h, lth, lmp, M);
+  G3L_HD static Occ occ(const DevHod &h, double rs, double lth, double lmp, const Mass &M) {
+    return P64::occ(h, rs, lth, lmp, M);
   }
   G3L_HD static double mpow(const Mass &M, double eps, double lmmin) {
     return P64::mpow(M, eps, lmmin);
@@ -924,11 +946,11 @@ struct PMix {
 
 template <class P>
 G3L_HD Occ occ1(const TermArgs &a, const Mass &M) {
-  return P::occ(a.h1, a.lth1, a.lmp1, M);
+  return P::occ(a.h1, a.rs1, a.lth1, a.lmp1, M);
 }
 template <class P>
 G3L_HD Occ occ2(const TermArgs &a, const Mass &M) {
-  return P::occ(a.h2, a.lth2, a.lmp2, M);
+  return P::occ(a.h2, a.rs2, a.lth2, a.lmp2, M);
 }
 
 // src/HOD.cu:78-94 with scale1 = scale2 = 1.
@@ -942,7 +964,9 @@ G3L_HD double nsatnsat(const TermArgs &a, double ns1, double ns2,
 
 // F kernel with the reference's k2/k2 (src/generalFunctions.cu:89-92).
 G3L_HD double fkern(double k1, double k2, double c) {
-  return 0.7143 + 0.2857 * c * c + 0.5 * c * (k1 / k2 + k2 / k2);
+  // k2 / k2: one, or NaN for zero and infinity
+  const double one = k2 > 0 && k2 < __builtin_inf() ? 1.0 : __builtin_nan("");
+  return 0.7143 + 0.2857 * c * c + 0.5 * c * (k1 / k2 + one);
 }
 // Tree-level bispectrum (src/generalFunctions.cu:94-147).
 G3L_HD double bilin(const DevTables &T, double k1, double k2, double cosphi,
@@ -1080,12 +1104,14 @@ G3L_HD double f_of(const TermArgs &a, int fsel) {
 template <int KIND>
 G3L_HD void zfactors(const DevTables &T, const TermArgs &a, int zi, double z, double w,
                      double &zpre, double &zfac) {
+  zfac = 0;
   if constexpr (KIND <= kNN3) {
-    zpre = 1. / a.nb1[zi] / a.nb2[zi] / T.rho[zi];
-    zfac = 1. / T.dwdz[zi] * T.g[zi] * T.p1[zi] * T.p2[zi] / w / w / w * (1. + z);
+    zpre = div_rn(1. / a.nb1[zi] / a.nb2[zi], T.rho[zi], T.rrho[zi]);
+    if constexpr (KIND != kNN3)   // applied in the reference's order there (proj_3h)
+      zfac = 1. / T.dwdz[zi] * T.g[zi] * T.p1[zi] * T.p2[zi] / w / w / w * (1. + z);
   } else {
     const double rho = T.rho[zi];
-    zpre = 1. / a.nb1[zi] / rho / rho;
+    zpre = div_rn(div_rn(1. / a.nb1[zi], rho, T.rrho[zi]), rho, T.rrho[zi]);
     zfac = 1. / T.dwdz[zi] * T.g[zi] * T.g[zi] * T.p1[zi] / w / w * (1. + z) * (1. + z);
   }
 }
@@ -1105,16 +1131,6 @@ template <>
 struct EvalPolicy<kNbar, P64> {
   using type = P64R;
 };
-
-// a / d correctly rounded from rd = RN(1/d): q = RN(a rd), then one FMA
-// residual correction (Markstein's theorem: with rd the correctly rounded
-// reciprocal the corrected quotient is RN(a / d) for normal operands, no
-// overflow or underflow).  Three instructions instead of the IEEE division
-// sequence, for divisors that repeat over many points.
-G3L_HD double div_rn(double a, double d, double rd) {
-  const double q = a * rd;
-  return fma(fma(-d, q, a), rd, q);
-}
 
 // The NNMap 3-halo projection b = B / dwdz g p1 p2 / w^3 (1+z) in the
 // reference's order (src/NNMap_Model.cu:1031-1033), from the divisors and

@@ -87,6 +87,14 @@ __device__ __forceinline__ void rule_point(int q, const double *c, const double 
   }
 }
 
+// The coordinate with code `code` (gm_code) along a dimension with centre c and
+// half-width h, as rule_point gives it.
+__device__ __forceinline__ double rule_coord(int code, double c, double h) {
+  const double r = h * (code < 3 ? kLam2 : code < 5 ? kLam4 : kLam5);
+  const double x = (code & 1) ? c - r : c + r;
+  return code == 0 ? c : x;
+}
+
 // s + p[0] + p[1] + ... + p[N-1], added in that order.  The values are
 // loaded in batches of 16 before they are added: left to the compiler, the
 // chain kept one LDS load in flight and waited a full LDS round trip for
