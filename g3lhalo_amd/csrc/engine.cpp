@@ -175,7 +175,14 @@ int ctx_create_bare(g3l_ctx **out) {
 
 // ---------------------------------------------------------------------------
 // Batched engine: all jobs refine together; per round one selection launch
-// and one evaluation launch per integrand kind.
+// and one evaluation launch per integrand kind, or one for all kinds while a
+// round is small.
+
+// Rounds queued at a time at most, and most blocks of a round that is queued
+// before the last one's outcome is known (its blocks are a bound, mostly twice
+// what it needs; anything from 512 to 20000 takes the same time).
+constexpr uint32_t kBurstRounds = 16;
+constexpr uint64_t kBurstBlocks = 4096;
 
 int refine_jobs(g3l_ctx *c, const EngineBufs &B, uint32_t nj, bool timed, int prec,
                 bool use_graph) {
@@ -199,6 +206,7 @@ int refine_jobs(g3l_ctx *c, const EngineBufs &B, uint32_t nj, bool timed, int pr
   R.counters = dcnt;
   R.njobs = nj;
   G3L_HIP(launch_zero(dcnt, kNumKinds + 1, s));
+  if (B.rows) G3L_HIP(launch_zero(B.rows, kRows * kRowWords, s));
   G3L_HIP(launch_roots(R, s));
 
   EvalLaunch EL{};
@@ -230,13 +238,17 @@ int refine_jobs(g3l_ctx *c, const EngineBufs &B, uint32_t nj, bool timed, int pr
   bool kind_used[kNumKinds];
   uint64_t launches = 0;
   uint32_t rounds = 0;
-  G3L_HIP(hipMemcpyAsync(hcnt, dcnt, (kNumKinds + 1) * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-  G3L_HIP(hipStreamSynchronize(s));
+  // the roots' lists: an entry per integral
+  for (int k = 0; k < kNumKinds; ++k) hcnt[k] = B.kind_jobs[k];
+  // regions of each kind, a bound (finished integrals' count too): a round's list
+  // has at most two entries for each
+  uint64_t live[kNumKinds];
+  for (int k = 0; k < kNumKinds; ++k) live[k] = B.kind_jobs[k];
   // graph mode: the round's launches and the counter copy are one graph
   // (every node records its events; they are read only when timed)
   RoundGraph &graph = c->graph;
   const KindLaunch KL = kind_launch(c, prec);
-  if (use_graph) {
+  auto ready_graph = [&]() -> int {
     // the executable graph is kept while the kinds, variants, precision,
     // job count and buffers stay the same (repeated calls of one workload)
     bool in_run[kNumKinds];
@@ -259,8 +271,95 @@ int refine_jobs(g3l_ctx *c, const EngineBufs &B, uint32_t nj, bool timed, int pr
         return rc;
       c->graph_key = key;
     }
-  }
+    return G3L_OK;
+  };
+  // Small rounds: every kind's evaluation in one launch, and rounds queued
+  // without waiting for the last one while the bound on their blocks stays
+  // small.  FP64 kinds only.
+  bool small_ok = B.rows != nullptr;
+  for (int k = 0; k < kNumKinds; ++k) small_ok = small_ok && (!per_kind[k] || KL.prec[k] == G3L_FP64);
+  uint32_t row = 0;
+  int clock_khz = 0;
+  if (small_ok && timed)
+    G3L_HIP(hipDeviceGetAttribute(&clock_khz, hipDeviceAttributeWallClockRate, c->device));
+  // the rounds from the lists of length hcnt on; the last one's counters to hcnt
+  auto run_small = [&]() -> int {
+    uint64_t bound[kNumKinds], most[kNumKinds];
+    for (int k = 0; k < kNumKinds; ++k) {
+      bound[k] = std::min<uint64_t>(hcnt[k], per_kind[k]);
+      most[k] = live[k];
+    }
+    if (row + kBurstRounds + 1 > kRows) {
+      G3L_HIP(launch_zero(B.rows, kRows * kRowWords, s));
+      row = 0;
+    }
+    const uint32_t first = row;
+    EvalSmallLaunch ES{};
+    ES.E = EL;
+    for (int k = 0; k < kNumKinds; ++k) {
+      ES.lists[k] = lists[k];
+      ES.count[k] = (uint32_t)bound[k];
+    }
+    uint32_t n = 0;
+    do {
+      small_ends(bound, ES.end);
+      uint32_t *here = B.rows + (size_t)row * kRowWords;
+      ES.row = n ? here - kRowWords : nullptr;
+      ES.clock = reinterpret_cast<uint64_t *>(here);
+      G3L_HIP(launch_eval_small(ES, s));
+      SelectLaunch SR = SL;
+      SR.counters = here;
+      SR.clock = ES.clock;
+      G3L_HIP(launch_select(SR, nj, s));
+      ++row;
+      ++n;
+      for (int k = 0; k < kNumKinds; ++k) {
+        bound[k] = std::min<uint64_t>(2 * most[k], per_kind[k]);
+        most[k] *= 2;
+      }
+    } while (n < kBurstRounds && small_blocks(bound) <= kBurstBlocks);
+    G3L_HIP(hipMemcpyAsync(B.hrows, B.rows + (size_t)first * kRowWords,
+                           (size_t)n * kRowWords * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+    G3L_HIP(hipStreamSynchronize(s));
+    for (uint32_t r = 0; r < n; ++r) {
+      const uint32_t *h = B.hrows + (size_t)r * kRowWords;
+      const uint64_t *t = reinterpret_cast<const uint64_t *>(h);
+      uint64_t eval_end = t[kRowStart];
+      for (int k = 1; k < kNumKinds; ++k) {
+        if (!hcnt[k]) continue;
+        ++launches;
+        ++kind_launches[k];
+        if (!clock_khz) continue;
+        eval_end = std::max(eval_end, t[kRowKindEnd + k]);
+        kind_ms[k] += (double)(t[kRowKindEnd + k] - t[kRowStart]) / clock_khz;
+      }
+      if (clock_khz) {
+        eval_ms += (double)(eval_end - t[kRowStart]) / clock_khz;
+        if (t[kRowSelectEnd] > t[kRowSelect])
+          select_ms += (double)(t[kRowSelectEnd] - t[kRowSelect]) / clock_khz;
+      }
+      for (int k = 0; k <= kNumKinds; ++k) hcnt[k] = h[k];
+      for (int k = 0; k < kNumKinds; ++k) live[k] += hcnt[k] / 2;
+      ++rounds;
+      if (hcnt[kNumKinds] == 0) break;
+    }
+    return G3L_OK;
+  };
+  bool have_graph = false;
   for (;;) {
+    if (small_ok) {
+      uint64_t now[kNumKinds];
+      for (int k = 0; k < kNumKinds; ++k) now[k] = hcnt[k];
+      if (small_blocks(now) <= kSmallBlocks) {
+        if ((rc = run_small())) return rc;
+        if (hcnt[kNumKinds] == 0) break;
+        continue;
+      }
+    }
+    if (use_graph && !have_graph) {
+      if ((rc = ready_graph())) return rc;
+      have_graph = true;
+    }
     uint32_t cnt[kNumKinds];
     for (int k = 0; k < kNumKinds; ++k) {
       cnt[k] = (uint32_t)std::min<uint64_t>(hcnt[k], per_kind[k]);
@@ -303,6 +402,7 @@ int refine_jobs(g3l_ctx *c, const EngineBufs &B, uint32_t nj, bool timed, int pr
       }
     }
     ++rounds;
+    for (int k = 0; k < kNumKinds; ++k) live[k] += hcnt[k] / 2;
     if (hcnt[kNumKinds] == 0) break;
   }
   c->last.eval_ms = eval_ms;
@@ -340,6 +440,7 @@ int run_engine(g3l_ctx *c, EngineJobs &E, std::vector<JobState> &out, bool timed
     d.base = (uint32_t)B.slots;
     B.slots += d.cap;
     B.per_kind[d.kind] += 2ull * d.cap;
+    ++B.kind_jobs[d.kind];
   }
   if (B.slots >= (1ull << 32) - 1) return G3L_ENOMEM;
   uint64_t list_total = 0;
@@ -352,8 +453,10 @@ int run_engine(g3l_ctx *c, EngineJobs &E, std::vector<JobState> &out, bool timed
   if ((rc = c->state.ensure(nj * sizeof(JobState)))) return rc;
   if ((rc = c->args.ensure(E.args.size() * sizeof(TermArgs)))) return rc;
   if ((rc = c->boxes.ensure(E.boxes.size() * sizeof(double)))) return rc;
-  if ((rc = c->counters.ensure(64))) return rc;
-  if ((rc = c->hcounters.ensure(64))) return rc;
+  // the counters, and behind them the rows
+  constexpr size_t kCountBytes = 64 + kRows * kRowWords * sizeof(uint32_t);
+  if ((rc = c->counters.ensure(kCountBytes))) return rc;
+  if ((rc = c->hcounters.ensure(kCountBytes))) return rc;
   hipStream_t s = c->stream;
   if (trace && c->trace_cap > 0) {
     const size_t entries = (size_t)nj * c->trace_cap;
@@ -383,6 +486,8 @@ int run_engine(g3l_ctx *c, EngineJobs &E, std::vector<JobState> &out, bool timed
   B.boxes = c->boxes.as<double>();
   B.dcnt = c->counters.as<uint32_t>();
   B.hcnt = c->hcounters.as<uint32_t>();
+  B.rows = B.dcnt + 16;
+  B.hrows = B.hcnt + 16;
   if ((rc = refine_jobs(c, B, nj, timed, prec, c->launch_mode == G3L_LAUNCH_GRAPH))) return rc;
   G3L_HIP(hipMemcpyAsync(out.data(), B.state, nj * sizeof(JobState), hipMemcpyDeviceToHost, s));
   G3L_HIP(hipStreamSynchronize(s));

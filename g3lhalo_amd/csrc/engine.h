@@ -215,6 +215,11 @@ struct EngineBufs {
   double *boxes = nullptr;
   uint32_t *dcnt = nullptr;
   uint32_t *hcnt = nullptr;
+  // records of rounds the host does not wait for (kRows rows on the device and
+  // in pinned memory); null: it waits for every round
+  uint32_t *rows = nullptr;
+  uint32_t *hrows = nullptr;
+  uint32_t kind_jobs[kNumKinds] = {};   // integrals per kind
   uint32_t *trace = nullptr;
   uint32_t trace_cap = 0;
 };

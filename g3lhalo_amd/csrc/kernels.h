@@ -21,6 +21,49 @@ struct EvalLaunch {
   uint32_t njobs;     // entries naming a slot >= stride or a job >= njobs are skipped
 };
 
+// A round's record when the host does not wait for it: the counters the
+// selection leaves for the next round (uint32_t [kNumKinds + 2], as
+// SelectLaunch::counters), and from kRowStart on, in 64-bit words, clock readings:
+// evaluation start, selection start and end, end of each kind's evaluation.
+constexpr int kRowWords = 32;                 // uint32_t per row
+constexpr int kRowStart = 6, kRowSelect = 7, kRowSelectEnd = 8, kRowKindEnd = 9;
+constexpr int kRows = 256;
+static_assert(kNumKinds + 2 <= 2 * kRowStart && kRowKindEnd + kNumKinds <= kRowWords / 2, "row");
+
+// All kinds of a round in one launch (FP64): blocks [end[k - 1], end[k]) take
+// kind k's groups of small_group(k) regions; its list's length is row[k], or
+// count[k] without a row.
+constexpr int kSmallThreads = 512;
+struct EvalSmallLaunch {
+  EvalLaunch E;                      // list and count unused
+  const EvalItem *lists[kNumKinds];
+  uint32_t count[kNumKinds];
+  uint32_t end[kNumKinds];
+  const uint32_t *row;
+  uint64_t *clock;                   // the round's record; may be null
+};
+// Regions per block of kind k, blocks for lists of n[k] entries, and the ends of
+// the kinds' block ranges.
+uint32_t small_group(int kind);
+inline uint64_t small_blocks(const uint64_t (&n)[kNumKinds]) {
+  uint64_t b = 0;
+  for (int k = 1; k < kNumKinds; ++k) b += (n[k] + small_group(k) - 1) / small_group(k);
+  return b;
+}
+inline void small_ends(const uint64_t (&n)[kNumKinds], uint32_t (&end)[kNumKinds]) {
+  uint32_t e = 0;
+  end[0] = 0;
+  for (int k = 1; k < kNumKinds; ++k)
+    end[k] = e += (uint32_t)((n[k] + small_group(k) - 1) / small_group(k));
+}
+// Most blocks of a round that goes out in one launch.  Time of a run with 9
+// integrals / 33 / 165 / 1650 when rounds of up to 0, 1024, 8192, 16384, 40000
+// blocks do: 5.99, 4.29, 3.47, 3.18, 3.19 ms / 20.1, 19.2, 18.6, 18.25, 18.2 /
+// 29.8, 28.9, 28.4, 28.07, 28.06 / 264 at all of them; with no limit 3.1, 18.9, 30.2
+// and 299 ms, the large rounds' shapes being the faster ones for large rounds.
+constexpr uint64_t kSmallBlocks = 20000;
+hipError_t launch_eval_small(const EvalSmallLaunch &L, hipStream_t s);
+
 struct RootsLaunch {
   const JobDesc *jobs;
   const double *boxes;  // per job: lo[kMaxDim], hi[kMaxDim]
@@ -49,6 +92,7 @@ struct SelectLaunch {
   // (2 per popped region) at trace[J * trace_cap + r], r < trace_cap; may be null
   uint32_t *trace;
   uint32_t trace_cap;
+  uint64_t *clock;   // the round's record (kRowSelect, kRowSelectEnd); may be null
 };
 
 // New integrals joining a running engine: their descriptors and parameters

@@ -111,13 +111,14 @@ __device__ __forceinline__ uint32_t block_group() {
 }
 
 template <int D, int G, int NT>
-__device__ __forceinline__ int stage_regions(const EvalLaunch &L, Stage<D, G> &S) {
+__device__ __forceinline__ int stage_regions(const EvalLaunch &L, const EvalItem *list,
+                                             uint32_t count, uint32_t group, Stage<D, G> &S) {
   const int tid = threadIdx.x;
-  const uint32_t first = block_group() * G;
-  const int ng = (L.count - first) < (uint32_t)G ? (int)(L.count - first) : G;
+  const uint32_t first = group * G;
+  const int ng = (count - first) < (uint32_t)G ? (int)(count - first) : G;
   const uint64_t St = L.stride;
   if (tid < ng) {
-    EvalItem it = L.list[first + tid];
+    EvalItem it = list[first + tid];
     bool ok = it.slot < St && it.job < L.njobs;
     S.slot[tid] = ok ? it.slot : 0xffffffffu;
     if (ok) {
@@ -259,8 +260,8 @@ struct Cache {
 };
 
 // Class indices of every point in one 16-byte load; a byte load with its address
-// arithmetic per index, and a region's points rebuilt by rule_point for every
-// class, were a fifth of a point's instructions.  Packed look-ups, coordinates
+// arithmetic per index, and whole rule points rebuilt for one or two of their
+// coordinates, were a good part of a point's instructions.  Packed look-ups, coordinates
 // by code and quotients by known reciprocals (DevTables) together took the
 // evaluation of the 550-triplet workload from 281 to 254 ms, values
 // bit-identical.  Word 0 l1, l2, z (3 bits each), l3 (6),
@@ -887,12 +888,33 @@ __device__ __forceinline__ void u_eval_sorted(Cache<KIND> &C, int i, const uint1
   C.u[i] = P::u_a1(C.u[i], Nfw{0.0, en.c[fs], en.lc[fs], en.F[fs]});
 }
 
-// At most 64 VGPRs (8 waves per SIMD): the FP64 5-D and 7-D kinds otherwise
-// compile to 70-80 and run 6-7 waves per SIMD.  The few registers this
-// spills cost less than the lost occupancy: NNMap 1h 4.12 -> 3.69 ms and
-// 3h 4.26 -> 3.93 ms per launch on the 550-triplet workload, 2h unchanged.
+// LDS of an evaluation block.
+template <int KIND>
+struct EvalLds {
+  using S = Spec<kind_of_kv(KIND)>;
+  static constexpr int G = KGroup<KIND>::G, NP = KGroup<KIND>::P;
+  static constexpr int NU = Cache<KIND>::NU_TOTAL;
+  static constexpr bool kSort = sort_u<KIND>();
+  // f holds the point values of pass 3, and before that the branch lists of the
+  // u items (2 NU entries of 16 bits)
+  static constexpr int NF = kSort && (4 * NU + 7) / 8 > G * NP ? (4 * NU + 7) / 8 : G * NP;
+  static constexpr int NUNF = kSort ? NU : 1;
+  using Stg = Stage<S::D, G>;
+  Stg St;
+  Cache<KIND> C;
+  double f[NF];
+  unsigned long long ucnt;   // u items per branch, 21-bit fields
+  uint16_t unf[NUNF];
+};
+
+// Evaluates group `group` of the list: its regions' values, errors and split
+// dimensions.  The block has KGroup<KIND>::NT threads and all of them call it.
 template <int KIND, class P>
-__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8))) void k_eval(EvalLaunch L) {
+__device__ __forceinline__ void eval_block(const EvalLaunch &L, const EvalItem *list,
+                                           uint32_t count, uint32_t group,
+                                           typename EvalLds<KIND>::Stg &St, Cache<KIND> &C,
+                                           double *s_f, unsigned long long &s_ucnt,
+                                           uint16_t *s_unf) {
   using S = Spec<kind_of_kv(KIND)>;
   constexpr int D = S::D;
   constexpr int NP = KGroup<KIND>::P;
@@ -905,16 +927,7 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8))) void 
   using Q = typename EvalPolicy<kind_of_kv(KIND), P>::type;
   constexpr bool kSort = sort_u<KIND>();
   constexpr int NU = Cache<KIND>::NU_TOTAL;
-  // s_f holds the point values of pass 3, and before that the branch lists
-  // of the u items (2 NU entries of 16 bits)
-  constexpr int NF = kSort && (4 * NU + 7) / 8 > G * NP ? (4 * NU + 7) / 8 : G * NP;
-  __shared__ Stage<D, G> St;
-  __shared__ Cache<KIND> C;
-  __shared__ double s_f[NF];
-  __shared__ unsigned long long s_ucnt;   // u items per branch, 21-bit fields
-  __shared__ uint16_t s_unf[kSort ? NU : 1];
-  if (block_group() * G >= L.count) return;
-  const int ng = stage_regions<D, G, NT>(L, St);
+  const int ng = stage_regions<D, G, NT>(L, list, count, group, St);
   const int tid = threadIdx.x;
   const DevTables T = L.T;
   if (kSort && tid == 0) s_ucnt = 0;
@@ -961,6 +974,77 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8))) void 
   }
   __syncthreads();
   reduce_regions<D, G, NP>(L, St, s_f, ng);
+}
+
+// At most 64 VGPRs (8 waves per SIMD): the FP64 5-D and 7-D kinds otherwise
+// compile to 70-80 and run 6-7 waves per SIMD.  The few registers this
+// spills cost less than the lost occupancy: NNMap 1h 4.12 -> 3.69 ms and
+// 3h 4.26 -> 3.93 ms per launch on the 550-triplet workload, 2h unchanged.
+template <int KIND, class P>
+__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8))) void k_eval(EvalLaunch L) {
+  // variables of their own, not one EvalLds: the compiler then knows them apart
+  // (as one struct, 550 triplets took 262.8 ms rather than 261.6, the 2h kind most)
+  using M = EvalLds<KIND>;
+  __shared__ typename M::Stg St;
+  __shared__ Cache<KIND> C;
+  __shared__ double s_f[M::NF];
+  __shared__ unsigned long long s_ucnt;
+  __shared__ uint16_t s_unf[M::NUNF];
+  const uint32_t group = block_group();
+  if (group * KGroup<KIND>::G >= L.count) return;
+  eval_block<KIND, P>(L, L.list, L.count, group, St, C, s_f, s_ucnt, s_unf);
+}
+
+// A whole round's evaluation in one launch, for small rounds (kSmallBlocks): the
+// kinds run beside each other and fill the chip together instead of one after
+// the other, each with its launch gap and its last wave of blocks, and the
+// lists' lengths are read where the selection left them, so that the host can
+// queue a round before it knows the last one's outcome.  Every kind in its
+// 512-thread shape, which differs from the large rounds' only in speed.
+template <int KIND>
+struct SmallKv {
+  static constexpr int kv = make_kv(KIND, kind_dim(KIND) == 6 ? 3 : 1);
+  static_assert(KGroup<kv>::NT == kSmallThreads, "one block size for all kinds");
+};
+template <int KIND>
+__device__ __forceinline__ void eval_small(const EvalSmallLaunch &L, uint32_t group,
+                                           unsigned char *lds) {
+  constexpr int kv = SmallKv<KIND>::kv;
+  const uint32_t count = L.row ? L.row[KIND] : L.count[KIND];
+  if (group * KGroup<kv>::G >= count) return;
+  EvalLds<kv> &M = *reinterpret_cast<EvalLds<kv> *>(lds);
+  eval_block<kv, P64>(L.E, L.lists[KIND], count, group, M.St, M.C, M.f, M.ucnt, M.unf);
+  if (L.clock && threadIdx.x == 0)
+    atomicMax(reinterpret_cast<unsigned long long *>(L.clock) + kRowKindEnd + KIND,
+              (unsigned long long)wall_clock64());
+}
+__global__ __launch_bounds__(kSmallThreads) __attribute__((amdgpu_waves_per_eu(8))) void
+k_eval_small(EvalSmallLaunch L) {
+  constexpr size_t a = sizeof(EvalLds<SmallKv<kNN1>::kv>), b = sizeof(EvalLds<SmallKv<kNN2>::kv>),
+                   c = sizeof(EvalLds<SmallKv<kNN3>::kv>), d = sizeof(EvalLds<SmallKv<kNM1>::kv>),
+                   e = sizeof(EvalLds<SmallKv<kNM2>::kv>), f = sizeof(EvalLds<SmallKv<kNM3>::kv>);
+  constexpr size_t ab = a > b ? a : b, cd = c > d ? c : d, ef = e > f ? e : f,
+                   abcd = ab > cd ? ab : cd;
+  __shared__ __align__(16) unsigned char lds[abcd > ef ? abcd : ef];
+  const uint32_t bl = blockIdx.x;
+  if (L.clock && bl == 0 && threadIdx.x == 0) L.clock[kRowStart] = (uint64_t)wall_clock64();
+  if (bl < L.end[kNN1]) eval_small<kNN1>(L, bl, lds);
+  else if (bl < L.end[kNN2]) eval_small<kNN2>(L, bl - L.end[kNN1], lds);
+  else if (bl < L.end[kNN3]) eval_small<kNN3>(L, bl - L.end[kNN2], lds);
+  else if (bl < L.end[kNM1]) eval_small<kNM1>(L, bl - L.end[kNN3], lds);
+  else if (bl < L.end[kNM2]) eval_small<kNM2>(L, bl - L.end[kNM1], lds);
+  else eval_small<kNM3>(L, bl - L.end[kNM2], lds);
+}
+uint32_t small_group(int kind) {
+  const int d = kind_dim(kind);
+  return d == 5 ? KGroup<SmallKv<kNN1>::kv>::G
+                : d == 6 ? KGroup<SmallKv<kNN2>::kv>::G : KGroup<SmallKv<kNN3>::kv>::G;
+}
+hipError_t launch_eval_small(const EvalSmallLaunch &L, hipStream_t s) {
+  const uint32_t blocks = L.end[kNumKinds - 1];
+  if (blocks == 0) return hipSuccess;
+  hipLaunchKernelGGL(k_eval_small, dim3(blocks), dim3(kSmallThreads), 0, s, L);
+  return hipGetLastError();
 }
 
 // ----------------------------------------------------------------- roots
@@ -1657,15 +1741,19 @@ __global__ __launch_bounds__(NT) void k_select(SelectLaunch L) {
     S.bad = 0;
   }
   __syncthreads();
+  if (L.clock && blockIdx.x == 0 && threadIdx.x == 0) L.clock[kRowSelect] = (uint64_t)wall_clock64();
   if (S.st.flags & kJobDone) return;
   const JobDesc d = L.jobs[J];
   if (S.st.n <= 256) {
     if (threadIdx.x >= 64) return;
     if (S.st.n <= 64) select_wave<1>(L, J, d, S.st, S.search, S.sel);
     else select_wave<4>(L, J, d, S.st, S.search, S.sel);
-    return;
+  } else {
+    select_block<NT>(L, J, d, S);
   }
-  select_block<NT>(L, J, d, S);
+  if (L.clock && threadIdx.x == 0)
+    atomicMax(reinterpret_cast<unsigned long long *>(L.clock) + kRowSelectEnd,
+              (unsigned long long)wall_clock64());
 }
 
 

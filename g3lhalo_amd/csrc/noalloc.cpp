@@ -113,6 +113,7 @@ extern "C" int g3l_eval_batch_noalloc(g3l_ctx *c, const g3l_request *reqs, size_
     const JobDesc d = desc_of(reqs[i], 0, 0);
     B.slots += d.cap;
     B.per_kind[d.kind] += 2ull * d.cap;
+    ++B.kind_jobs[d.kind];
   }
   uint64_t list_total = 0;
   for (int k = 0; k < kNumKinds; ++k) list_total += B.per_kind[k];

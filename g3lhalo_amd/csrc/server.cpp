@@ -320,7 +320,26 @@ int g3l_server_step(g3l_server *s, g3l_server_status *status) {
   uint32_t *hc = s->hcounters.as<uint32_t>();
   const KindLaunch KL = kind_launch(c, s->precision);
   const int *var = KL.variant;
-  if (c->launch_mode == G3L_LAUNCH_GRAPH) {
+  // a small round's kinds go out in one launch (as in refine_jobs)
+  uint64_t fill[kNumKinds];
+  bool small = true;
+  for (int k = 0; k < kNumKinds; ++k) {
+    fill[k] = s->fill[k];
+    small = small && (!fill[k] || KL.prec[k] == G3L_FP64);
+  }
+  if (small && small_blocks(fill) <= kSmallBlocks) {
+    EvalSmallLaunch ES{};
+    ES.E = EL;
+    for (int k = 0; k < kNumKinds; ++k) {
+      ES.lists[k] = s->lists_k[k];
+      ES.count[k] = s->fill[k];
+    }
+    small_ends(fill, ES.end);
+    G3L_HIP(launch_eval_small(ES, st));
+    G3L_HIP(launch_zero(dcnt, kNumKinds + 2, st));
+    G3L_HIP(launch_select(SL, na, st));
+    G3L_HIP(hipMemcpyAsync(hc, dcnt, (kNumKinds + 2) * sizeof(uint32_t), hipMemcpyDeviceToHost, st));
+  } else if (c->launch_mode == G3L_LAUNCH_GRAPH) {
     if (!s->graph.exec || !s->graph.selects(na) || !std::equal(var, var + kNumKinds, s->graph_variant) ||
         !std::equal(KL.prec, KL.prec + kNumKinds, s->graph_prec)) {
       bool in_use[kNumKinds];

@@ -167,7 +167,8 @@ typedef struct g3l_batch_stats {
   uint64_t evals;        /* integrand evaluations */
   uint32_t rounds;
   uint32_t pad;
-  /* per integrand kind (0 n_bar, 1-3 NNMap 1h-3h, 4-6 NMapMap 1h-3h) */
+  /* per integrand kind (0 n_bar, 1-3 NNMap 1h-3h, 4-6 NMapMap 1h-3h); in small
+   * rounds the kinds are evaluated side by side, and their times overlap */
   double kind_ms[8];
   uint64_t kind_launches[8];
   uint64_t kind_evals[8];
@@ -219,7 +220,9 @@ int g3l_set_variant(g3l_ctx *ctx, int32_t kind, int32_t precision, int32_t varia
  * G3L_LAUNCH_GRAPH (the default): each round's evaluation, counter-clear,
  * selection and counter-copy operations are one instantiated HIP graph whose
  * kernel nodes are re-sized per round; G3L_LAUNCH_STREAM: the same kernels
- * launched one by one on the context's stream.  Results are identical. */
+ * launched one by one on the context's stream.  In both, small FP64 rounds go
+ * to the stream as one evaluation of all kinds and one selection.  Results are
+ * identical. */
 typedef enum g3l_launch_mode { G3L_LAUNCH_STREAM = 0, G3L_LAUNCH_GRAPH = 1 } g3l_launch_mode;
 int g3l_set_launch_mode(g3l_ctx *ctx, int32_t mode);
 
