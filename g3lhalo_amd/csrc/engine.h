@@ -152,7 +152,7 @@ struct g3l_ctx {
   // 1-D integrals: node stores of the resident blocks, inputs, outcome
   DevBuf od_store, od_in;
   // plain engine
-  DevBuf pgeo, psplit, plist, pjob, parg;
+  DevBuf plist, pjob, parg;
   HostBuf hgeo, hsplit;
   uint32_t pcap = 0;
   // launch variant (block shape) per precision and integrand kind (n_bar,
