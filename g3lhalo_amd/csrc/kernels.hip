@@ -544,7 +544,7 @@ __device__ __forceinline__ void pass1(const DevTables &T, const Stage<Spec<kind_
         const bool need = slot == 0 ? uses_nfw<kind_of_kv(KIND)>(0, fs)
                                     : slot == 1 ? uses_nfw<kind_of_kv(KIND)>(1, fs) : uses_nfw<kind_of_kv(KIND)>(2, fs);
         if (need) {
-          const Nfw nf = make_nfw(T, M, zt, f_of(a, fs));
+          const Nfw nf = make_nfw<P>(T, M, zt, f_of(a, fs));
           en.c[fs] = nf.c;
           en.lc[fs] = nf.lc;
           en.F[fs] = nf.F;
@@ -607,7 +607,7 @@ __device__ __forceinline__ void pass1b(const DevTables &T, const Stage<Spec<kind
                                 : slot == 1 ? uses_nfw<kind_of_kv(KIND)>(1, fs) : uses_nfw<kind_of_kv(KIND)>(2, fs);
     if (!need || g >= ng || St.slot[g] == 0xffffffffu) return;
     const MassC &e = C.m[slot][g][c];
-    const Nfw nf = make_nfw(T, mass_of(e), e.zt, f_of(St.args[g], fs));
+    const Nfw nf = make_nfw<P>(T, mass_of(e), e.zt, f_of(St.args[g], fs));
     NfwC &en = C.nf[slot][g][c];
     en.c[fs] = nf.c;
     en.lc[fs] = nf.lc;
@@ -692,7 +692,7 @@ __device__ __forceinline__ bool u_inputs(const DevTables &T,
       M.ir = e.ir;
       M.it = e.it;
       M.r200 = e.r200;
-      n = make_nfw(T, M, C.zt[g][cz], f_of(St.args[g], F::s.fsel));
+      n = make_nfw<P>(T, M, C.zt[g][cz], f_of(St.args[g], F::s.fsel));
     }
     dst = i;
     return true;
