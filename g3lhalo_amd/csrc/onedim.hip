@@ -23,7 +23,7 @@
 // expressions in the same order whichever integral asked first.
 //
 // Measured, a call to its results on the host: one HOD set (256 integrals)
-// 3.7 -> 0.77 ms, 256 sets 104 -> 25 ms, the precomputation 118 -> 9 ms.  A round
+// 3.7 -> 0.70 ms, 256 sets 104 -> 23 ms, the precomputation 118 -> 9.4 ms.  A round
 // of a block is a chain of a few microseconds each: the selection of one wave,
 // the scattered loads of the nodes' values (384 MB of them at 256 sets, from
 // HBM), the rule's 450 dependent instructions, three barriers; two blocks per
@@ -44,17 +44,19 @@ namespace {
 
 constexpr int kThreads = 512, kWaves = kThreads / 64;
 static_assert(kWaves == kOneDimMaxUnit, "one wave per integral of a unit");
-constexpr int kPts = 15;
+constexpr int kPts = 15, kRec = 16;
 constexpr uint32_t kMaxSplit = kOneDimCap / 2;   // regions cut in one round
 constexpr uint32_t kChunk = 32;                  // regions reduced together (precomputation)
 static_assert(kChunk * kPts <= kThreads, "a point per thread");
 
 // Device memory of a block: `nodes` nodes and the regions of `waves` integrals.
-// Node values are field-major so that the lanes of a wave, which reduce
-// neighbouring nodes, read neighbouring words.
+// A node's values lie together, in records of 16: a lane that reduces a node reads
+// three cache lines where a row per point meant thirty, and the nodes of a wave's
+// regions are neighbours only while the tree is young (one HOD set 0.77 -> 0.70 ms,
+// 256 sets 25.2 -> 23.0).
 struct Store {
-  double2 *ab;            // [kPts][nodes]
-  int32_t *ix;            // [kPts][nodes]
+  double2 *ab;            // [nodes][kRec]
+  int32_t *ix;            // [nodes][kRec]
   double *c, *h;          // [nodes]
   double *val, *err;      // [waves][kOneDimCap]: rule value, error
   uint16_t *node;         // [waves][kOneDimCap]
@@ -62,12 +64,12 @@ struct Store {
   __device__ __forceinline__ Store(unsigned char *p, uint32_t nodes_, uint32_t waves)
       : nodes(nodes_) {
     ab = reinterpret_cast<double2 *>(p);
-    c = reinterpret_cast<double *>(ab + (size_t)kPts * nodes);
+    c = reinterpret_cast<double *>(ab + (size_t)kRec * nodes);
     h = c + nodes;
     val = h + nodes;
     err = val + (size_t)waves * kOneDimCap;
     ix = reinterpret_cast<int32_t *>(err + (size_t)waves * kOneDimCap);
-    node = reinterpret_cast<uint16_t *>(ix + (size_t)kPts * nodes);
+    node = reinterpret_cast<uint16_t *>(ix + (size_t)kRec * nodes);
   }
 };
 
@@ -75,8 +77,8 @@ struct Store {
 // breadth-first order, from its group's table (k_onedim_top; nd 0: none), the
 // others from its own store.
 struct TopStore {
-  double2 ab[kPts][kOneDimTop];
-  int32_t ix[kPts][kOneDimTop];
+  double2 ab[kOneDimTop][kRec];
+  int32_t ix[kOneDimTop][kRec];
   double c[kOneDimTop], h[kOneDimTop];
 };
 struct Nodes {
@@ -334,14 +336,13 @@ __device__ __forceinline__ void block_reduce(const OneDimLaunch &L, int mode, co
       if (!place(N, i, count, root, w, id, slot)) continue;
       const double *hmf = L.T.hmf + S.row[w];
       const bool top = id < N.nd;
-      const size_t stride = top ? kOneDimTop : G.nodes;
-      const double2 *ab = top ? &N.top->ab[0][id] : G.ab + (id - N.nd);
-      const int32_t *ix = top ? &N.top->ix[0][id] : G.ix + (id - N.nd);
+      const double2 *ab = top ? N.top->ab[id] : G.ab + (size_t)(id - N.nd) * kRec;
+      const int32_t *ix = top ? N.top->ix[id] : G.ix + (size_t)(id - N.nd) * kRec;
       double f[kPts], v, e;
 #pragma unroll
       for (int j = 0; j < kPts; ++j) {
-        const double2 q = ab[j * stride];
-        f[j] = q.x * hmf[ix[j * stride]] * q.y;
+        const double2 q = ab[j];
+        f[j] = q.x * hmf[ix[j]] * q.y;
       }
       gk_reduce(f, N.h(id), v, e);
       G.val[w * kOneDimCap + slot] = v;
@@ -358,7 +359,7 @@ __device__ __forceinline__ void block_reduce(const OneDimLaunch &L, int mode, co
         const double c = N.c(id), h = N.h(id);
         double x;
         rule_point<1>((int)j, &c, &h, &x);
-        S.f[tid] = precomp_point(mode, S.job[w], x, G.ab[(size_t)j * G.nodes + id]);
+        S.f[tid] = precomp_point(mode, S.job[w], x, G.ab[(size_t)id * kRec + j]);
       }
       __syncthreads();
       if (tid < kChunk && i0 + tid < total && place(N, i0 + tid, count, root, w, id, slot)) {
@@ -420,7 +421,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
           const double c = 0.5 * (g.lo + g.hi), h = 0.5 * (g.hi - g.lo);
           double x;
           rule_point<1>(tid, &c, &h, &x);
-          one_dim_node<PRE>(L.T, g, t1, x, G.ab[(size_t)tid * G.nodes], G.ix[(size_t)tid * G.nodes]);
+          one_dim_node<PRE>(L.T, g, t1, x, G.ab[tid], G.ix[tid]);
         }
       }
     }
@@ -463,7 +464,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
         const double h = N.h(v) * 0.5, c = right ? N.c(v) + h : N.c(v) - h;
         double x;
         rule_point<1>(j, &c, &h, &x);
-        one_dim_node<PRE>(L.T, g, t1, x, G.ab[(size_t)j * G.nodes + id], G.ix[(size_t)j * G.nodes + id]);
+        one_dim_node<PRE>(L.T, g, t1, x, G.ab[(size_t)id * kRec + j], G.ix[(size_t)id * kRec + j]);
         if (j == 0) {
           G.c[id] = c;
           G.h[id] = h;
@@ -508,7 +509,7 @@ __global__ __launch_bounds__(256) void k_onedim_top(OneDimLaunch L, TopStore *to
   }
   rule_point<1>(j, &c, &h, &x);
   TopStore &t = top[blockIdx.y];
-  one_dim_node<false>(L.T, g, 0.0, x, t.ab[j][id], t.ix[j][id]);
+  one_dim_node<false>(L.T, g, 0.0, x, t.ab[id][j], t.ix[id][j]);
   if (j == 0) {
     t.c[id] = c;
     t.h[id] = h;
@@ -516,7 +517,7 @@ __global__ __launch_bounds__(256) void k_onedim_top(OneDimLaunch L, TopStore *to
 }
 
 size_t one_dim_store_bytes(uint32_t nodes, uint32_t waves) {
-  const size_t b = (size_t)nodes * (kPts * (sizeof(double2) + sizeof(int32_t)) + 2 * sizeof(double)) +
+  const size_t b = (size_t)nodes * (kRec * (sizeof(double2) + sizeof(int32_t)) + 2 * sizeof(double)) +
                    (size_t)waves * kOneDimCap * (2 * sizeof(double) + sizeof(uint16_t));
   return (b + 255) / 256 * 256;
 }
