@@ -37,16 +37,16 @@ KIND_NAMES = {0: "n_bar", 1: "NNMap 1h", 2: "NNMap 2h", 3: "NNMap 3h", 4: "NMapM
 
 # HBM bytes per launch of the dominant kernel, from rocprofv3 FETCH_SIZE and
 # WRITE_SIZE runs of this workload scaled by a copy kernel of known size
-# (profiles/k_eval_nnmap550_counters.md): 123.6 MB read + 14.6 MB written per
+# (profiles/k_eval_nnmap550_counters.md): 124.2 MB read + 14.7 MB written per
 # k_eval<NNMap 2h, FP64> launch of the nnmap550 step.
-TRAFFIC_BYTES_PER_LAUNCH = {("nnmap550", 2): 138210534}
+TRAFFIC_BYTES_PER_LAUNCH = {("nnmap550", 2): 138860000}
 
 # Hardware FP64 flops per evaluation, (kind, launch variant) -> 2 FMA + ADD +
 # MUL + TRANS of the SQ_INSTS_VALU_*_F64 counters x 64 lanes / evaluations,
 # from the same profile: the FP64 instructions the kernel issues (a lane
 # masked off in a branch still counts), against the credited algorithmic
 # work of flops.FLOPS_PER_EVAL.
-HW_FP64_FLOPS_PER_EVAL = {(1, 0): 777, (2, 3): 1114, (3, 2): 1079}
+HW_FP64_FLOPS_PER_EVAL = {(1, 0): 627, (2, 3): 884, (3, 2): 1003}
 
 # Algorithmic HBM bytes per region an evaluation launch handles: the
 # region's centre, half-widths and volume (2D + 1 doubles) and its list item
@@ -328,7 +328,7 @@ def precompute_line(nbins: int = 128, cpu_nbins: int = 32):
     dt = time.perf_counter() - t0
     line = {"nbins": nbins, "seconds": round(dt, 3), "adaptive_integrals": integrals(nbins),
             "integrals_per_s": round(integrals(nbins) / dt, 1),
-            "note": "all seven tables; the integrals refine on the device's batched GK15 engine"}
+            "note": "all seven tables; each integral refines whole in one kernel"}
     ref = os.path.join(ROOT, "oracle", "_ref", "doPrecomputations.x")
     if os.path.exists(ref):
         threads = int(os.environ.get("OMP_NUM_THREADS", os.cpu_count() or 1))
