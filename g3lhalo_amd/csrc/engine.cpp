@@ -920,7 +920,7 @@ int g3l_ctx_create(const g3l_tables *t, g3l_ctx **out) {
     c->rho[i] = c->Om * (1 + z) * (1 + z) * (1 + z) / E * c->rho_crit;
   }
   const size_t n1 = nb, n2 = (size_t)nb * nb;
-  const size_t total = 8 * n1 + 4 * n2 + n1;
+  const size_t total = 8 * n1 + 4 * n2 + n1 + DevTables::kConsts;
   if (c->tables.ensure(total * sizeof(double))) {
     g3l_ctx_destroy(c);
     return G3L_ENOMEM;
@@ -938,7 +938,13 @@ int g3l_ctx_create(const g3l_tables *t, g3l_ctx **out) {
     rw[i] = 1. / t->w[i];
     rrho[i] = 1. / c->rho[i];
   }
-  const size_t orw = put(rw.data(), n1), orr = put(rrho.data(), n1);
+  const long double lmm = std::log((long double)c->mmin);
+  double lo[kMaxDim], hi[kMaxDim];
+  term_box(c, 1, lo, hi);
+  double consts[DevTables::kConsts] = {(double)lmm, (double)(lmm - (double)lmm),
+                                       0.5 * (lo[3] + hi[3])};
+  const size_t orw = put(rw.data(), n1), orr = put(rrho.data(), n1),
+               oconst = put(consts, DevTables::kConsts);
   size_t og = put(t->g, n1), op1 = put(t->p_lens1, n1),
          op2 = put(t->p_lens2 ? t->p_lens2 : t->p_lens1, n1), ow = put(t->w, n1),
          odw = put(t->dwdz, n1), orho = put(c->rho.data(), n1), ohmf = put(t->hmf, n2),
@@ -969,6 +975,11 @@ int g3l_ctx_create(const g3l_tables *t, g3l_ctx **out) {
   T.rrho = d + orr;
   T.g = d + og; T.p1 = d + op1; T.p2 = d + op2; T.w = d + ow; T.dwdz = d + odw;
   T.rho = d + orho; T.hmf = d + ohmf; T.plin = d + opl; T.bh = d + obh; T.conc = d + oc;
+  if (launch_mass_centre(T, d + oconst + 3, c->stream) != hipSuccess ||
+      hipStreamSynchronize(c->stream) != hipSuccess) {
+    g3l_ctx_destroy(c);
+    return G3L_EHIP;
+  }
   *out = c;
   return G3L_OK;
 }

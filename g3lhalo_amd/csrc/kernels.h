@@ -146,6 +146,8 @@ KernelRef zero_kernel_ref();     // k_zero(uint32_t *p, int n)
 // variant: block shape, 0 .. eval_num_variants() - 1 (the same values for all)
 hipError_t launch_eval(int kind, int prec, int variant, const EvalLaunch &L, hipStream_t s);
 int eval_num_variants();
+// Writes the index argument of the mass coordinates' centre, DevTables::xc_ix.
+hipError_t launch_mass_centre(const DevTables &T, double *out, hipStream_t s);
 hipError_t launch_roots(const RootsLaunch &L, hipStream_t s);
 hipError_t launch_select(const SelectLaunch &L, uint32_t njobs, hipStream_t s);
 hipError_t launch_zero(uint32_t *p, int n, hipStream_t s);

@@ -1120,6 +1120,16 @@ __global__ void k_gather(GatherLaunch L) {
   if (t < L.n) L.out[t] = L.state[L.ids[t]];
 }
 
+// The index argument of the mass coordinates' centre (DevTables::xc_ix) to out.
+__global__ void k_mass_centre(DevTables T, double *out) {
+  double m, L;
+  *out = mass_chain(T, T.xc(), m, L);
+}
+hipError_t launch_mass_centre(const DevTables &T, double *out, hipStream_t s) {
+  hipLaunchKernelGGL(k_mass_centre, dim3(1), dim3(1), 0, s, T, out);
+  return hipGetLastError();
+}
+
 __global__ void k_zero(uint32_t *p, int n) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = 0;
