@@ -377,13 +377,23 @@ G3L_HD int zix_round(const DevTables &T, double z) {
 G3L_HD int zix_trunc(const DevTables &T, double z) {
   return clampi((int)div_rn((z - T.zmin) * T.nb, T.zmax - T.zmin, T.rdz), T.nb - 1);
 }
-// Held in [-1, nb^2 + nb] before the conversion: a huge k would otherwise
-// convert out of int's range, and zi * nb + ki could overflow.  Every finite k
-// in that range keeps its index; beyond it the row-spill read lands past the
-// padded table either way and pk's clamp gives the same entry.  NaN, and an
-// infinite k (a zero comoving distance, whose u_NFW is NaN), map to 0.
+// Held in [-1, nb^2 + nb] before the conversion: an infinite k (a zero
+// comoving distance) would otherwise convert out of int's range, and
+// zi * nb + ki could overflow.  Every finite k in that range keeps its
+// index; beyond it the row-spill read lands past the padded table either
+// way and pk's clamp gives the same entry.  NaN maps to 0.
+//
+// The argument by the short logarithm, which differs from the library's by less than
+// 1e-10; within 1e-9 of a half-integer, where that could matter, and for a k that is
+// zero (l3 of a squeezed point: index -1, P = 0), negative, infinite or NaN, the
+// library's with IEEE divisions.  550 triplets 254.0 -> 250.7 ms, the
+// same values.
 G3L_HD int kix_round(const DevTables &T, double k) {
-  const double x = round(div_rn(log(div_rn(k, T.kmin, T.rkmin)) * T.nb, T.lkr, T.rlkr));
+  const double q = div_rn(k, T.kmin, T.rkmin);
+  double x = div_rn(log_pos(q) * T.nb, T.lkr, T.rlkr);
+  const bool direct = q > 1e-290 && q < 1e290 && fabs(x) < 1e5 && fabs(x - rint(x)) < 0.5 - 1e-9;
+  if (!direct) x = log(k / T.kmin) * T.nb / T.lkr;
+  x = round(x);
   const double top = (double)T.nb * T.nb + T.nb;
   return x >= 0 ? (int)fmin(x, top) : (x < 0 ? (int)fmax(x, -1.0) : 0);
 }

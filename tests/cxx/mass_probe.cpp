@@ -1,7 +1,8 @@
-// Host build of mass_direct (physics.h) against mass_chain: reads nb, log10 mmin,
-// log10 mmax and a seed; prints the arguments taken directly, those of them whose
-// indices differ from the chain's, the largest difference of the index argument
-// and the largest relative error of the mass.
+// Host build of mass_direct (physics.h) against mass_chain, and of kix_round against
+// its chain with the library's logarithm: reads nb, log10 mmin, log10 mmax and a
+// seed; prints the arguments taken directly, those of them whose indices differ from
+// the chain's, the largest difference of the index argument, the largest relative
+// error of the mass, the non-masses taken directly, and the k whose index differs.
 #include "../../g3lhalo_amd/csrc/physics.h"
 
 #include <cmath>
@@ -49,5 +50,27 @@ int main(int argc, char **argv) {
     double m, L, a;
     special += mass_direct(T, x, m, L, a);
   }
-  printf("%ld %ld %.3g %.3g %d\n", taken, wrong, far, err, special);
+  // the same range as wave numbers
+  T.kmin = T.mmin;
+  T.kmax = T.mmax;
+  T.rkmin = T.rmmin;
+  T.lkr = T.lmr;
+  T.rlkr = T.rlmr;
+  const double top = (double)T.nb * T.nb + T.nb;
+  auto chain = [&](double k) {
+    const double x = std::round(std::log(k / T.kmin) * T.nb / T.lkr);
+    return x >= 0 ? (int)std::fmin(x, top) : (x < 0 ? (int)std::fmax(x, -1.0) : 0);
+  };
+  long kwrong = 0;
+  for (int i = 0; i < 400000; ++i) {
+    double ix = (1.5 * U(rng) - 0.2) * T.nb;
+    if (i & 1) ix = 0.5 + std::rint(ix) + (U(rng) - 0.5) * std::pow(10., -4 - 11 * U(rng));
+    if (i % 16 == 1) ix = 0.5 + std::floor(ix);
+    const double k = T.kmin * std::exp(ix * T.lkr / T.nb);
+    kwrong += kix_round(T, k) != chain(k);
+  }
+  for (double k : {0., -0., -1., (double)NAN, (double)INFINITY, -(double)INFINITY, 1e-300, 1e-310,
+                   1e300, 1.7e308, T.kmin, T.kmax})
+    kwrong += kix_round(T, k) != chain(k);
+  printf("%ld %ld %.3g %.3g %d %ld\n", taken, wrong, far, err, special, kwrong);
 }

@@ -1,7 +1,8 @@
 """Masses and their look-up indices without pow and log (mass_direct) against the
 reference's chain (mass_chain), on the host: wherever the direct form says that it
 holds, both indices equal the chain's, from the smallest to the largest number of
-bins, at and around every kind of tie and beyond both ends of the range.
+bins, at and around every kind of tie and beyond both ends of the range.  P(k)'s
+index, from the short logarithm away from ties, equals the library chain's everywhere.
 
 The chain's argument L nb / ln(mmax / mmin) carries the roundings of m and of L, 2^-53
 of ln-values up to 40 each and a few of its own: below 40 x 6 x 1.2e-16 nb / ln(mmax /
@@ -32,10 +33,11 @@ def probe(tmp_path_factory):
 def test_indices(probe, nb, lo, hi):
     out = subprocess.run([probe, str(nb), str(lo), str(hi), "5"], capture_output=True, text=True,
                          check=True).stdout
-    taken, wrong, far, err, special = out.split()
+    taken, wrong, far, err, special, kwrong = out.split()
     print(out)
     assert int(taken) > 100000
     assert int(wrong) == 0
     assert float(far) < 1e-10
     assert float(err) < 1.5 * 2.0 ** -53
     assert int(special) == 0
+    assert int(kwrong) == 0
