@@ -250,6 +250,12 @@ G3L_HD double div_rn(double a, double d, double rd) {
   const double q = a * rd;
   return fma(fma(-d, q, a), rd, q);
 }
+// The same for operands that may be infinite and divisors that may be zero, where
+// the residual is NaN and a rd is the IEEE quotient.
+G3L_HD double div_any(double a, double d, double rd) {
+  const double q = div_rn(a, d, rd);
+  return q == q ? q : a * rd;
+}
 
 // Tables resident in HBM (z-major 2-D tables, nb*nb + nb for P_lin).
 struct DevTables {
@@ -372,10 +378,10 @@ G3L_HD double precomp_amplitude(const PrecompParams &p, double x, double R) {
 // outside the tables.
 G3L_HD int clampi(int i, int hi) { return i < 0 ? 0 : (i > hi ? hi : i); }
 G3L_HD int zix_round(const DevTables &T, double z) {
-  return clampi((int)round(div_rn((z - T.zmin) * T.nb, T.zmax - T.zmin, T.rdz)), T.nb - 1);
+  return clampi((int)round(div_any((z - T.zmin) * T.nb, T.zmax - T.zmin, T.rdz)), T.nb - 1);
 }
 G3L_HD int zix_trunc(const DevTables &T, double z) {
-  return clampi((int)div_rn((z - T.zmin) * T.nb, T.zmax - T.zmin, T.rdz), T.nb - 1);
+  return clampi((int)div_any((z - T.zmin) * T.nb, T.zmax - T.zmin, T.rdz), T.nb - 1);
 }
 // Held in [-1, nb^2 + nb] before the conversion: an infinite k (a zero
 // comoving distance) would otherwise convert out of int's range, and
@@ -416,8 +422,8 @@ struct Mass {
 // The reference's chain; returns the indices' argument.
 G3L_HD double mass_chain(const DevTables &T, double x, double &m, double &L) {
   m = pow(10.0, x);
-  L = log(div_rn(m, T.mmin, T.rmmin));
-  return div_rn(L * T.nb, T.lmr, T.rlmr);
+  L = log(div_any(m, T.mmin, T.rmmin));
+  return div_any(L * T.nb, T.lmr, T.rlmr);
 }
 // m = 10^x, L and the indices' argument without pow and log: m by the reduction
 // x = k log10 2 + b, L = x ln 10 - ln mmin, both with the rounding
@@ -838,9 +844,11 @@ G3L_HD double u_nfw(const Nfw &n, double k) {
   return u_nfw_a1<P>(nfw_a1(n, k), n);
 }
 
-// x / sigma / 1.414213562, rs = RN(1 / sigma).
+// x / sigma / 1.414213562, rs = RN(1 / sigma).  An infinite M_th, an empty population
+// (x = -inf), and an infinite sigma, a flat occupation (rs = 0), are valid parameters.
 G3L_HD double over_sigma(double x, double sigma, double rs) {
-  return div_rn(div_rn(x, sigma, rs), 1.414213562, 1.0 / 1.414213562);
+  const double q = div_rn(div_rn(x, sigma, rs), 1.414213562, 1.0 / 1.414213562);
+  return q == q ? q : x * rs * (1.0 / 1.414213562);
 }
 
 // FP64 policy
@@ -1240,12 +1248,12 @@ G3L_HD void zfactors(const DevTables &T, const TermArgs &a, int zi, double z, do
                      double &zpre, double &zfac) {
   zfac = 0;
   if constexpr (KIND <= kNN3) {
-    zpre = div_rn(1. / a.nb1[zi] / a.nb2[zi], T.rho[zi], T.rrho[zi]);
+    zpre = div_any(1. / a.nb1[zi] / a.nb2[zi], T.rho[zi], T.rrho[zi]);
     if constexpr (KIND != kNN3)   // applied in the reference's order there (proj_3h)
       zfac = 1. / T.dwdz[zi] * T.g[zi] * T.p1[zi] * T.p2[zi] / w / w / w * (1. + z);
   } else {
     const double rho = T.rho[zi];
-    zpre = div_rn(div_rn(1. / a.nb1[zi], rho, T.rrho[zi]), rho, T.rrho[zi]);
+    zpre = div_any(div_any(1. / a.nb1[zi], rho, T.rrho[zi]), rho, T.rrho[zi]);
     zfac = 1. / T.dwdz[zi] * T.g[zi] * T.g[zi] * T.p1[zi] / w / w * (1. + z) * (1. + z);
   }
 }
