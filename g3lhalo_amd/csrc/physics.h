@@ -1107,7 +1107,7 @@ G3L_HD double nsatnsat(const TermArgs &a, double ns1, double ns2,
 // F kernel with the reference's k2/k2 (src/generalFunctions.cu:89-92).
 G3L_HD double fkern(double k1, double k2, double c) {
   // k2 / k2: one, or NaN for zero and infinity
-  const double one = k2 > 0 && k2 < __builtin_inf() ? 1.0 : __builtin_nan("");
+  const double a2 = fabs(k2), one = a2 > 0 && a2 < __builtin_inf() ? 1.0 : __builtin_nan("");
   return 0.7143 + 0.2857 * c * c + 0.5 * c * (k1 / k2 + one);
 }
 // Tree-level bispectrum (src/generalFunctions.cu:94-147).

@@ -1,5 +1,5 @@
-// Host build of the HOD occupations, the mass chain and the redshift factors
-// (physics.h) at the ends of their parameters' ranges, against the same expressions
+// Host build of the HOD occupations, the mass chain, the redshift factors and the F
+// kernel (physics.h) at the ends of their parameters' ranges, against the same expressions
 // with IEEE divisions: prints the number of values compared and every one that
 // differs.
 #include "../../g3lhalo_amd/csrc/physics.h"
@@ -69,5 +69,8 @@ int main() {
       zfactors<kNM1>(T, a, 0, 0.3, 1., zpre, zfac);
       same("NMapMap density factor", zpre, 1. / n / rho / rho);
     }
+  // the bispectrum's kernel, whose k2 / k2 is one for either sign
+  for (double k : {-inf, -1e300, -0.3, -1e-310, -0., 0., 1e-310, 0.3, 1e300, inf, (double)NAN})
+    same("F", fkern(0.2, k, 0.5), 0.7143 + 0.2857 * 0.5 * 0.5 + 0.5 * 0.5 * (0.2 / k + k / k));
   printf("%d %d\n", count, bad);
 }
