@@ -427,10 +427,12 @@ G3L_HD double mass_chain(const DevTables &T, double x, double &m, double &L) {
 }
 // m = 10^x, L and the indices' argument without pow and log: m by the reduction
 // x = k log10 2 + b, L = x ln 10 - ln mmin, both with the rounding
-// errors carried.  The argument differs from the library chain's by less than 1e-10,
-// so wherever it is further than that from an integer and a half-integer both give
-// the same indices; false elsewhere (and beyond 1e+-300), for the library's chain,
-// whose own rounding then decides.  A sixth of the chain's instructions, in the
+// errors carried.  Wherever the argument is further from an integer and a half-integer
+// than it can differ from the library chain's, both give the same indices; false
+// elsewhere (and beyond 1e+-300), for the library's chain, whose own rounding then
+// decides.  L differs by a few roundings of ln-values, at most 6 x 1.2e-16 x 1400 for any
+// table of masses from 1e-300 to 1e300, and the argument by nb / ln(mmax / mmin) times
+// that: 1e-9 on twice the argument covers up to 500 bins in a factor e.  A sixth of the chain's instructions, in the
 // longest items of an evaluation block's first pass: 550 triplets 257.4 -> 253.6 ms
 // (1-halo kind 72.1 -> 69.5), 137 NMapMap triplets 61.0 -> 59.1.  Errors against 40
 // digits: m rms 0.433 x 2^-53 (pow 0.608), L 3.95e-16 (the chain 4.04e-16).
@@ -458,8 +460,8 @@ G3L_HD bool mass_direct(const DevTables &T, double x, double &m, double &L, doub
   const double h = x * ln10;
   L = (h - T.lmm()) + ((fma(x, ln10, -h) + x * ln10_lo) - T.lmm_lo());
   ix = div_rn(L * T.nb, T.lmr, T.rlmr);
-  const double d = 2 * ix;
-  return fabs(x) < 300. && fabs(d - rint(d)) > 1e-9;
+  const double d = 2 * ix, margin = fmax(1e-9, 2e-12 * T.nb * T.rlmr);
+  return fabs(x) < 300. && fabs(d - rint(d)) > margin;
 }
 template <class P>
 G3L_HD Mass make_mass(const DevTables &T, double x, int zt) {
