@@ -1,11 +1,14 @@
-// select_math.h -- fixed-point error arithmetic of the batch selection
-// (k_select), shared by the device kernel and host-side checks.
+// select_math.h -- error keys and fixed-point error arithmetic of the batch
+// selection, shared by the device kernels and host-side checks.
 //
 // The Gladwell batch of src/hcubature.cpp:971-985 pops regions in decreasing
-// error until the remaining error meets the tolerance.  k_select finds that
-// count with integer sums of the errors in fixed point, which are exact and
-// independent of summation order: every error key e is mapped to
-// e * 2^shift truncated to an integer.  The shift puts the largest key below
+// error until the remaining error meets the tolerance.  Beyond 256 regions
+// k_select first names the histogram bin that holds the last region popped,
+// from integer sums of the errors in fixed point, which do not depend on the
+// order of its atomics: every error key e is mapped to e * 2^shift truncated to
+// an integer.  The count itself comes from compensated FP64 sums (find_boundary
+// of select_wave.h, which k_onedim shares; bisection over the keys where the
+// truncated sums named the wrong bin).  The shift puts the largest key below
 // 2^(47 - extra), where 2^(16 + extra) >= n (the number of regions), so a sum
 // over all n keys stays below 2^63 and cannot wrap.  At n <= 2^16 (every
 // integral whose budget is below about 1.2e7 evaluations, and every
@@ -44,7 +47,8 @@ G3L_SEL_HD unsigned long long fixed_err(uint64_t k, int shift) {
 }
 
 // Error (in fixed-point units) the batch must remove: the total minus the
-// tolerance |V| reltol, at least one unit (at least one region is popped).
+// tolerance |V| reltol, at least one unit (at least one region is popped).  The
+// host check of the fixed-point units counts pops with it; no kernel does.
 G3L_SEL_HD uint64_t batch_need(uint64_t total, double thr) {
   if (thr >= (double)total) return 1;
   const uint64_t need = total - (uint64_t)floor(thr);
