@@ -211,7 +211,11 @@ int g3l_autotune(g3l_ctx *ctx, int32_t hodset, int32_t precision, g3l_tune_repor
  * integral. */
 int g3l_set_mixed_policy(g3l_ctx *ctx, uint32_t fp32_kinds);
 int g3l_get_mixed_policy(g3l_ctx *ctx, uint32_t *fp32_kinds);
-/* Sets one kind's variant directly (kind 1-6, variant 0-3). */
+/* Sets one kind's variant directly (kind 1-6, variant 0-3).  It holds for the plain
+ * entry point, for every round of g3l_eval_batch_noalloc and of runs with a G3L_MIXED
+ * kind, and for the large rounds of the other runs and of the servers; their small
+ * FP64 rounds, all kinds in one launch, have one shape of their own, which is in
+ * g3l_autotune's ms for every variant alike. */
 int g3l_set_variant(g3l_ctx *ctx, int32_t kind, int32_t precision, int32_t variant);
 
 /* How the refinement rounds of g3l_eval_batch and of the servers made on
