@@ -505,14 +505,19 @@ int run_engine(g3l_ctx *c, EngineJobs &E, std::vector<JobState> &out, bool timed
 // ---------------------------------------------------------------------------
 // 1-D integrals (k_onedim).
 
-int run_one_dim(g3l_ctx *c, const std::vector<OneDimGroup> &groups,
-                const std::vector<OneDimJob> &jobs, bool precomp, double reltol, double scale) {
-  if (groups.size() >= (1u << 24)) return G3L_ENOMEM;
+// Most integrals of a launch: group and integral numbers have to fit the kernel's words,
+// and its lists grow with them.  Every resident block still has a hundred units and
+// more, so that what the last ones take alone is small.
+constexpr size_t kOneDimBatch = 1u << 20;
+
+static int run_one_dim_batch(g3l_ctx *c, const std::vector<OneDimGroup> &groups,
+                             const std::vector<OneDimJob> &jobs, bool precomp, double reltol,
+                             double scale) {
   int cus = 0;
   G3L_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device));
   size_t total = 0;
   for (const OneDimGroup &g : groups) total += g.count;
-  if (total >= (1ull << 31)) return G3L_ENOMEM;
+  if (groups.size() > kOneDimBatch || total > kOneDimBatch) return G3L_EINVAL;
   const size_t resident = (size_t)std::max(1, cus) * one_dim_blocks_per_cu();
   // integrals per unit: as many as still give every resident block one
   const uint32_t per =
@@ -590,6 +595,27 @@ int run_one_dim(g3l_ctx *c, const std::vector<OneDimGroup> &groups,
     G3L_HIP(hipStreamSynchronize(s));
   }
   return oc.failed == ~0ull ? (int)G3L_OK : status_of((uint32_t)(oc.failed & 0xff));
+}
+
+int run_one_dim(g3l_ctx *c, const std::vector<OneDimGroup> &groups,
+                const std::vector<OneDimJob> &jobs, bool precomp, double reltol, double scale) {
+  std::vector<OneDimGroup> part;
+  size_t n = 0;
+  for (const OneDimGroup &g : groups)
+    for (uint32_t first = 0; first < g.count;) {
+      OneDimGroup p = g;
+      p.count = (uint32_t)std::min<size_t>(g.count - first, kOneDimBatch - n);
+      p.job0 += first;
+      p.out += first;
+      first += p.count;
+      n += p.count;
+      part.push_back(p);
+      if (n < kOneDimBatch) continue;
+      if (int rc = run_one_dim_batch(c, part, jobs, precomp, reltol, scale)) return rc;
+      part.clear();
+      n = 0;
+    }
+  return n ? run_one_dim_batch(c, part, jobs, precomp, reltol, scale) : (int)G3L_OK;
 }
 
 }  // namespace g3l

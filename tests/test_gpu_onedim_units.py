@@ -68,3 +68,20 @@ def test_precomputation_does_not_depend_on_company(n):
         x, y = np.asarray(x), np.asarray(b[key])
         y = y[::4, ::4] if x.ndim == 2 else y[::4]
         np.testing.assert_array_equal(x, y, err_msg=key)
+
+
+def test_more_integrals_than_one_launch_takes():
+    """2^20 integrals and 400 more (every set has four of them), in two launches: each
+    set's densities are those of its parameters, whichever launch it is in."""
+    from g3lhalo_amd import _lib
+    t = T.make_tables(2)
+    h = T.hod_prior_draws(7, seed=3)
+    n = (1 << 18) + 100
+    ctx = _lib.Context(t)
+    say(f"units: {n} sets of 2 bins in one call")
+    alone = [ctx.densities(ctx.hodset(x, x)) for x in h]
+    first = ctx.hodsets([h[i % 7] for i in range(n)])
+    for i in [*range(0, n, 997), *range((1 << 18) - 8, n)]:
+        for x, y in zip(ctx.densities(first + i), alone[i % 7]):
+            np.testing.assert_array_equal(x, y, err_msg=f"set {i}")
+    ctx.close()
