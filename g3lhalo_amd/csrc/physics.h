@@ -52,11 +52,19 @@ namespace g3l {
 // correction of the quotient (within one unit in the last place; about a third
 // of the instructions of the IEEE division sequence, which also handles
 // denormal and infinite operands that cannot occur here).
-G3L_HD double fdiv(double a, double b) {
+// frcp: its reciprocal.
+G3L_HD double frcp(double b) {
 #if defined(__HIP_DEVICE_COMPILE__)
   double r = __builtin_amdgcn_rcp(b);
   r = fma(fma(-b, r, 1.0), r, r);
-  r = fma(fma(-b, r, 1.0), r, r);
+  return fma(fma(-b, r, 1.0), r, r);
+#else
+  return 1. / b;
+#endif
+}
+G3L_HD double fdiv(double a, double b) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const double r = frcp(b);
   const double q = a * r;
   return fma(fma(-b, q, a), r, q);
 #else
@@ -87,11 +95,12 @@ G3L_HD double fma_k(double a, double z, double c) {
 // zero, negative, infinite and denormal arguments.  Used for the Ci(x) of
 // u_NFW, whose arguments are in (0, 4); the look-up indices keep the
 // library's log.
-// Its parts: k, f, f^2/2 and s (f^2/2 + R).
+// Its parts: k, f, f^2/2 and s (f^2/2 + R); quot(f) gives s.
 struct LogParts {
   double k, f, hfsq, rest;
 };
-G3L_HD LogParts log_parts(double x) {
+template <class Q>
+G3L_HD LogParts log_parts(double x, Q quot) {
   int k;
   double m = frexp(x, &k);   // x = m 2^k, m in [1/2, 1)
   if (m < 0.70710678118654752440) {
@@ -99,7 +108,7 @@ G3L_HD LogParts log_parts(double x) {
     k -= 1;
   }
   const double f = m - 1.0;
-  const double s = fdiv(f, 2.0 + f);
+  const double s = quot(f);
   const double z = s * s, w = z * z;
   const double t1 = w * fma(w, fma(w, 1.531383769920937332e-01, 2.222219843214978396e-01),
                             3.999999999940941908e-01);
@@ -112,16 +121,22 @@ G3L_HD LogParts log_parts(double x) {
   return LogParts{(double)k, f, hfsq, s * (hfsq + R)};
 }
 G3L_HD double log_pos(double x) {
-  const LogParts p = log_parts(x);
+  const LogParts p = log_parts(x, [](double f) { return fdiv(f, 2.0 + f); });
   return p.k * 6.93147180369123816490e-01 -
          ((p.hfsq - (p.rest + p.k * 1.90821492927058770002e-10)) - p.f);
 }
 // lc = ln(1 + c) and F = lc - c / (1 + c) for c > -1, by the same method, with the
 // roundings of 1 + c (its share of the logarithm is that over 1 + c = 1 / (1 - q)), of
-// k ln 2 + f, of taking f^2 / 2 from it and of the quotient q carried.
+// k ln 2 + f, of taking f^2 / 2 from it and of the quotient q carried.  q and s come from
+// one reciprocal, of (1 + c)(2 + f): two divisions take 550 triplets 0.3 % longer.
 G3L_HD void log_norm(double c, double &lc, double &F) {
-  const double x = 1. + c, lo = c - (x - 1.), q = c / x;
-  const LogParts p = log_parts(x);
+  const double x = 1. + c, lo = c - (x - 1.);
+  double q;
+  const LogParts p = log_parts(x, [&](double f) {
+    const double d = 2.0 + f, rp = frcp(x * d), rd = x * rp, s = f * rd;
+    q = c * d * rp;
+    return fma(fma(-d, s, f), rd, s);
+  });
   const double hi = p.k * 6.93147180369123816490e-01;
   const double a = hi + p.f, ea = p.f - (a - hi);
   const double b = a - p.hfsq, eb = (a - b) - p.hfsq;
