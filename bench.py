@@ -46,7 +46,7 @@ TRAFFIC_BYTES_PER_LAUNCH = {("nnmap550", 2): 138860000}
 # from the same profile: the FP64 instructions the kernel issues (a lane
 # masked off in a branch still counts), against the credited algorithmic
 # work of flops.FLOPS_PER_EVAL.
-HW_FP64_FLOPS_PER_EVAL = {(1, 0): 590, (2, 3): 802, (3, 2): 975}
+HW_FP64_FLOPS_PER_EVAL = {(1, 0): 596, (2, 3): 809, (3, 2): 975}
 
 # Algorithmic HBM bytes per region an evaluation launch handles: the
 # region's centre, half-widths and volume (2D + 1 doubles) and its list item

@@ -23,9 +23,9 @@
 // expressions in the same order whichever integral asked first.
 //
 // Measured, a call to its results on the host: one HOD set (256 integrals)
-// 3.7 -> 0.70 ms, 256 sets 104 -> 23 ms, the precomputation 118 -> 9.4 ms.  A round
+// 3.7 -> 0.70 ms, 256 sets 104 -> 23 ms, the precomputation 118 -> 9.1 ms.  A round
 // of a block is a chain of a few microseconds each: the selection of one wave,
-// the scattered loads of the nodes' values (384 MB of them at 256 sets, from
+// the scattered loads of the nodes' values (384 MB of nodes at 256 sets, 46 GB read from
 // HBM), the rule's 450 dependent instructions, three barriers; two blocks per
 // compute unit do not fill it.
 #include <hip/hip_runtime.h>

@@ -152,7 +152,7 @@ G3L_HD void log_norm(double c, double &lc, double &F) {
 // to infinity, underflow to 0, NaN kept; relative error at most 1.07 x 2^-53, rms 0.43
 // (the library's 1.23 and 0.44).  Half the library's instructions, a third of which
 // are moves of its coefficients into vector registers (fma_k).  With one_plus_erf
-// and the logarithm of make_nfw 550 triplets take 255.3 ms rather than 260.5, the
+// and log_pos for make_nfw's logarithm 550 triplets took 255.3 ms rather than 260.5, the
 // 2-halo kind 90.8 rather than 94.1.
 G3L_HD double exp_k(double x) {
 #if defined(__HIP_DEVICE_COMPILE__)
